@@ -43,10 +43,10 @@ HBM_PEAK_GBS = 8000.0
 
 
 # tgh_rk4 flags per form (include/tgh.h)
-FORMS = {"brick-split": 8, "brick-fused": 2, "blocks-fused": 4 | 2, "blocks-split": 4 | 8}
-KERNEL = {"brick-fused": "k_brick_rhs<4, KS, hole>", "blocks-fused": "k_rhs<4, KS, hole, RK4 epilogue>",
+FORMS = {"brick": 0, "brick-split": 8, "brick-fused": 2, "blocks-fused": 4 | 2, "blocks-split": 4 | 8}
+KERNEL = {"brick": "k_brick_stage<4, KS, hole>", "brick-fused": "k_brick_stage<4, KS, hole>", "blocks-fused": "k_rhs<4, KS, hole, RK4 epilogue>",
           "brick-split:head": "k_brick_head<4, KS, hole>", "brick-split:pi": "k_brick_pi<4>",
-          "blocks-split:head": "k_head<4, KS, hole, RK4 epilogue>", "blocks-split:pi": "k_pi<4, RK4 epilogue>"}
+          "blocks-split": "k_block_stage<4, KS, hole>"}
 
 
 def note(msg):
@@ -63,9 +63,9 @@ def parse():
     ap.add_argument("--no-sampled", action="store_true", help="skip the sampled-gauge-source line")
     ap.add_argument("--no-adjoint", action="store_true", help="skip the adjoint's cost line")
     ap.add_argument("--nblocks", type=int, default=16, help="blocks per axis (16 = the full workload)")
-    ap.add_argument("--form", choices=tuple(FORMS), default="brick-split",
-                    help="the stepper's layout and kernels: the brick layout (default), or the "
-                         "per-block work arrays with one fused kernel or head + Pi launches")
+    ap.add_argument("--form", choices=tuple(FORMS), default="brick",
+                    help="the stepper's layout and kernels: the library's default (the brick layout, one "
+                         "kernel a stage), the brick's head + Pi launches, or the per-block work arrays")
     ap.add_argument("--no-plain", action="store_true", help="skip the plain (verbs) form")
     ap.add_argument("--no-per-block", action="store_true", help="skip the plain per-block form")
     ap.add_argument("--no-batch", action="store_true", help="skip the four-hole batch")
@@ -614,7 +614,7 @@ def main():
     f_pi = f_rhs - f_head
     # Per launch: F per point of that kernel's half over the N^3 points of each
     # block, plus its half of a quarter of the stage combination.
-    if not args.form.endswith("split"):
+    if not prof[5]:  # one kernel a stage
         head_tf = (f_rhs + f_combine / 4) * points / (head_ms * 1e-3) / 1e12
         pi_tf = None
         dom = args.form

@@ -15,8 +15,9 @@
  * message of the last failure on the calling thread. All work is ordered on
  * the problem's HIP stream and every verb synchronises before returning.
  * Device memory is allocated by tgh_problem_create and tgh_batch_create,
- * by the first brick-layout step and the first constraint monitor, and by
- * tgh_transfer for its plan (freed before it returns).
+ * by the first brick-layout step, the first right-hand side or step of a hole
+ * (its layer's targets), the first constraint monitor, and by tgh_transfer for
+ * its plan (freed before it returns).
  */
 #ifndef TGH_H
 #define TGH_H
@@ -79,11 +80,11 @@ enum { /* tgh_rk4 flags */
                          layout (every point once, a frame of ghosts around
                          the whole brick) */
   TGH_RK4_SPLIT = 8,  /* the right-hand side as two launches: the head (with
-                         d_t h) and the ten Pi components (on the block layout
-                         each block run as a brick, LDS-tiled, where the case
-                         has no bounds, :pasted core, matter, sampled source
-                         or general interior); without FUSED or SPLIT the
-                         layout's faster form is used */
+                         d_t h) and the ten Pi components; on the block layout,
+                         where the case has no bounds, :pasted core, matter or
+                         general interior, each block run as a brick in tiles;
+                         without FUSED or SPLIT the layout's faster form is
+                         used (the brick's is FUSED) */
   TGH_RK4_PER_BLOCK = 16 /* the plain per-block form: the per-block work arrays
                          and the fused kernel launched once per block and
                          stage (implies BLOCKS and FUSED; the baseline the
@@ -321,7 +322,7 @@ int tgh_add_noise(tgh_problem* p, double* u, uint64_t base, double amplitude);
  * TGH_RK4_BLOCKS is set; either way every owned point of u, face copies
  * included, advances as the reference steps its state vector (a copy by its
  * primary's increment). The first call in the brick layout allocates its
- * arrays (4 x 20 doubles per point of the ghosted brick, and 24 more with
+ * arrays (4 x 20 doubles per point of the ghosted brick, and 25 more with
  * TGH_RK4_SPLIT). */
 int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int32_t flags);
 /* gh_constraint!(p, u, t) then constraint_norms(p)'s gauge rows
@@ -375,16 +376,16 @@ int tgh_autotune(tgh_problem* p, double* u, double t0, double dt, double* ms);
  * 0 is the default). */
 int tgh_set_tile(tgh_problem* p, int32_t tile);
 /* Several independent problems stepped together (the batched form: holes of
- * uneven block counts in one launch per kernel, driven by a device-side table
+ * uneven block counts in one launch per stage, driven by a device-side table
  * of each problem's ranges and arguments). The reference steps each problem
  * by its own gh_solve (src/stepping.jl:208-239); a problem in a batch computes
- * the bits tgh_rk4 computes for it alone in the brick layout's split form.
+ * the bits tgh_rk4 computes for it alone in the brick layout's default form.
  * With a forest with levels or a tracked or :fitted interior among them the
- * batch runs on the block layout instead (one head and one Pi launch over
- * every block of every problem per stage, each problem computing the bits of
- * tgh_rk4 with TGH_RK4_BLOCKS | TGH_RK4_SPLIT; with a range projection or a
- * general interior among them one fused launch, the bits of TGH_RK4_BLOCKS |
- * TGH_RK4_FUSED), and moving holes are refused there
+ * batch runs on the block layout instead (one launch over every block of
+ * every problem per stage, each problem computing the bits of tgh_rk4 with
+ * TGH_RK4_BLOCKS | TGH_RK4_SPLIT; with a range projection or a general
+ * interior among them the bits of TGH_RK4_BLOCKS | TGH_RK4_FUSED), and moving
+ * holes are refused there
  * (TGH_EUNSUPPORTED). The problems share the order q, the gauge-source kind
  * and the kind of interior (one kernel specialisation), and none is :pasted;
  * each keeps its own arrays (brick arrays allocated here if missing). The

@@ -1787,8 +1787,8 @@ def gh_solve_regrid(p, u, tspan, *, cfl, every, refinement, graph=False):
 
 class GHBatch:
     """Several independent problems (holes of uneven block counts) stepped
-    together: each RK4 stage is one head and one Pi launch over all of them,
-    driven by a device-side table of the problems' ranges and arguments. The
+    together: each RK4 stage is one launch over all of them, driven by a
+    device-side table of the problems' ranges and arguments. The
     problems share q, the gauge-source kind and whether they have an interior;
     each computes the bits gh_solve computes for it alone. No reference
     counterpart: the reference steps each problem by its own gh_solve

@@ -420,8 +420,7 @@ dim3 tgh::grid_brick_tiles(const tgh_problem* p, int tx, int ty, int tz) {
 namespace {
 
 // ---------------------------------------------------------------------------
-// The brick stepper. Its default right-hand side form (measured on MI355X):
-constexpr bool kBrickSplitDefault = true;
+// The brick stepper.
 void launch_frame(tgh_problem* p, double* W, double t, double toff = 0.0) {
   const Brick& k = p->brick;
   const long E = (long)(k.n[0] + 2 * k.G) * (k.n[1] + 2 * k.G) * (k.n[2] + 2 * k.G);
@@ -440,30 +439,35 @@ bool static_background(const CaseP& c) {
   return !c.moving && (kind == BG_MINKOWSKI || kind == BG_KERR_SCHILD || kind == BG_SHIFTED || kind == BG_HARMONIC);
 }
 
-// The layer box (k_brick_layer) of a moving :damped hole or of a harmonic hole
-// at rest, on the finest level's grid: the layer's bounding box about c(t) with
+// The layer box (k_brick_layer) of a moving :damped hole or of a hole at
+// rest, on the finest level's grid: the layer's bounding box about c(t) with
 // a point of margin each side, whatever t (slots wrap modulo B). Nothing for
 // other cases.
 Brick layer_grid(const tgh_problem* p);
 int ensure_layer_box(tgh_problem* p) {
-  if (p->Blayer || p->cs.general || p->cs.interior == INT_NONE) return TGH_OK;
+  if (p->Blayer || p->cs.general || p->cs.interior == INT_NONE || p->cs.interior == INT_PASTED) return TGH_OK;
   const bool moving = p->cs.moving && p->cs.interior == INT_DAMPED;
-  // a harmonic hole at rest (no gauge source): its layer's target is a dual
-  // pass of the harmonic chart, the same at every t, so the box is filled once
-  const bool harmonic = !p->cs.moving && p->cs.gauge == GAUGE_NONE;
-  if (!moving && !harmonic) return TGH_OK;
+  // a hole at rest: its layer's target is the same at every t, so the box is filled once
+  const bool rest = !p->cs.moving;
+  if (!moving && !rest) return TGH_OK;
   int lmax = 0;
   for (int l : p->level_host) lmax = std::max(lmax, l);
   p->layer_lmax = lmax;
   p->layer_B = 2 * (int)std::ceil(p->cs.r1 * p->geom.inv_h * (double)(1 << lmax)) + 4;
-  const size_t lb = sizeof(double) * LAYER_FIELDS * (size_t)p->layer_B * p->layer_B * p->layer_B;
+  const size_t lb = sizeof(double) * (moving ? LAYER_FIELDS : 20) * (size_t)p->layer_B * p->layer_B * p->layer_B;
   hipError_t e = hipMalloc(&p->Blayer, lb);
   if (e != hipSuccess) {
     p->Blayer = nullptr;
+    // a sourced hole at rest has its target in closed form too: without the
+    // box the stepper takes the split form, whose head evaluates it
+    if (rest && p->cs.gauge != GAUGE_NONE) {
+      (void)hipGetLastError();
+      return TGH_OK;
+    }
     return fail(TGH_EDEVICE, std::string("allocating the layer box: ") + hipGetErrorString(e));
   }
-  p->layer_static = harmonic;
-  if (harmonic) {
+  p->layer_static = rest;
+  if (rest) {
     const long B3 = (long)p->layer_B * p->layer_B * p->layer_B;
     LayerArgs la{layer_grid(p), p->cs, 0.0, nullptr, 0.0, p->Blayer, p->layer_B};
     hipLaunchKernelGGL(k_brick_layer<false>, dim3((unsigned)((B3 + 255) / 256), 1), dim3(256), 0, p->stream, la);
@@ -530,10 +534,8 @@ int ensure_brick(tgh_problem* p) {
   const bool static_bg = static_background(p->cs);
   // a wrapped or mirrored frame reads the stage's own values: refilled every stage
   p->frame_static = static_bg && !g.periodic[0] && !g.periodic[1] && !g.periodic[2] && !reflects(g);
-  if (p->frame_static) {
-    launch_frame(p, p->BW[0], 0.0);
-    launch_frame(p, p->BW[1], 0.0);
-  }
+  if (p->frame_static)  // every array is a stage input in one of the forms
+    for (double** a : arrs) launch_frame(p, *a, 0.0);
   {
     const int rc = ensure_layer_box(p);
     if (rc) return rc;
@@ -553,38 +555,84 @@ int ensure_brick(tgh_problem* p) {
 void launch_bounds_brick(tgh_problem* p, double* A, double* B);
 void launch_paste(tgh_problem* p, int mode, double* A, double* B, double t, double toff = 0.0);
 
-// One RK4 step on the brick arrays (u_n in Bus, the stage input in BW[0]).
-void rk4_brick_launches(tgh_problem* p, double t, double dt) {
+// Whether the one-kernel stage runs this problem: its interior's targets come
+// from the layer box (a :pasted interior has no layer).
+bool stage_ok(const tgh_problem* p) {
+  return p->cs.interior == INT_NONE || p->cs.interior == INT_PASTED || p->Blayer != nullptr;
+}
+// Whether its stages keep the stage values instead of an accumulator (StageIO):
+// not where a limiter or the fill changes them.
+bool stage_values(const tgh_problem* p) {
+  return !p->has_bounds && p->cs.interior != INT_PASTED && !reflects(p->geom);
+}
+void launch_stage(tgh_problem* p, const RhsArgs& a, const StageIO& io) {
+  switch (p->q) {
+    case 2: launch_stage_brick<2>(p, a, io); break;
+    case 4: launch_stage_brick<4>(p, a, io); break;
+    case 6: launch_stage_brick<6>(p, a, io); break;
+    default: launch_stage_brick<8>(p, a, io); break;
+  }
+}
+void launch_split(tgh_problem* p, const RhsArgs& a) {
+  switch (p->q) {
+    case 2: launch_rhs_brick<2>(p, a); break;
+    case 4: launch_rhs_brick<4>(p, a); break;
+    case 6: launch_rhs_brick<6>(p, a); break;
+    default: launch_rhs_brick<8>(p, a); break;
+  }
+}
+// The stage's arguments on the brick: its ghosts and, for a moving hole, its
+// layer box are filled first.
+RhsArgs brick_stage_args(tgh_problem* p, double* Wc, double t, double toff) {
+  if (!p->frame_static) {
+    const bool prof = p->profiling;
+    int e0 = prof ? mark(p) : -1;
+    launch_frame(p, Wc, t, toff);
+    if (prof) p->ev_fill.push_back({e0, mark(p)});
+  }
+  RhsArgs a = rhs_args(p, Wc, t, nullptr);
+  a.clock = p->clock_use;
+  a.toff = toff;
+  if (p->Blayer) launch_layer_box(p, t, toff, a);
+  a.Hsrc = p->BH;
+  return a;
+}
+
+// Stage s's arrays in the stage-value form, Y[0] = u_n, Y[s] the stage input,
+// the result in out.
+StageIO stage_io(double* const Y[4], double* out, int s, double dt) {
+  const double c_next[4] = {dt / 2, dt / 2, dt, 0.0};
+  return StageIO{STAGE_Y1 + s, dt / 6, c_next[s], Y[0], nullptr, Y[1], Y[2], out};
+}
+
+// One RK4 step on the brick arrays. In the stage-value form u_n and u_{n+1}
+// are in BW[0] and Y1, Y2, Y3 in BW[1], Bus and Bacc; otherwise u_n is in Bus
+// and, as the first stage's input, in BW[0], and Bacc accumulates.
+void rk4_brick_launches(tgh_problem* p, double t, double dt, bool split) {
   const double c_acc[4] = {dt / 6, dt / 3, dt / 3, dt / 6};
   const double c_next[4] = {dt / 2, dt / 2, dt, 0.0};
   const double t_off[4] = {0.0, dt / 2, dt / 2, dt};
   const double t_stage[4] = {t, t + dt / 2, t + dt / 2, t + dt};
+  if (!split && stage_values(p)) {
+    double* const Y[4] = {p->BW[0], p->BW[1], p->Bus, p->Bacc};
+    for (int s = 0; s < 4; ++s)
+      launch_stage(p, brick_stage_args(p, Y[s], t_stage[s], t_off[s]), stage_io(Y, Y[(s + 1) % 4], s, dt));
+    return;
+  }
   for (int s = 0; s < 4; ++s) {
     double* Wc = p->BW[s % 2];
     double* Wn = p->BW[(s + 1) % 2];
-    if (!p->frame_static) {
-      const bool prof = p->profiling;
-      int e0 = prof ? mark(p) : -1;
-      launch_frame(p, Wc, t_stage[s], t_off[s]);
-      if (prof) p->ev_fill.push_back({e0, mark(p)});
-    }
-    RhsArgs a = rhs_args(p, Wc, t_stage[s], nullptr);
-    a.clock = p->clock_use;
-    a.toff = t_off[s];
-    if (p->Blayer) launch_layer_box(p, t_stage[s], t_off[s], a);
-    a.Hsrc = p->BH;
+    RhsArgs a = brick_stage_args(p, Wc, t_stage[s], t_off[s]);
     a.us = p->Bus;
     a.acc = p->Bacc;
     a.Wn = Wn;
     a.cacc = c_acc[s];
     a.cnext = c_next[s];
     a.stage = s + 1;
-    switch (p->q) {
-      case 2: launch_rhs_brick<2>(p, a); break;
-      case 4: launch_rhs_brick<4>(p, a); break;
-      case 6: launch_rhs_brick<6>(p, a); break;
-      default: launch_rhs_brick<8>(p, a); break;
-    }
+    if (split)
+      launch_split(p, a);
+    else
+      launch_stage(p, a, StageIO{s + 1, c_acc[s], c_next[s], p->Bus, p->Bus, p->Bacc, nullptr, Wn});
     // the stage limiter on the stage value (and on the step's result): the
     // range projection, then the :pasted overwrite
     if (p->has_bounds) launch_bounds_brick(p, s == 3 ? p->Bus : Wn, s == 3 ? Wn : nullptr);
@@ -593,6 +641,8 @@ void rk4_brick_launches(tgh_problem* p, double t, double dt) {
                    t_off[s < 3 ? s + 1 : 3]);
   }
 }
+// The brick array that holds u_n between steps.
+double* brick_un(tgh_problem* p, bool split) { return !split && stage_values(p) ? p->BW[0] : p->Bus; }
 
 // The range projection on the state (mode 0, with accounting partials), on
 // a block work array's owned points (+ the state), or on the brick points
@@ -655,10 +705,32 @@ void launch_paste(tgh_problem* p, int mode, double* A, double* B, double t, doub
   hipLaunchKernelGGL(p->cs.moving ? k_paste<true> : k_paste<false>, grid, dim3(256), 0, p->stream, a);
 }
 
-// One RK4 step on the block layout run as bricks (form 5): u_n in Wus, the
-// accumulator in Wacc, the coefficients in Wcoef (all in the work layout), the
-// stage input in W[0] holding u_n with its ghosts unfilled.
-void rk4_block_lds_launches(tgh_problem* p, double t, double dt) {
+// One stage in one kernel on the block layout.
+void launch_stage_block(tgh_problem* p, const RhsArgs& a, const StageIO& io) {
+  switch (p->q) {
+    case 2: launch_stage_blocks<2>(p, a, io); break;
+    case 4: launch_stage_blocks<4>(p, a, io); break;
+    case 6: launch_stage_blocks<6>(p, a, io); break;
+    default: launch_stage_blocks<8>(p, a, io); break;
+  }
+}
+// Whether the block layout runs each block's work array as a brick in tiles
+// (form 5): not with bounds, :pasted, matter or the general interior.
+bool block_stage_ok(const tgh_problem* p) {
+  return !p->has_bounds && p->cs.interior != INT_PASTED && !p->mat.rho && !p->cs.general && stage_ok(p);
+}
+int ensure_block_stage(tgh_problem* p) {
+  if (p->Wus) return TGH_OK;
+  const size_t wbytes = sizeof(double) * (size_t)p->work_len;
+  HIP_TRY(hipMalloc(&p->Wus, wbytes));
+  HIP_TRY(hipMalloc(&p->Wacc, wbytes));
+  return TGH_OK;
+}
+// One RK4 step on the block layout in tiles (form 5): u_n in Wus, the
+// accumulator in Wacc (both in the work layout), the stage input in W[0]
+// holding u_n with its ghosts unfilled. The stage values cannot stand in for
+// the accumulator here: the fill overwrites the face copies' own.
+void rk4_block_stage_launches(tgh_problem* p, double t, double dt) {
   const double c_acc[4] = {dt / 6, dt / 3, dt / 3, dt / 6};
   const double c_next[4] = {dt / 2, dt / 2, dt, 0.0};
   const double t_off[4] = {0.0, dt / 2, dt / 2, dt};
@@ -674,16 +746,7 @@ void rk4_block_lds_launches(tgh_problem* p, double t, double dt) {
     a.clock = p->clock_use;
     a.toff = t_off[s];
     if (p->Blayer) launch_layer_box(p, t_stage[s], t_off[s], a);
-    a.cacc = c_acc[s];
-    a.cnext = c_next[s];
-    a.stage = s + 1;
-    const BlockBricks bb{Wc, p->Wcoef, p->Wus, p->Wacc, Wn, p->layer_lmax};
-    switch (p->q) {
-      case 2: launch_rhs_blocks_lds<2>(p, a, bb); break;
-      case 4: launch_rhs_blocks_lds<4>(p, a, bb); break;
-      case 6: launch_rhs_blocks_lds<6>(p, a, bb); break;
-      default: launch_rhs_blocks_lds<8>(p, a, bb); break;
-    }
+    launch_stage_block(p, a, StageIO{s + 1, c_acc[s], c_next[s], p->Wus, p->Wus, p->Wacc, nullptr, Wn});
   }
 }
 
@@ -1146,7 +1209,6 @@ int tgh_problem_destroy(tgh_problem* p) {
   (void)hipFree(p->d_clock);
   (void)hipFree(p->Wus);
   (void)hipFree(p->Wacc);
-  (void)hipFree(p->Wcoef);
   (void)hipFree(p->Blayer);
   (void)hipFree(p->d_bcoord);
   (void)hipFree(p->d_lookup);
@@ -1548,41 +1610,35 @@ int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int
   if ((flags & TGH_RK4_FUSED) && (flags & TGH_RK4_SPLIT))
     return fail(TGH_EINVAL, "TGH_RK4_FUSED and TGH_RK4_SPLIT exclude each other");
   // forms: 0 block layout, head + Pi; 1 block layout, fused; 2 brick layout,
-  // fused; 3 brick layout, head + LDS-tiled Pi; 4 block layout, fused, one
-  // launch per block; 5 block layout, each block run as a brick by the
-  // brick's head and LDS-tiled Pi kernel (not with bounds, :pasted, matter,
-  // the sampled source or the general interior: form 0 there). Without FUSED
-  // or SPLIT the layout's faster form on MI355X (measured: the brick's split
-  // form; on the block layout form 5 where it runs, else the fused kernel).
-  const bool lds_ok = !p->has_bounds && p->cs.interior != INT_PASTED && !p->mat.rho &&
-                      p->cs.gauge != GAUGE_SAMPLED && !p->cs.general;
-  const bool split = (flags & TGH_RK4_SPLIT) != 0 ||
-                     (!(flags & TGH_RK4_FUSED) && (blocks ? lds_ok : kBrickSplitDefault));
+  // one kernel a stage; 3 brick layout, head + LDS-tiled Pi; 4 block layout,
+  // fused, one launch per block; 5 block layout, each block run as a brick in
+  // one kernel a stage (block_stage_ok; else form 0). Without FUSED or SPLIT the layout's faster form on MI355X (measured: the
+  // brick's one kernel a stage; on the block layout form 5 where it runs,
+  // else the fused kernel).
+  {
+    int rc = blocks ? ensure_layer_box(p) : ensure_brick(p);
+    if (rc) return rc;
+  }
+  const bool lds_ok = block_stage_ok(p);
+  const bool split = (flags & TGH_RK4_SPLIT) != 0 || (!(flags & TGH_RK4_FUSED) && blocks && lds_ok) ||
+                     (!blocks && !stage_ok(p));
   const int form = (flags & TGH_RK4_PER_BLOCK) ? 4 : blocks ? (split ? (lds_ok ? 5 : 0) : 1) : (split ? 3 : 2);
   const bool in_brick = form == 2 || form == 3;
   if (in_brick) {
-    int rc = ensure_brick(p);
-    if (rc) return rc;
     if (form == 3 && !p->Bcoef) {
       HIP_TRY(hipMalloc(&p->Bcoef, sizeof(double) * CF_N * (size_t)p->brick.fs));
       HIP_TRY(hipMemsetAsync(p->Bcoef, 0, sizeof(double) * CF_N * (size_t)p->brick.fs, p->stream));
     }
-    // u_n into the stepper's u_n and first stage input
-    BrickCopyArgs ca{p->geom, p->brick, u, p->BW[0], p->Bus, 0};
+    // u_n into the first stage input, and into the stepper's u_n where that is another array
+    double* un = brick_un(p, split);
+    BrickCopyArgs ca{p->geom, p->brick, u, p->BW[0], un == p->BW[0] ? nullptr : un, 0};
     hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, p->stream, ca);
   } else {
-    int rc = ensure_layer_box(p);
-    if (rc) return rc;
     // the first stage input: u_n scattered into W[0]
     launch_scatter(p, u, p->W[0], 1);
     if (form == 5) {
-      const size_t wbytes = sizeof(double) * (size_t)p->work_len;
-      if (!p->Wus) {
-        HIP_TRY(hipMalloc(&p->Wus, wbytes));
-        HIP_TRY(hipMalloc(&p->Wacc, wbytes));
-        HIP_TRY(hipMalloc(&p->Wcoef, wbytes / 20 * CF_N));
-        HIP_TRY(hipMemsetAsync(p->Wcoef, 0, wbytes / 20 * CF_N, p->stream));
-      }
+      int rc = ensure_block_stage(p);
+      if (rc) return rc;
       launch_scatter(p, u, p->Wus, 1);  // and u_n, in the work layout too
     }
   }
@@ -1590,13 +1646,13 @@ int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int
     HIP_TRY(hipGraphExecDestroy(p->graph_exec));
     p->graph_exec = nullptr;
   }
-  p->fused = form == 1 || form == 2 || form == 4;
+  p->fused = form == 1 || form == 4;
   p->per_block = form == 4;
   auto step = [&](double t) {
     if (in_brick)
-      rk4_brick_launches(p, t, dt);
+      rk4_brick_launches(p, t, dt, split);
     else if (form == 5)
-      rk4_block_lds_launches(p, t, dt);
+      rk4_block_stage_launches(p, t, dt);
     else
       rk4_step_launches(p, u, t, dt);
   };
@@ -1661,7 +1717,7 @@ int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int
   if (rc == TGH_OK && in_brick) {
     // u_{n+1} back into the state: the copies, then the primaries
     for (int pass = 0; pass < 2; ++pass) {
-      BrickCopyArgs ca{p->geom, p->brick, p->Bus, u, nullptr, pass};
+      BrickCopyArgs ca{p->geom, p->brick, brick_un(p, split), u, nullptr, pass};
       hipLaunchKernelGGL(k_brick_out, grid_points(p), dim3(256), 0, p->stream, ca);
     }
   }
@@ -1730,26 +1786,25 @@ int adj_theta(tgh_problem* p, double* out) {
   return TGH_OK;
 }
 
-// One RK4 stage on explicit brick arrays (rk4_brick_launches' stage s with
-// the stage input Wc and the next stage's Wn).
-void brick_stage(tgh_problem* p, double* Wc, double* Wn, double t, double dt, int s) {
+// The stage inputs of one step from u_n = Y[0]: Y[1 .. 3], and u_{n+1} in Y[4].
+void brick_step_slots(tgh_problem* p, double* const Y[5], double t, double dt) {
   const double c_acc[4] = {dt / 6, dt / 3, dt / 3, dt / 6};
   const double c_next[4] = {dt / 2, dt / 2, dt, 0.0};
   const double t_stage[4] = {t, t + dt / 2, t + dt / 2, t + dt};
-  if (!p->frame_static) launch_frame(p, Wc, t_stage[s]);
-  RhsArgs a = rhs_args(p, Wc, t_stage[s], nullptr);
-  a.Hsrc = p->BH;
-  a.us = p->Bus;
-  a.acc = p->Bacc;
-  a.Wn = Wn;
-  a.cacc = c_acc[s];
-  a.cnext = c_next[s];
-  a.stage = s + 1;
-  switch (p->q) {
-    case 2: launch_rhs_brick<2>(p, a); break;
-    case 4: launch_rhs_brick<4>(p, a); break;
-    case 6: launch_rhs_brick<6>(p, a); break;
-    default: launch_rhs_brick<8>(p, a); break;
+  const bool split = !stage_ok(p);
+  for (int s = 0; s < 4; ++s) {
+    RhsArgs a = brick_stage_args(p, Y[s], t_stage[s], 0.0);
+    if (!split) {
+      launch_stage(p, a, stage_io(Y, Y[s + 1], s, dt));
+      continue;
+    }
+    a.us = p->Bus;
+    a.acc = p->Bacc;
+    a.Wn = Y[s + 1];
+    a.cacc = c_acc[s];
+    a.cnext = c_next[s];
+    a.stage = s + 1;
+    launch_split(p, a);
   }
 }
 
@@ -1800,7 +1855,7 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
     HIP_TRY(hipMalloc(&p->adjCkpt, nseg * fb20));
     p->adjCkptN = nseg;
   }
-  if (!p->Bcoef) {
+  if (!stage_ok(p) && !p->Bcoef) {
     HIP_TRY(hipMalloc(&p->Bcoef, sizeof(double) * CF_N * (size_t)k.fs));
     HIP_TRY(hipMemsetAsync(p->Bcoef, 0, sizeof(double) * CF_N * (size_t)k.fs, p->stream));
   }
@@ -1808,7 +1863,7 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
   auto ckpt = [&](size_t i) { return p->adjCkpt + i * 20 * (size_t)k.fs; };
   hipEvent_t ev[4];
   for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
-  p->fused = false;  // the split form (head + LDS-tiled Pi), the stepper's default
+  const bool split = !stage_ok(p);  // as tgh_rk4's default
   // ---- forward: u_0 into the brick, a checkpoint at each segment's start ----
   HIP_TRY(hipEventRecord(ev[0], p->stream));
   BrickCopyArgs ca{p->geom, k, u, p->BW[0], p->Bus, 0};
@@ -1816,11 +1871,11 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
   for (size_t sg = 0; sg < nseg; ++sg) {
     HIP_TRY(hipMemcpyAsync(ckpt(sg), p->BW[0], fb20, hipMemcpyDeviceToDevice, p->stream));
     const int n0 = (int)(sg * every), n1 = std::min(nsteps, (int)((sg + 1) * every));
-    for (int n = n0; n < n1; ++n) rk4_brick_launches(p, t0 + n * dt, dt);
+    for (int n = n0; n < n1; ++n) rk4_brick_launches(p, t0 + n * dt, dt, split);
   }
   HIP_TRY(hipEventRecord(ev[1], p->stream));
   for (int pass = 0; pass < 2; ++pass) {
-    BrickCopyArgs co{p->geom, k, p->Bus, u, nullptr, pass};
+    BrickCopyArgs co{p->geom, k, brick_un(p, split), u, nullptr, pass};
     hipLaunchKernelGGL(k_brick_out, grid_points(p), dim3(256), 0, p->stream, co);
   }
   // J = the masked L2 error at T, and lambda_T = dJ/du_T
@@ -1834,7 +1889,7 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
   }
   *J = den > 0 ? std::sqrt(num / den) : 0.0;
   double *lam = p->adjL[0], *lacc = p->adjL[1], *kb = p->adjK[0], *kbn = p->adjK[1];
-  launch_adj_init(p, AdjInitArgs{k, p->cs, T, *J, den, dt / 6, p->Bus, lam, kb});
+  launch_adj_init(p, AdjInitArgs{k, p->cs, T, *J, den, dt / 6, brick_un(p, split), lam, kb});
   HIP_TRY(hipMemsetAsync(p->adjTh, 0, sizeof(double) * ADJ_NPAR * adj_runs(k), p->stream));
   // ---- backward: per segment, its stage inputs recomputed from the
   // checkpoint, then its steps reversed ----
@@ -1843,9 +1898,11 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
   for (size_t sg = nseg; sg-- > 0;) {
     const int n0 = (int)(sg * every), n1 = std::min(nsteps, (int)((sg + 1) * every)), ns = n1 - n0;
     HIP_TRY(hipMemcpyAsync(slot(0), ckpt(sg), fb20, hipMemcpyDeviceToDevice, p->stream));
-    HIP_TRY(hipMemcpyAsync(p->Bus, ckpt(sg), fb20, hipMemcpyDeviceToDevice, p->stream));
-    for (int j = 0; j < ns; ++j)
-      for (int s = 0; s < 4; ++s) brick_stage(p, slot(4 * j + s), slot(4 * j + s + 1), t0 + (n0 + j) * dt, dt, s);
+    if (split) HIP_TRY(hipMemcpyAsync(p->Bus, ckpt(sg), fb20, hipMemcpyDeviceToDevice, p->stream));
+    for (int j = 0; j < ns; ++j) {
+      double* const Y[5] = {slot(4 * j), slot(4 * j + 1), slot(4 * j + 2), slot(4 * j + 3), slot(4 * j + 4)};
+      brick_step_slots(p, Y, t0 + (n0 + j) * dt, dt);
+    }
     for (int j = ns; j-- > 0;) {
       const double t = t0 + (n0 + j) * dt;
       const double t_stage[4] = {t, t + dt / 2, t + dt / 2, t + dt};
@@ -1947,22 +2004,22 @@ int tgh_copy_work(tgh_problem* p, double* dst) {
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
-// Batches: several problems stepped by one head and one Pi launch per stage.
+// Batches: several problems stepped by one launch per stage.
 struct tgh_batch {
   std::vector<tgh_problem*> probs;
   int q = 4, gauge = 0;
-  int hole = 0;  // the head's interior kind: 0, 1 (the sphere) or HOLE_BOXED
+  int hole = 0;  // whether the problems have an interior
   // The block layout (a problem on a forest with levels or with the general
   // interior among them): one fused launch over every block of every problem
   // per stage; the RK4 epilogue writes the states in place, so the tables and
   // the graph hold the states' pointers.
   bool blocks = false;
-  bool lds = false;                  // the block layout with its blocks run as bricks
+  bool lds = false;                  // the block layout in tiles, one kernel a stage
   int hole_kind = 0;                 // 0 none, 1 the sphere, 2 the general interior
   std::vector<double*> tab_u, graph_u;
   BatchEntry* d_tab = nullptr;  // 4 stage tables of n entries
   BatchEntry* h_tab = nullptr;  // pinned staging of the tables
-  int head_total = 0, pi_total = 0;
+  int total = 0;                // logical workgroups of a stage's launch
   double tab_key[2] = {0, 0};   // (dt, t) the uploaded tables hold
   std::vector<unsigned> tab_ver;  // the problems' versions the tables were built from
   bool tab_valid = false;
@@ -1977,13 +2034,23 @@ struct tgh_batch {
 };
 
 namespace {
-void pi_tile_dims(int q, int& tx, int& ty, int& tz) {
-  switch (q) {
-    case 2: tx = PiTile<2>::X; ty = PiTile<2>::Y; tz = PiTile<2>::Z * PiTile<2>::PZ; break;
-    case 4: tx = PiTile<4>::X; ty = PiTile<4>::Y; tz = PiTile<4>::Z * PiTile<4>::PZ; break;
-    case 6: tx = PiTile<6>::X; ty = PiTile<6>::Y; tz = PiTile<6>::Z * PiTile<6>::PZ; break;
-    default: tx = PiTile<8>::X; ty = PiTile<8>::Y; tz = PiTile<8>::Z * PiTile<8>::PZ; break;
+int stage_tiles(const tgh_problem* p) {  // the brick's tiles in a launch
+  switch (p->q) {
+    case 2: return brick_stage_tiles<2>(p->brick);
+    case 4: return brick_stage_tiles<4>(p->brick);
+    case 6: return brick_stage_tiles<6>(p->brick);
+    default: return brick_stage_tiles<8>(p->brick);
   }
+}
+// Stage s of a table entry: its arrays and coefficients.
+void entry_io(BatchEntry& e, const StageIO& io) {
+  e.a.stage = io.stage;
+  e.a.cacc = io.cacc;
+  e.a.cnext = io.cnext;
+  e.us = (decltype(e.us))io.us;
+  e.acc = (decltype(e.acc))io.acc;
+  e.y2 = (decltype(e.y2))io.y2;
+  e.Wn = (decltype(e.Wn))io.out;
 }
 // The stage tables at step time t: problem i's stage-s arguments, as
 // rk4_brick_launches sets them for the problem alone.
@@ -1992,46 +2059,32 @@ int batch_tables(tgh_batch* b, double t, double dt) {
   const double c_acc[4] = {dt / 6, dt / 3, dt / 3, dt / 6};
   const double c_next[4] = {dt / 2, dt / 2, dt, 0.0};
   const double t_stage[4] = {t, t + dt / 2, t + dt / 2, t + dt};
-  int h0 = 0, p0 = 0, tx, ty, tz;
-  pi_tile_dims(b->q, tx, ty, tz);
+  int w0 = 0;
   for (int i = 0; i < n; ++i) {
     tgh_problem* p = b->probs[i];
-    const Brick& k = p->brick;
-    const long plane = (long)k.n[0] * k.n[1];
-    const int runs = (int)((plane + 255) / 256) * k.n[2];
-    const int tiles = ((k.n[0] + tx - 1) / tx) * ((k.n[1] + ty - 1) / ty) * ((k.n[2] + tz - 1) / tz);
+    double* const Y[4] = {p->BW[0], p->BW[1], p->Bus, p->Bacc};
+    const bool values = stage_values(p);
     for (int s = 0; s < 4; ++s) {
       BatchEntry& e = b->h_tab[s * n + i];
-      e.a = rhs_args(p, p->BW[s % 2], t_stage[s], nullptr);
+      std::memset(&e, 0, sizeof(e));
+      double* Wc = values ? Y[s] : p->BW[s % 2];
+      e.a = rhs_args(p, Wc, t_stage[s], nullptr);
       e.a.Hsrc = p->BH;
-      e.a.us = p->Bus;
-      e.a.acc = p->Bacc;
-      e.a.Wn = p->BW[(s + 1) % 2];
-      e.a.du = nullptr;
-      e.a.coef = p->Bcoef;
-      e.a.cacc = c_acc[s];
-      e.a.cnext = c_next[s];
-      e.a.stage = s + 1;
-      if (b->hole == HOLE_BOXED) {
+      if (p->Blayer) {
         e.a.lbox = p->Blayer;
         e.a.lB3 = (long)p->layer_B * p->layer_B * p->layer_B;
         e.a.lB = p->layer_B;
       }
-      e.k = k;
+      e.k = p->brick;
       e.W = (decltype(e.W))e.a.W;
       e.Hsrc = (decltype(e.Hsrc))e.a.Hsrc;
-      e.coef = (decltype(e.coef))e.a.coef;
-      e.us = (decltype(e.us))e.a.us;
-      e.acc = (decltype(e.acc))e.a.acc;
-      e.Wn = (decltype(e.Wn))e.a.Wn;
-      e.head0 = h0;
-      e.pi0 = p0;
+      entry_io(e, values ? stage_io(Y, Y[(s + 1) % 4], s, dt)
+                         : StageIO{s + 1, c_acc[s], c_next[s], p->Bus, p->Bus, p->Bacc, nullptr, p->BW[(s + 1) % 2]});
+      e.wg0 = w0;
     }
-    h0 += runs;
-    p0 += tiles;
+    w0 += stage_tiles(p);
   }
-  b->head_total = h0;
-  b->pi_total = p0;
+  b->total = w0;
   HIP_TRY(hipMemcpyAsync(b->d_tab, b->h_tab, sizeof(BatchEntry) * 4 * n, hipMemcpyHostToDevice, b->stream));
   // the pinned tables are rewritten only after this copy has run
   HIP_TRY(hipStreamSynchronize(b->stream));
@@ -2047,41 +2100,30 @@ int batch_tables_blocks(tgh_batch* b, double* const* u, double t, double dt) {
   const double c_acc[4] = {dt / 6, dt / 3, dt / 3, dt / 6};
   const double c_next[4] = {dt / 2, dt / 2, dt, 0.0};
   const double t_stage[4] = {t, t + dt / 2, t + dt / 2, t + dt};
-  int w0 = 0, pw0 = 0;
+  int w0 = 0;
   for (int i = 0; i < n; ++i) {
     tgh_problem* p = b->probs[i];
-    const int wgpb = (p->geom.P * p->geom.P * p->geom.P + 255) / 256;
+    const int wgpb = b->lds ? block_tiles(p->geom.P) : (p->geom.P * p->geom.P * p->geom.P + 255) / 256;
     for (int s = 0; s < 4; ++s) {
       BatchEntry& e = b->h_tab[s * n + i];
       std::memset(&e, 0, sizeof(e));
       e.a = rhs_args(p, p->W[s % 2], t_stage[s], nullptr);
-      e.a.us = b->lds ? p->Wus : u[i];
-      e.a.acc = b->lds ? p->Wacc : p->acc;
-      e.a.Wn = p->W[(s + 1) % 2];
-      e.a.du = nullptr;
-      e.a.cacc = c_acc[s];
-      e.a.cnext = c_next[s];
-      e.a.stage = s + 1;
-      if (b->lds) e.a.coef = p->Wcoef;
+      if (b->lds && p->Blayer) {
+        e.a.lbox = p->Blayer;
+        e.a.lB3 = (long)p->layer_B * p->layer_B * p->layer_B;
+        e.a.lB = p->layer_B;
+        e.a.lLmax = p->layer_lmax;
+      }
       e.W = (decltype(e.W))e.a.W;
       e.Hsrc = (decltype(e.Hsrc))e.a.Hsrc;
-      e.us = (decltype(e.us))e.a.us;
-      e.acc = (decltype(e.acc))e.a.acc;
-      e.Wn = (decltype(e.Wn))e.a.Wn;
-      e.coef = (decltype(e.coef))e.a.coef;
-      e.head0 = w0;
-      e.pi0 = pw0;
+      double* us = b->lds ? p->Wus : u[i];
+      entry_io(e, StageIO{s + 1, c_acc[s], c_next[s], us, us, b->lds ? p->Wacc : p->acc, nullptr, p->W[(s + 1) % 2]});
+      e.wg0 = w0;
       e.lLmax = p->layer_lmax;
     }
     w0 += wgpb * p->geom.nblocks;
-    if (b->lds) {
-      const int P = p->geom.P;
-      using T = PiTile<4, PI_TILE_BLOCK>;  // the block tile's shape is the same at every order
-      pw0 += ((P + T::X - 1) / T::X) * ((P + T::Y - 1) / T::Y) * ((P + T::Z - 1) / T::Z) * p->geom.nblocks;
-    }
   }
-  b->head_total = w0;
-  b->pi_total = pw0;
+  b->total = w0;
   HIP_TRY(hipMemcpyAsync(b->d_tab, b->h_tab, sizeof(BatchEntry) * 4 * n, hipMemcpyHostToDevice, b->stream));
   HIP_TRY(hipStreamSynchronize(b->stream));
   b->tab_key[0] = dt;
@@ -2089,6 +2131,15 @@ int batch_tables_blocks(tgh_batch* b, double* const* u, double t, double dt) {
   b->tab_u.assign(u, u + n);
   b->tab_valid = true;
   return TGH_OK;
+}
+void launch_batch_stage(tgh_batch* b, const BatchEntry* tab) {
+  const int n = (int)b->probs.size();
+  switch (b->q) {
+    case 2: launch_batch<2>(b->stream, tab, n, b->total, b->gauge, b->hole, b->blocks); break;
+    case 4: launch_batch<4>(b->stream, tab, n, b->total, b->gauge, b->hole, b->blocks); break;
+    case 6: launch_batch<6>(b->stream, tab, n, b->total, b->gauge, b->hole, b->blocks); break;
+    default: launch_batch<8>(b->stream, tab, n, b->total, b->gauge, b->hole, b->blocks); break;
+  }
 }
 void batch_step_launches_blocks(tgh_batch* b, double t, double dt) {
   const int n = (int)b->probs.size();
@@ -2098,19 +2149,13 @@ void batch_step_launches_blocks(tgh_batch* b, double t, double dt) {
     for (tgh_problem* p : b->probs) launch_fill(p, p->W[s % 2], t_stage[s], t_off[s]);
     const BatchEntry* tab = b->d_tab + s * n;
     if (b->lds) {
-      const int ht = b->head_total, pt = b->pi_total, hk = b->hole_kind ? 1 : 0;
-      switch (b->q) {
-        case 2: launch_batch_blocks_lds<2>(b->stream, tab, n, ht, pt, b->gauge, hk); break;
-        case 4: launch_batch_blocks_lds<4>(b->stream, tab, n, ht, pt, b->gauge, hk); break;
-        case 6: launch_batch_blocks_lds<6>(b->stream, tab, n, ht, pt, b->gauge, hk); break;
-        default: launch_batch_blocks_lds<8>(b->stream, tab, n, ht, pt, b->gauge, hk); break;
-      }
+      launch_batch_stage(b, tab);
     } else {
       switch (b->q) {
-        case 2: launch_batch_blocks<2>(b->stream, tab, n, b->head_total, b->gauge, b->hole_kind); break;
-        case 4: launch_batch_blocks<4>(b->stream, tab, n, b->head_total, b->gauge, b->hole_kind); break;
-        case 6: launch_batch_blocks<6>(b->stream, tab, n, b->head_total, b->gauge, b->hole_kind); break;
-        default: launch_batch_blocks<8>(b->stream, tab, n, b->head_total, b->gauge, b->hole_kind); break;
+        case 2: launch_batch_blocks<2>(b->stream, tab, n, b->total, b->gauge, b->hole_kind); break;
+        case 4: launch_batch_blocks<4>(b->stream, tab, n, b->total, b->gauge, b->hole_kind); break;
+        case 6: launch_batch_blocks<6>(b->stream, tab, n, b->total, b->gauge, b->hole_kind); break;
+        default: launch_batch_blocks<8>(b->stream, tab, n, b->total, b->gauge, b->hole_kind); break;
       }
     }
     for (int i = 0; i < n; ++i) {
@@ -2134,19 +2179,14 @@ void batch_step_launches(tgh_batch* b, double t, double dt) {
   const double t_stage[4] = {t, t + dt / 2, t + dt / 2, t + dt};
   for (int s = 0; s < 4; ++s) {
     for (tgh_problem* p : b->probs) {
-      if (!p->frame_static) launch_frame(p, p->BW[s % 2], t_stage[s], t_off[s]);
-      if (b->hole == HOLE_BOXED) {
-        RhsArgs unused = rhs_args(p, p->BW[s % 2], t_stage[s], nullptr);
+      double* const Y[4] = {p->BW[0], p->BW[1], p->Bus, p->Bacc};
+      if (!p->frame_static) launch_frame(p, stage_values(p) ? Y[s] : p->BW[s % 2], t_stage[s], t_off[s]);
+      if (p->Blayer) {
+        RhsArgs unused = rhs_args(p, p->BW[0], t_stage[s], nullptr);
         launch_layer_box(p, t_stage[s], t_off[s], unused);
       }
     }
-    const BatchEntry* tab = b->d_tab + s * n;
-    switch (b->q) {
-      case 2: launch_batch<2>(b->stream, tab, n, b->head_total, b->pi_total, b->gauge, b->hole); break;
-      case 4: launch_batch<4>(b->stream, tab, n, b->head_total, b->pi_total, b->gauge, b->hole); break;
-      case 6: launch_batch<6>(b->stream, tab, n, b->head_total, b->pi_total, b->gauge, b->hole); break;
-      default: launch_batch<8>(b->stream, tab, n, b->head_total, b->pi_total, b->gauge, b->hole); break;
-    }
+    launch_batch_stage(b, b->d_tab + s * n);
     for (tgh_problem* p : b->probs)
       if (p->has_bounds) launch_bounds_brick(p, s == 3 ? p->Bus : p->BW[(s + 1) % 2], s == 3 ? p->BW[(s + 1) % 2] : nullptr);
   }
@@ -2207,39 +2247,28 @@ int tgh_batch_create(tgh_problem* const* probs, int32_t n, tgh_batch** out) {
     return rc;
   };
   if (blocks && b->hole_kind != 2) {
-    // the blocks run as bricks where every problem allows it (as tgh_rk4's form 5)
+    // in tiles where every problem allows it (as tgh_rk4's form 5)
     bool ok = true;
-    for (tgh_problem* p : b->probs)
-      ok = ok && !p->has_bounds && p->cs.interior != INT_PASTED && !p->mat.rho && p->cs.gauge != GAUGE_SAMPLED &&
-           !p->cs.general;
+    for (tgh_problem* p : b->probs) {
+      int rc = ensure_layer_box(p);
+      if (rc) return bail(rc);
+      ok = ok && block_stage_ok(p);
+    }
     b->lds = ok;
     for (tgh_problem* p : b->probs) {
-      if (!b->lds || p->Wus) continue;
-      const size_t wbytes = sizeof(double) * (size_t)p->work_len;
-      if (hipMalloc(&p->Wus, wbytes) != hipSuccess || hipMalloc(&p->Wacc, wbytes) != hipSuccess ||
-          hipMalloc(&p->Wcoef, wbytes / 20 * CF_N) != hipSuccess ||
-          hipMemset(p->Wcoef, 0, wbytes / 20 * CF_N) != hipSuccess)
-        return bail(fail(TGH_EDEVICE, "allocating a batch's work-layout arrays"));
+      int rc = b->lds ? ensure_block_stage(p) : TGH_OK;
+      if (rc) return bail(rc);
+      rc = sync(p);
+      if (rc) return bail(rc);
     }
   }
   for (tgh_problem* p : b->probs) {
     if (blocks) continue;
     int rc = ensure_brick(p);
     if (rc) return bail(rc);
-    if (!p->Bcoef) {
-      const size_t bytes = sizeof(double) * CF_N * (size_t)p->brick.fs;
-      if (hipMalloc(&p->Bcoef, bytes) != hipSuccess) return bail(fail(TGH_EDEVICE, "allocating a batch's coefficients"));
-      if (hipMemsetAsync(p->Bcoef, 0, bytes, p->stream) != hipSuccess) return bail(fail(TGH_EDEVICE, "clearing them"));
-    }
+    if (!stage_ok(p)) return bail(fail(TGH_EDEVICE, "allocating a batch's layer boxes"));
     rc = sync(p);
     if (rc) return bail(rc);
-  }
-  // moving :damped holes with their layer boxes: the head reads the boxes, as
-  // each problem's own steps do, so that every problem computes its own bits
-  if (!blocks && b->hole) {
-    bool boxed = true;
-    for (tgh_problem* p : b->probs) boxed = boxed && p->Blayer;
-    if (boxed) b->hole = HOLE_BOXED;
   }
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
     return bail(fail(TGH_EDEVICE, "creating the batch's stream"));
@@ -2281,7 +2310,8 @@ int tgh_batch_rk4(tgh_batch* b, double* const* u, double t0, double dt, int32_t 
       if (b->lds) launch_scatter(p, u[i], p->Wus, 1);  // and the work-layout u_n
       continue;
     }
-    BrickCopyArgs ca{p->geom, p->brick, u[i], p->BW[0], p->Bus, 0};
+    double* un = brick_un(p, false);
+    BrickCopyArgs ca{p->geom, p->brick, u[i], p->BW[0], un == p->BW[0] ? nullptr : un, 0};
     hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, b->stream, ca);
   }
   const std::vector<double*> uv(u, u + n);
@@ -2336,7 +2366,7 @@ int tgh_batch_rk4(tgh_batch* b, double* const* u, double t0, double dt, int32_t 
     for (int i = 0; i < n && !b->blocks; ++i) {  // (the block layout wrote u in place)
       tgh_problem* p = b->probs[i];
       for (int pass = 0; pass < 2; ++pass) {
-        BrickCopyArgs ca{p->geom, p->brick, p->Bus, u[i], nullptr, pass};
+        BrickCopyArgs ca{p->geom, p->brick, brick_un(p, false), u[i], nullptr, pass};
         hipLaunchKernelGGL(k_brick_out, grid_points(p), dim3(256), 0, b->stream, ca);
       }
     }

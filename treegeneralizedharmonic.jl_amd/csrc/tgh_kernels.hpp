@@ -2322,38 +2322,6 @@ __device__ __forceinline__ bool tile_map(const Brick& k, int TX, int TY, int TZ,
   return true;
 }
 
-// The fused right-hand side with the RK4 epilogue on the brick layout: the
-// stage input W, its successor Wn, u_n and the accumulator all in the brick
-// layout, so one index addresses a point in every one of them.
-template <int Q, int GAUGE, int HOLE>
-__global__ __launch_bounds__(256) void k_brick_rhs(RhsArgs a, Brick k, const double* __restrict__ W,
-                                                   TGH_OUT_PARAMS) {
-  a.t = stage_time(a.t, a.clock, a.toff);
-  int x, y, z;
-  if (!brick_map(k, x, y, z)) return;
-  const long off = brick_index(k, x, y, z);
-  PointRef pr;
-  pr.w0 = W + off;
-  pr.sv = k.fs;
-  pr.s2 = (int)k.py;
-  pr.s3 = (int)k.pz;
-  pr.x[0] = k.lo[0] + (double)(x + k.gx0[0]) * k.h;
-  pr.x[1] = k.lo[1] + (double)(y + k.gx0[1]) * k.h;
-  pr.x[2] = k.lo[2] + (double)(z + k.gx0[2]) * k.h;
-  pr.si0 = off;
-  pr.ssv = k.fs;
-  pr.wi0 = off;
-  pr.Hp = a.Hsrc ? a.Hsrc + off : nullptr;
-  pr.hs = k.fs;
-  pr.m_rho = nullptr;
-  pr.m_S = nullptr;
-  pr.m_Sij = nullptr;
-  pr.ms = 0;
-  pr.lslot = a.lbox ? layer_slot((x + k.gx0[0]) << k.lsh, (y + k.gx0[1]) << k.lsh, (z + k.gx0[2]) << k.lsh, a.lB)
-                    : 0;
-  rhs_point<Q, GAUGE, HOLE, EPI_RK4>(a, pr, k.inv_h, TGH_OUT_ARGS);
-}
-
 // The split form on the brick layout, first half: the head at one point per
 // thread (brick_map's order), leaving the Pi coefficients in coef (CF_N
 // arrays of the brick's field size, indexed like the brick).
@@ -2450,15 +2418,11 @@ __device__ __forceinline__ void brick_head_at(const RhsArgs& a, const Brick& k, 
 // same arithmetic in the same order: only the staging differs, so the
 // results are the same bits.
 constexpr int PI_TILES = 6;
-// The tile of a block run as a brick (17 x 5 x 3 threads, one point each): a
-// block's 17 points along x in one row, 4 x 6 tiles a block, 80 % of the
-// threads busy, where the brick's 8 x 8 x 4 tile would keep 43 %.
-constexpr int PI_TILE_BLOCK = 6;
 template <int Q, int TC = 0> struct PiTile {
-  static constexpr int X = TC == PI_TILE_BLOCK ? 17 : TC == 0 || TC >= 4 ? TGH_PI_TILE_X : TC == 1 ? 8 : TC == 2 ? 10 : 16;
-  static constexpr int Y = TC == PI_TILE_BLOCK ? 5 : TC == 0 || TC >= 4 ? TGH_PI_TILE_Y : TC == 1 ? 12 : TC == 2 ? 10 : 8;
-  static constexpr int Z = TC == PI_TILE_BLOCK ? 3 : Q == 8 ? 2 : TC == 0 || TC >= 4 ? TGH_PI_TILE_Z : TC == 3 ? 2 : 4;
-  static constexpr int PZ = TC == PI_TILE_BLOCK || Q == 8 || !(TC == 0 || TC >= 4) ? 1 : TGH_PI_POINTS_Z;
+  static constexpr int X = TC == 0 || TC >= 4 ? TGH_PI_TILE_X : TC == 1 ? 8 : TC == 2 ? 10 : 16;
+  static constexpr int Y = TC == 0 || TC >= 4 ? TGH_PI_TILE_Y : TC == 1 ? 12 : TC == 2 ? 10 : 8;
+  static constexpr int Z = Q == 8 ? 2 : TC == 0 || TC >= 4 ? TGH_PI_TILE_Z : TC == 3 ? 2 : 4;
+  static constexpr int PZ = Q == 8 || !(TC == 0 || TC >= 4) ? 1 : TGH_PI_POINTS_Z;
   static constexpr int pitch(int bx) {
     return TC == 4 ? (bx <= 25 ? 25 : bx) : TC == 5 ? (bx <= 26 ? 26 : bx) : (bx <= 24 ? 24 : bx);
   }
@@ -2606,11 +2570,11 @@ __device__ __forceinline__ void brick_pi_tile(const RhsArgs& a, const Brick& k, 
 // ---------------------------------------------------------------------------
 // Several problems in one launch (independent holes of uneven block counts):
 // a device-side table holds each problem's stage arguments, its brick and the
-// first logical workgroup of its range in the head and the Pi launches. A
-// workgroup takes its logical index in wg_logical's XCD-contiguous order over
-// the whole launch, finds the problem whose range holds it, and runs that
-// problem's run (head) or tile (Pi) -- the same code as the one-problem
-// kernels, so a problem in a batch computes the bits it computes alone.
+// first logical workgroup of its range in the launch. A workgroup takes its
+// logical index in wg_logical's XCD-contiguous order over the whole launch,
+// finds the problem whose range holds it, and runs that problem's tile -- the
+// same code as the one-problem kernels, so a problem in a batch computes the
+// bits it computes alone.
 // The table's arrays, typed as global memory on the device: pointers loaded
 // from memory are otherwise generic, and their loads and stores flat.
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -2623,55 +2587,21 @@ struct BatchEntry {
   Brick k;
   TGH_GLOBAL const double* W;  // the stage input
   TGH_GLOBAL const double* Hsrc;
-  TGH_GLOBAL double* coef;
   TGH_GLOBAL double* us;
   TGH_GLOBAL double* acc;
+  TGH_GLOBAL double* y2;
   TGH_GLOBAL double* Wn;  // the next stage's input
-  int head0, pi0;  // first logical workgroup in the head and the Pi launch
-  int lLmax;       // the block layout run as bricks: the problem's finest level
+  int wg0;    // first logical workgroup of the launch
+  int lLmax;  // the block layout's tiles: the problem's finest level
 };
-__device__ __forceinline__ int batch_find(const BatchEntry* __restrict__ tab, int n, int L, bool pi) {
+__device__ __forceinline__ int batch_find(const BatchEntry* __restrict__ tab, int n, int L) {
   int p = 0;
-  while (p + 1 < n && L >= (pi ? tab[p + 1].pi0 : tab[p + 1].head0)) ++p;
+  while (p + 1 < n && L >= tab[p + 1].wg0) ++p;
   return p;
 }
-template <int Q, int GAUGE, int HOLE>
-__global__ __launch_bounds__(256) void k_brick_head_batch(const BatchEntry* __restrict__ tab, int n,
-                                                                        int total) {
-  const int L = wg_logical(total);
-  if (L >= total) return;
-  const BatchEntry& e = tab[batch_find(tab, n, L, false)];
-  int x, y, z;
-  if (!brick_run(e.k, L - e.head0, x, y, z)) return;
-  brick_head_at<Q, GAUGE, HOLE>(e.a, e.k, (const double*)e.W, (const double*)e.Hsrc, (double*)e.coef, nullptr,
-                                (double*)e.us, (double*)e.acc, (double*)e.Wn, x, y, z);
-}
-template <int Q>
-__global__ __launch_bounds__(PiTile<Q>::X * PiTile<Q>::Y * PiTile<Q>::Z) void k_brick_pi_batch(
-    const BatchEntry* __restrict__ tab, int n, int total) {
-  const int L = wg_logical(total);
-  if (L >= total) return;  // uniform over the workgroup
-  const BatchEntry& e = tab[batch_find(tab, n, L, true)];
-  int X0, Y0, Z0;
-  tile_at(e.k, PiTile<Q>::X, PiTile<Q>::Y, PiTile<Q>::Z * PiTile<Q>::PZ, L - e.pi0, X0, Y0, Z0);
-  brick_pi_tile<Q>(e.a, e.k, (const double*)e.W, (const double*)e.coef, nullptr, (double*)e.us, (double*)e.acc,
-                   (double*)e.Wn, X0, Y0, Z0);
-}
-
-// The block layout's split form with the brick's code: block b's work array
-// is a brick of P^3 points (strides S, S^2, S^3 per variable, G ghosts) at
-// index offset B N, run by the brick head (one point a thread) and the
-// LDS-tiled Pi kernel (PI_TILE_BLOCK tiles). During a step u_n, the
-// accumulator and the Pi coefficients sit in the work layout beside W, so
-// that one index addresses a point in all of them, as on the brick.
-struct BlockBricks {
-  const double* __restrict__ W;
-  double* __restrict__ coef;  // CF_N fields of S^3 points a block
-  double* __restrict__ us;
-  double* __restrict__ acc;
-  double* __restrict__ Wn;
-  int lLmax;  // the finest level (the layer box's grid)
-};
+// Block b's work array as a brick of P^3 points (strides S, S^2, S^3 per
+// variable, G ghosts) at index offset B N; lLmax the finest level (the layer
+// box's grid).
 __device__ __forceinline__ Brick block_brick(const Geom& g, int b, int lLmax) {
   Brick k;
   const int* B = g.bcoord + 3 * b;
@@ -2695,88 +2625,18 @@ __device__ __forceinline__ Brick block_brick(const Geom& g, int b, int lLmax) {
   k.lsh = lLmax - block_level(g, b);
   return k;
 }
-template <int Q, int GAUGE, int HOLE>
-__global__ __launch_bounds__(256) void k_block_head(RhsArgs a, BlockBricks bb) {
-  a.t = stage_time(a.t, a.clock, a.toff);
-  const Geom& g = a.g;
-  const int P = g.P, P3 = g.P * g.P * g.P;
-  int b, wx;
-  if (!wg_map((P3 + 255) / 256, g.nblocks, b, wx)) return;
-  const int p = wx * 256 + (int)threadIdx.x;
-  if (p >= P3) return;
-  const Brick k = block_brick(g, b, bb.lLmax);
-  const long wb = (long)b * 20 * k.fs;
-  brick_head_at<Q, GAUGE, HOLE>(a, k, bb.W + wb, nullptr, bb.coef + (long)b * CF_N * k.fs, nullptr, bb.us + wb,
-                                bb.acc + wb, bb.Wn + wb, p % P, (p / P) % P, p / (P * P));
-}
-template <int Q>
-__global__ __launch_bounds__((PiTile<Q, PI_TILE_BLOCK>::X * PiTile<Q, PI_TILE_BLOCK>::Y *
-                              PiTile<Q, PI_TILE_BLOCK>::Z)) void k_block_pi(RhsArgs a, BlockBricks bb) {
-  a.t = stage_time(a.t, a.clock, a.toff);
-  using T = PiTile<Q, PI_TILE_BLOCK>;
-  const Geom& g = a.g;
-  const int P = g.P;
-  const int tx = (P + T::X - 1) / T::X, ty = (P + T::Y - 1) / T::Y, tz = (P + T::Z - 1) / T::Z;
-  int b, wx;
-  if (!wg_map(tx * ty * tz, g.nblocks, b, wx)) return;  // uniform over the workgroup
-  const int X0 = (wx % tx) * T::X, Y0 = ((wx / tx) % ty) * T::Y, Z0 = (wx / (tx * ty)) * T::Z;
-  const Brick k = block_brick(g, b, bb.lLmax);
-  const long wb = (long)b * 20 * k.fs;
-  brick_pi_tile<Q, PI_TILE_BLOCK>(a, k, bb.W + wb, bb.coef + (long)b * CF_N * k.fs, nullptr, bb.us + wb,
-                                  bb.acc + wb, bb.Wn + wb, X0, Y0, Z0);
-}
-
-// A batch on the block layout with its blocks run as bricks: one head and one
-// Pi launch over every block of every problem, each entry's blocks a range of
-// logical workgroups from head0 (head) and pi0 (Pi tiles); W, Wn, us, acc and
-// coef the problem's work-layout arrays.
-template <int Q, int GAUGE, int HOLE>
-__global__ __launch_bounds__(256) void k_block_head_batch(const BatchEntry* __restrict__ tab, int n, int total) {
-  const int L = wg_logical(total);
-  if (L >= total) return;
-  const BatchEntry& e = tab[batch_find(tab, n, L, false)];
-  const Geom& g = e.a.g;
-  const int P = g.P, P3 = g.P * g.P * g.P, wgpb = (P3 + 255) / 256;
-  const int loc = L - e.head0, b = loc / wgpb;
-  const int p = (loc - b * wgpb) * 256 + (int)threadIdx.x;
-  if (p >= P3) return;
-  const Brick k = block_brick(g, b, e.lLmax);
-  const long wb = (long)b * 20 * k.fs;
-  brick_head_at<Q, GAUGE, HOLE>(e.a, k, (const double*)e.W + wb, nullptr, (double*)e.coef + (long)b * CF_N * k.fs,
-                                nullptr, (double*)e.us + wb, (double*)e.acc + wb, (double*)e.Wn + wb, p % P,
-                                (p / P) % P, p / (P * P));
-}
-template <int Q>
-__global__ __launch_bounds__((PiTile<Q, PI_TILE_BLOCK>::X * PiTile<Q, PI_TILE_BLOCK>::Y *
-                              PiTile<Q, PI_TILE_BLOCK>::Z)) void k_block_pi_batch(const BatchEntry* __restrict__ tab,
-                                                                                   int n, int total) {
-  using T = PiTile<Q, PI_TILE_BLOCK>;
-  const int L = wg_logical(total);
-  if (L >= total) return;  // uniform over the workgroup
-  const BatchEntry& e = tab[batch_find(tab, n, L, true)];
-  const Geom& g = e.a.g;
-  const int P = g.P;
-  const int tx = (P + T::X - 1) / T::X, ty = (P + T::Y - 1) / T::Y, tz = (P + T::Z - 1) / T::Z;
-  const int loc = L - e.pi0, b = loc / (tx * ty * tz), wx = loc - b * (tx * ty * tz);
-  const int X0 = (wx % tx) * T::X, Y0 = ((wx / tx) % ty) * T::Y, Z0 = (wx / (tx * ty)) * T::Z;
-  const Brick k = block_brick(g, b, e.lLmax);
-  const long wb = (long)b * 20 * k.fs;
-  brick_pi_tile<Q, PI_TILE_BLOCK>(e.a, k, (const double*)e.W + wb, (double*)e.coef + (long)b * CF_N * k.fs, nullptr,
-                                  (double*)e.us + wb, (double*)e.acc + wb, (double*)e.Wn + wb, X0, Y0, Z0);
-}
-
 // One RK4 stage of a batch on the block layout: the fused kernel over every
 // block of every problem in the table (forests of any depth and problems with
 // the general interior among them), each entry's blocks a contiguous range of
-// logical workgroups from head0.
+// logical workgroups from wg0.
 template <int Q, int GAUGE, int HOLE>
 __global__ __launch_bounds__(256) void k_rhs_batch(const BatchEntry* __restrict__ tab, int n, int total) {
   const int L = wg_logical(total);
   if (L >= total) return;
-  const BatchEntry& e = tab[batch_find(tab, n, L, false)];
+  const BatchEntry& e = tab[batch_find(tab, n, L)];
   const RhsArgs& a = e.a;
   const int wgpb = (a.g.P * a.g.P * a.g.P + 255) / 256;
-  const int loc = L - e.head0;
+  const int loc = L - e.wg0;
   const int b = loc / wgpb;
   PointRef pr;
   long pi;
@@ -2858,10 +2718,10 @@ __global__ __launch_bounds__(256) void k_brick_layer(LayerArgs a) {
   if (!core && !(r < c.r1)) return;  // the head reads core and layer points only
   double* dst = a.box + layer_slot(p[0], p[1], p[2], B);
   if constexpr (!MOVING) {
-    // a harmonic hole at rest: the layer's target, once (the core's rates are zero)
+    // a hole at rest: the layer's target, once (the core's rates are zero)
     if (core) return;
     double ue[20];
-    case_state<bg_set_for(GAUGE_NONE)>(c, a.t, x, ue);
+    case_state<BGS_STATIC>(c, a.t, x, ue);
 #pragma unroll
     for (int v = 0; v < 20; ++v) dst[v * B3] = ue[v];
     return;
@@ -3051,7 +2911,7 @@ __global__ __launch_bounds__(256) void k_brick_in(BrickCopyArgs a) {
   for (int v = 0; v < 20; ++v) {
     const double val = s[v * psz];
     a.dst0[off + v * k.fs] = val;
-    a.dst1[off + v * k.fs] = val;
+    if (a.dst1) a.dst1[off + v * k.fs] = val;
   }
 }
 __global__ __launch_bounds__(256) void k_brick_out(BrickCopyArgs a) {

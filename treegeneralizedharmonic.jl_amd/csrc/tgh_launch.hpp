@@ -6,6 +6,11 @@
 
 namespace tgh {
 
+// The split kernels read the layer box where their own evaluation of the
+// target is a dual pass (moving and harmonic holes).
+inline bool boxed_head(const tgh_problem* p, const RhsArgs& a) {
+  return a.lbox && (p->cs.gauge == GAUGE_KS_MOVING || p->cs.gauge == GAUGE_NONE_MOVING || p->cs.gauge == GAUGE_NONE);
+}
 
 // The brick Pi kernel with tile shape TC.
 template <int Q, int TC>
@@ -78,7 +83,7 @@ void launch_rhs_g(tgh_problem* p, const RhsArgs& a) {
     return;
   }
   if constexpr (EPI == EPI_RK4) {
-    if (a.lbox) {  // a moving :damped hole or a harmonic hole at rest, with its layer box
+    if (boxed_head(p, a)) {  // a moving :damped hole or a harmonic hole at rest, with its layer box
       if (p->cs.gauge == GAUGE_KS_MOVING)
         launch_rhs_q<Q, GAUGE_KS_MOVING, HOLE_BOXED, EPI>(p, a);
       else if (p->cs.gauge == GAUGE_NONE_MOVING)
@@ -121,32 +126,26 @@ template <int Q, int GAUGE, int HOLE>
 void launch_brick_rhs_q(tgh_problem* p, const RhsArgs& a) {
   const bool prof = p->profiling;
   int e0 = prof ? mark(p) : -1;
-  if (p->fused) {
-    hipLaunchKernelGGL((k_brick_rhs<Q, GAUGE, HOLE>), grid_brick(p), dim3(256), 0, p->stream, a, p->brick,
-                       a.W, a.du, a.us, a.acc, a.Wn);
-    if (prof) p->ev_rhs.push_back({e0, mark(p)});
-  } else {
-    hipLaunchKernelGGL((k_brick_head<Q, GAUGE, HOLE>), grid_brick(p), dim3(256), 0, p->stream, a, p->brick,
-                       a.W, p->Bcoef, a.du, a.us, a.acc, a.Wn);
-    int e1 = prof ? mark(p) : -1;
-    switch (p->pi_tile) {
-      case 1: launch_brick_pi<Q, 1>(p, a); break;
-      case 2: launch_brick_pi<Q, 2>(p, a); break;
-      case 3: launch_brick_pi<Q, 3>(p, a); break;
-      case 4: launch_brick_pi<Q, 4>(p, a); break;
-      case 5: launch_brick_pi<Q, 5>(p, a); break;
-      default: launch_brick_pi<Q, 0>(p, a); break;
-    }
-    if (prof) {
-      p->ev_rhs.push_back({e0, e1});
-      p->ev_pi.push_back({e1, mark(p)});
-    }
+  hipLaunchKernelGGL((k_brick_head<Q, GAUGE, HOLE>), grid_brick(p), dim3(256), 0, p->stream, a, p->brick, a.W,
+                     p->Bcoef, a.du, a.us, a.acc, a.Wn);
+  int e1 = prof ? mark(p) : -1;
+  switch (p->pi_tile) {
+    case 1: launch_brick_pi<Q, 1>(p, a); break;
+    case 2: launch_brick_pi<Q, 2>(p, a); break;
+    case 3: launch_brick_pi<Q, 3>(p, a); break;
+    case 4: launch_brick_pi<Q, 4>(p, a); break;
+    case 5: launch_brick_pi<Q, 5>(p, a); break;
+    default: launch_brick_pi<Q, 0>(p, a); break;
+  }
+  if (prof) {
+    p->ev_rhs.push_back({e0, e1});
+    p->ev_pi.push_back({e1, mark(p)});
   }
 }
 template <int Q>
 void launch_brick_rhs_g(tgh_problem* p, const RhsArgs& a) {
   const bool hole = p->cs.interior != INT_NONE;
-  if (a.lbox) {  // a moving :damped hole or a harmonic hole at rest, with its layer box
+  if (boxed_head(p, a)) {  // a moving :damped hole or a harmonic hole at rest, with its layer box
     if (p->cs.gauge == GAUGE_KS_MOVING)
       launch_brick_rhs_q<Q, GAUGE_KS_MOVING, HOLE_BOXED>(p, a);
     else if (p->cs.gauge == GAUGE_NONE_MOVING)
@@ -182,96 +181,85 @@ void launch_rhs_brick(tgh_problem* p, const RhsArgs& a) {
   launch_brick_rhs_g<Q>(p, a);
 }
 
-// The block layout's split form run with the brick's code (k_block_head, then
-// k_block_pi over every block's tiles); timed while profiling as the brick's is.
-template <int Q, int GAUGE, int HOLE>
-void launch_block_lds_q(tgh_problem* p, const RhsArgs& a, const BlockBricks& bb) {
-  using T = PiTile<Q, PI_TILE_BLOCK>;
-  const int P = a.g.P;
-  const long P3 = (long)P * P * P;
-  const long tiles = (long)((P + T::X - 1) / T::X) * ((P + T::Y - 1) / T::Y) * ((P + T::Z - 1) / T::Z);
-  const bool prof = p->profiling;
-  int e0 = prof ? mark(p) : -1;
-  hipLaunchKernelGGL((k_block_head<Q, GAUGE, HOLE>), xcd_grid((P3 + 255) / 256 * a.g.nblocks), dim3(256), 0,
-                     p->stream, a, bb);
-  int e1 = prof ? mark(p) : -1;
-  hipLaunchKernelGGL((k_block_pi<Q>), xcd_grid(tiles * a.g.nblocks), dim3(T::X * T::Y * T::Z), 0, p->stream, a,
-                     bb);
-  if (prof) {
-    p->ev_rhs.push_back({e0, e1});
-    p->ev_pi.push_back({e1, mark(p)});
-  }
-}
-template <int Q>
-void launch_rhs_blocks_lds(tgh_problem* p, const RhsArgs& a, const BlockBricks& bb) {
-  const bool hole = p->cs.interior != INT_NONE;
-  if (a.lbox) {  // a moving :damped hole or a harmonic hole at rest, with its layer box
-    if (p->cs.gauge == GAUGE_KS_MOVING)
-      launch_block_lds_q<Q, GAUGE_KS_MOVING, HOLE_BOXED>(p, a, bb);
-    else if (p->cs.gauge == GAUGE_NONE_MOVING)
-      launch_block_lds_q<Q, GAUGE_NONE_MOVING, HOLE_BOXED>(p, a, bb);
-    else
-      launch_block_lds_q<Q, GAUGE_NONE, HOLE_BOXED>(p, a, bb);
-    return;
-  }
-  switch (p->cs.gauge) {
-    case GAUGE_KS:
-      if (hole) launch_block_lds_q<Q, GAUGE_KS, true>(p, a, bb);
-      else launch_block_lds_q<Q, GAUGE_KS, false>(p, a, bb);
-      break;
-    case GAUGE_KS_MOVING:
-      launch_block_lds_q<Q, GAUGE_KS_MOVING, true>(p, a, bb);
-      break;
-    case GAUGE_NONE_MOVING:
-      launch_block_lds_q<Q, GAUGE_NONE_MOVING, true>(p, a, bb);
-      break;
-    default:  // GAUGE_NONE (the sampled source is read in the state layout: not this form)
-      if (hole) launch_block_lds_q<Q, GAUGE_NONE, true>(p, a, bb);
-      else launch_block_lds_q<Q, GAUGE_NONE, false>(p, a, bb);
-      break;
-  }
-}
-
-// One RK4 stage of a batch of problems: the head and the Pi kernel, each one
-// launch over every problem's runs or tiles (the table's ranges).
-template <int Q, int GAUGE, int HOLE>
-void launch_batch_q(hipStream_t st, const BatchEntry* tab, int n, int head_total, int pi_total) {
-  using T = PiTile<Q>;
-  hipLaunchKernelGGL((k_brick_head_batch<Q, GAUGE, HOLE>), xcd_grid(head_total), dim3(256), 0, st, tab, n,
-                     head_total);
-  hipLaunchKernelGGL((k_brick_pi_batch<Q>), xcd_grid(pi_total), dim3(T::X * T::Y * T::Z), 0, st, tab, n, pi_total);
-}
-template <int Q>
-void launch_batch(hipStream_t st, const BatchEntry* tab, int n, int head_total, int pi_total, int gauge, int hole) {
-  if (hole == HOLE_BOXED) {  // holes with their layer boxes
-    if (gauge == GAUGE_KS_MOVING)
-      launch_batch_q<Q, GAUGE_KS_MOVING, HOLE_BOXED>(st, tab, n, head_total, pi_total);
-    else if (gauge == GAUGE_NONE_MOVING)
-      launch_batch_q<Q, GAUGE_NONE_MOVING, HOLE_BOXED>(st, tab, n, head_total, pi_total);
-    else
-      launch_batch_q<Q, GAUGE_NONE, HOLE_BOXED>(st, tab, n, head_total, pi_total);
-    return;
-  }
+// A stage's launch for the case's specialisation: f.template run<GAUGE, HOLE>(),
+// an interior's targets read from the layer box.
+template <class F>
+void stage_dispatch(int gauge, bool hole, const F& f) {
   switch (gauge) {
     case GAUGE_KS:
-      if (hole) launch_batch_q<Q, GAUGE_KS, true>(st, tab, n, head_total, pi_total);
-      else launch_batch_q<Q, GAUGE_KS, false>(st, tab, n, head_total, pi_total);
+      if (hole) f.template run<GAUGE_KS, HOLE_BOXED>();
+      else f.template run<GAUGE_KS, 0>();
       break;
     case GAUGE_SAMPLED:
-      if (hole) launch_batch_q<Q, GAUGE_SAMPLED, true>(st, tab, n, head_total, pi_total);
-      else launch_batch_q<Q, GAUGE_SAMPLED, false>(st, tab, n, head_total, pi_total);
+      if (hole) f.template run<GAUGE_SAMPLED, HOLE_BOXED>();
+      else f.template run<GAUGE_SAMPLED, 0>();
       break;
-    case GAUGE_KS_MOVING:
-      launch_batch_q<Q, GAUGE_KS_MOVING, true>(st, tab, n, head_total, pi_total);
-      break;
-    case GAUGE_NONE_MOVING:
-      launch_batch_q<Q, GAUGE_NONE_MOVING, true>(st, tab, n, head_total, pi_total);
-      break;
+    case GAUGE_KS_MOVING: f.template run<GAUGE_KS_MOVING, HOLE_BOXED>(); break;  // a moving hole has an interior
+    case GAUGE_NONE_MOVING: f.template run<GAUGE_NONE_MOVING, HOLE_BOXED>(); break;
     default:
-      if (hole) launch_batch_q<Q, GAUGE_NONE, true>(st, tab, n, head_total, pi_total);
-      else launch_batch_q<Q, GAUGE_NONE, false>(st, tab, n, head_total, pi_total);
+      if (hole) f.template run<GAUGE_NONE, HOLE_BOXED>();
+      else f.template run<GAUGE_NONE, 0>();
       break;
   }
+}
+template <int Q>
+struct StageBrickLaunch {
+  tgh_problem* p;
+  const RhsArgs& a;
+  const StageIO& io;
+  template <int GAUGE, int HOLE>
+  void run() const {
+    using TT = StageTile<Q, TILE_BRICK>;
+    const Brick& k = p->brick;
+    const int total = brick_stage_tiles<Q>(k);
+    hipLaunchKernelGGL((k_brick_stage<Q, GAUGE, HOLE>), xcd_grid(total), dim3(256), 0, p->stream, a, k, a.W, a.Hsrc,
+                       io, total);
+  }
+};
+template <int Q>
+void launch_stage_brick(tgh_problem* p, const RhsArgs& a, const StageIO& io) {
+  const bool prof = p->profiling;
+  int e0 = prof ? mark(p) : -1;
+  stage_dispatch(p->cs.gauge, p->cs.interior != INT_NONE, StageBrickLaunch<Q>{p, a, io});
+  if (prof) p->ev_rhs.push_back({e0, mark(p)});
+}
+template <int Q>
+struct StageBlockLaunch {
+  tgh_problem* p;
+  const RhsArgs& a;
+  const StageIO& io;
+  template <int GAUGE, int HOLE>
+  void run() const {
+    hipLaunchKernelGGL((k_block_stage<Q, GAUGE, HOLE>), xcd_grid((long)block_tiles(a.g.P) * a.g.nblocks), dim3(256), 0,
+                       p->stream, a, a.W, a.Hsrc, io, p->layer_lmax);
+  }
+};
+template <int Q>
+void launch_stage_blocks(tgh_problem* p, const RhsArgs& a, const StageIO& io) {
+  const bool prof = p->profiling && io.stage != STAGE_STORE;
+  int e0 = prof ? mark(p) : -1;
+  stage_dispatch(p->cs.gauge, p->cs.interior != INT_NONE, StageBlockLaunch<Q>{p, a, io});
+  if (prof) p->ev_rhs.push_back({e0, mark(p)});
+}
+
+// One RK4 stage of a batch of problems: one launch over every problem's tiles.
+template <int Q>
+struct StageBatchLaunch {
+  hipStream_t st;
+  const BatchEntry* tab;
+  int n, total;
+  bool blocks;
+  template <int GAUGE, int HOLE>
+  void run() const {
+    if (blocks)
+      hipLaunchKernelGGL((k_block_stage_batch<Q, GAUGE, HOLE>), xcd_grid(total), dim3(256), 0, st, tab, n, total);
+    else
+      hipLaunchKernelGGL((k_brick_stage_batch<Q, GAUGE, HOLE>), xcd_grid(total), dim3(256), 0, st, tab, n, total);
+  }
+};
+template <int Q>
+void launch_batch(hipStream_t st, const BatchEntry* tab, int n, int total, int gauge, int hole, bool blocks) {
+  stage_dispatch(gauge, hole != 0, StageBatchLaunch<Q>{st, tab, n, total, blocks});
 }
 
 // One RK4 stage of a batch on the block layout (static gauge-source kinds;
@@ -285,25 +273,6 @@ void launch_batch_blocks_g(hipStream_t st, const BatchEntry* tab, int n, int tot
     hipLaunchKernelGGL((k_rhs_batch<Q, GAUGE, 1>), grid, dim3(256), 0, st, tab, n, total);
   else
     hipLaunchKernelGGL((k_rhs_batch<Q, GAUGE, 0>), grid, dim3(256), 0, st, tab, n, total);
-}
-// The same with the blocks run as bricks (static gauge-source kinds; hole 0 or 1).
-template <int Q, int GAUGE, int HOLE>
-void launch_batch_blocks_lds_q(hipStream_t st, const BatchEntry* tab, int n, int head_total, int pi_total) {
-  using T = PiTile<Q, PI_TILE_BLOCK>;
-  hipLaunchKernelGGL((k_block_head_batch<Q, GAUGE, HOLE>), xcd_grid(head_total), dim3(256), 0, st, tab, n,
-                     head_total);
-  hipLaunchKernelGGL((k_block_pi_batch<Q>), xcd_grid(pi_total), dim3(T::X * T::Y * T::Z), 0, st, tab, n, pi_total);
-}
-template <int Q>
-void launch_batch_blocks_lds(hipStream_t st, const BatchEntry* tab, int n, int head_total, int pi_total, int gauge,
-                             int hole) {
-  if (gauge == GAUGE_KS) {
-    if (hole) launch_batch_blocks_lds_q<Q, GAUGE_KS, 1>(st, tab, n, head_total, pi_total);
-    else launch_batch_blocks_lds_q<Q, GAUGE_KS, 0>(st, tab, n, head_total, pi_total);
-  } else {
-    if (hole) launch_batch_blocks_lds_q<Q, GAUGE_NONE, 1>(st, tab, n, head_total, pi_total);
-    else launch_batch_blocks_lds_q<Q, GAUGE_NONE, 0>(st, tab, n, head_total, pi_total);
-  }
 }
 template <int Q>
 void launch_batch_blocks(hipStream_t st, const BatchEntry* tab, int n, int total, int gauge, int hole) {
@@ -319,7 +288,7 @@ void launch_batch_blocks(hipStream_t st, const BatchEntry* tab, int n, int total
 #define TGH_INSTANTIATE_ORDER(Q)                                                            \
   template void tgh::launch_rhs_blocks<Q>(tgh_problem*, const tgh::RhsArgs&, int);          \
   template void tgh::launch_rhs_brick<Q>(tgh_problem*, const tgh::RhsArgs&);                \
-  template void tgh::launch_rhs_blocks_lds<Q>(tgh_problem*, const tgh::RhsArgs&, const tgh::BlockBricks&); \
+  template void tgh::launch_stage_brick<Q>(tgh_problem*, const tgh::RhsArgs&, const tgh::StageIO&); \
+  template void tgh::launch_stage_blocks<Q>(tgh_problem*, const tgh::RhsArgs&, const tgh::StageIO&); \
   template void tgh::launch_batch_blocks<Q>(hipStream_t, const tgh::BatchEntry*, int, int, int, int); \
-  template void tgh::launch_batch_blocks_lds<Q>(hipStream_t, const tgh::BatchEntry*, int, int, int, int, int); \
-  template void tgh::launch_batch<Q>(hipStream_t, const tgh::BatchEntry*, int, int, int, int, int);
+  template void tgh::launch_batch<Q>(hipStream_t, const tgh::BatchEntry*, int, int, int, int, bool);

@@ -11,6 +11,7 @@
 
 #include "../../include/tgh.h"
 #include "tgh_kernels.hpp"
+#include "tgh_stage.hpp"
 
 struct tgh_problem {
   tgh_desc desc;
@@ -72,11 +73,10 @@ struct tgh_problem {
   int layer_B = 0;
   int layer_lmax = 0;                 // the finest level, whose grid the box is on
   bool layer_static = false;          // filled once (a hole at rest)
-  // the block layout's LDS form: u_n, the accumulator and the Pi coefficients
-  // in the work layout during a step (allocated at its first use)
+  // the block layout's tiled form: u_n and the accumulator in the work layout
+  // during a step (allocated at its first use)
   double* Wus = nullptr;
   double* Wacc = nullptr;
-  double* Wcoef = nullptr;
   bool brick_ready = false;
   bool frame_static = false;          // the frame never changes: filled once
   hipStream_t cap_stream = nullptr;   // capture stream when the problem runs on the null stream
@@ -121,12 +121,18 @@ int mark(tgh_problem* p);  // a profiling event on the problem's stream
 // tgh_launch.hpp, instantiated in tgh_q<Q>.hip.
 template <int Q> void launch_rhs_blocks(tgh_problem* p, const RhsArgs& a, int epi);
 template <int Q> void launch_rhs_brick(tgh_problem* p, const RhsArgs& a);
-// the block layout's split form with the brick's head and LDS-tiled Pi kernel
-template <int Q> void launch_rhs_blocks_lds(tgh_problem* p, const RhsArgs& a, const BlockBricks& bb);
-extern template void launch_rhs_blocks_lds<2>(tgh_problem*, const RhsArgs&, const BlockBricks&);
-extern template void launch_rhs_blocks_lds<4>(tgh_problem*, const RhsArgs&, const BlockBricks&);
-extern template void launch_rhs_blocks_lds<6>(tgh_problem*, const RhsArgs&, const BlockBricks&);
-extern template void launch_rhs_blocks_lds<8>(tgh_problem*, const RhsArgs&, const BlockBricks&);
+// one RK4 stage on the brick layout in one kernel (k_brick_stage)
+template <int Q> void launch_stage_brick(tgh_problem* p, const RhsArgs& a, const StageIO& io);
+extern template void launch_stage_brick<2>(tgh_problem*, const RhsArgs&, const StageIO&);
+extern template void launch_stage_brick<4>(tgh_problem*, const RhsArgs&, const StageIO&);
+extern template void launch_stage_brick<6>(tgh_problem*, const RhsArgs&, const StageIO&);
+extern template void launch_stage_brick<8>(tgh_problem*, const RhsArgs&, const StageIO&);
+// the same on the block layout, each block's work array a brick
+template <int Q> void launch_stage_blocks(tgh_problem* p, const RhsArgs& a, const StageIO& io);
+extern template void launch_stage_blocks<2>(tgh_problem*, const RhsArgs&, const StageIO&);
+extern template void launch_stage_blocks<4>(tgh_problem*, const RhsArgs&, const StageIO&);
+extern template void launch_stage_blocks<6>(tgh_problem*, const RhsArgs&, const StageIO&);
+extern template void launch_stage_blocks<8>(tgh_problem*, const RhsArgs&, const StageIO&);
 extern template void launch_rhs_blocks<2>(tgh_problem*, const RhsArgs&, int);
 extern template void launch_rhs_blocks<4>(tgh_problem*, const RhsArgs&, int);
 extern template void launch_rhs_blocks<6>(tgh_problem*, const RhsArgs&, int);
@@ -135,10 +141,10 @@ extern template void launch_rhs_brick<2>(tgh_problem*, const RhsArgs&);
 extern template void launch_rhs_brick<4>(tgh_problem*, const RhsArgs&);
 extern template void launch_rhs_brick<6>(tgh_problem*, const RhsArgs&);
 extern template void launch_rhs_brick<8>(tgh_problem*, const RhsArgs&);
-// One RK4 stage of a batch of problems on the brick layout (the head and the
-// Pi launch over the table's ranges), at order Q.
+// One RK4 stage of a batch of problems in one launch over the table's tiles,
+// on the brick layout or (blocks) on the block layout, at order Q.
 template <int Q>
-void launch_batch(hipStream_t st, const BatchEntry* tab, int n, int head_total, int pi_total, int gauge, int hole);
+void launch_batch(hipStream_t st, const BatchEntry* tab, int n, int total, int gauge, int hole, bool blocks);
 // One RK4 stage of a batch on the block layout (the fused kernel over every
 // block of every problem), at order Q.
 template <int Q>
@@ -147,15 +153,8 @@ extern template void launch_batch_blocks<2>(hipStream_t, const BatchEntry*, int,
 extern template void launch_batch_blocks<4>(hipStream_t, const BatchEntry*, int, int, int, int);
 extern template void launch_batch_blocks<6>(hipStream_t, const BatchEntry*, int, int, int, int);
 extern template void launch_batch_blocks<8>(hipStream_t, const BatchEntry*, int, int, int, int);
-template <int Q>
-void launch_batch_blocks_lds(hipStream_t st, const BatchEntry* tab, int n, int head_total, int pi_total, int gauge,
-                             int hole);
-extern template void launch_batch_blocks_lds<2>(hipStream_t, const BatchEntry*, int, int, int, int, int);
-extern template void launch_batch_blocks_lds<4>(hipStream_t, const BatchEntry*, int, int, int, int, int);
-extern template void launch_batch_blocks_lds<6>(hipStream_t, const BatchEntry*, int, int, int, int, int);
-extern template void launch_batch_blocks_lds<8>(hipStream_t, const BatchEntry*, int, int, int, int, int);
-extern template void launch_batch<2>(hipStream_t, const BatchEntry*, int, int, int, int, int);
-extern template void launch_batch<4>(hipStream_t, const BatchEntry*, int, int, int, int, int);
-extern template void launch_batch<6>(hipStream_t, const BatchEntry*, int, int, int, int, int);
-extern template void launch_batch<8>(hipStream_t, const BatchEntry*, int, int, int, int, int);
+extern template void launch_batch<2>(hipStream_t, const BatchEntry*, int, int, int, int, bool);
+extern template void launch_batch<4>(hipStream_t, const BatchEntry*, int, int, int, int, bool);
+extern template void launch_batch<6>(hipStream_t, const BatchEntry*, int, int, int, int, bool);
+extern template void launch_batch<8>(hipStream_t, const BatchEntry*, int, int, int, int, bool);
 }  // namespace tgh
