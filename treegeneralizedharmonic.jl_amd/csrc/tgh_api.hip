@@ -293,6 +293,18 @@ void launch_scatter(tgh_problem* p, const double* u, double* W, int to_work) {
   hipLaunchKernelGGL(k_scatter, grid_points(p), dim3(256), 0, p->stream, a);
 }
 
+// prepare!: the work array W from the state, ghosts filled (uniform forests:
+// in one pass over W; with levels the owned points, then the plan).
+void launch_prepare(tgh_problem* p, const double* u, double* W, double t) {
+  if (p->forest) {
+    launch_scatter(p, u, W, 1);
+    launch_fill(p, W, t);
+    return;
+  }
+  FillArgs a{p->geom, p->cs, t, W, nullptr, 0.0};
+  hipLaunchKernelGGL(p->cs.moving ? k_prepare<true> : k_prepare<false>, grid_work(p), dim3(256), 0, p->stream, a, u);
+}
+
 // One right-hand side on the block layout (the fused kernel, or the head and
 // the Pi components as two launches).
 void launch_rhs(tgh_problem* p, const RhsArgs& a, int epi) {
@@ -458,12 +470,10 @@ int ensure_layer_box(tgh_problem* p) {
   hipError_t e = hipMalloc(&p->Blayer, lb);
   if (e != hipSuccess) {
     p->Blayer = nullptr;
+    (void)hipGetLastError();
     // a sourced hole at rest has its target in closed form too: without the
     // box the stepper takes the split form, whose head evaluates it
-    if (rest && p->cs.gauge != GAUGE_NONE) {
-      (void)hipGetLastError();
-      return TGH_OK;
-    }
+    if (rest && p->cs.gauge != GAUGE_NONE) return TGH_OK;
     return fail(TGH_EDEVICE, std::string("allocating the layer box: ") + hipGetErrorString(e));
   }
   p->layer_static = rest;
@@ -1173,8 +1183,7 @@ int tgh_transfer(tgh_problem* from, const double* u_from, double t, tgh_problem*
   HIP_TRY(hipMalloc(&d_ops, sizeof(int) * ops.size()));
   hipError_t e = hipMemcpy(d_ops, ops.data(), sizeof(int) * ops.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
-    launch_scatter(from, u_from, from->W[0], 1);
-    launch_fill(from, from->W[0], t);
+    launch_prepare(from, u_from, from->W[0], t);
     TransferArgs ta{from->W[0], u_to, (const PlanOp*)d_ops, (int)(ops.size() / 4), from->geom.S,
                     from->geom.P * from->geom.P * from->geom.P};
     const dim3 grid((ta.n + 255) / 256, 20);
@@ -1266,8 +1275,7 @@ int tgh_set_stream(tgh_problem* p, void* stream) {
 
 int tgh_prepare(tgh_problem* p, const double* u, double t) {
   if (!p || !u) return fail(TGH_EINVAL, "NULL argument");
-  launch_scatter(p, u, p->W[0], 1);
-  launch_fill(p, p->W[0], t);
+  launch_prepare(p, u, p->W[0], t);
   return sync(p);
 }
 
@@ -1279,14 +1287,22 @@ int tgh_rhs(tgh_problem* p, double* du, double t, const tgh_matter* matter) {
   if (matter && matter->rho && (!matter->S || !matter->Sij))
     return fail(TGH_EINVAL, "a matter adapter needs rho, S and Sij");
   RhsArgs a = rhs_args(p, p->W[0], t, matter);
-  a.du = du;
-  launch_rhs(p, a, EPI_STORE);
+  // in tiles, as a stage of the stepper, for vacuum and a hole at rest (whose
+  // layer box is filled once); the other cases, and a box that finds no
+  // memory, one point a thread
+  if (!(matter && matter->rho) && !p->cs.general && !p->cs.moving && ensure_layer_box(p) == TGH_OK && stage_ok(p)) {
+    if (p->Blayer) launch_layer_box(p, t, 0.0, a);
+    launch_stage_block(p, a, StageIO{STAGE_STORE, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr, du});
+  } else {
+    a.du = du;
+    launch_rhs(p, a, EPI_STORE);
+  }
   return sync(p);
 }
 
 int tgh_gh_rhs(tgh_problem* p, double* du, const double* u, double t, const tgh_matter* matter) {
-  int rc = tgh_prepare(p, u, t);
-  if (rc) return rc;
+  if (!p || !u) return fail(TGH_EINVAL, "NULL argument");
+  launch_prepare(p, u, p->W[0], t);
   return tgh_rhs(p, du, t, matter);
 }
 
@@ -1402,8 +1418,7 @@ int tgh_error_norms(tgh_problem* p, const double* u, double t, double* l2, doubl
 // magnitudes, [8] the weight).
 static int launch_monitor(tgh_problem* p, const double* u, double t, bool adm, double* gc) {
   const Geom& g = p->geom;
-  launch_scatter(p, u, p->W[0], 1);
-  launch_fill(p, p->W[0], t);
+  launch_prepare(p, u, p->W[0], t);
   GCArgs a{g, p->cs, t, p->W[0], p->Hsrc, gc};
   if (adm) {
     switch (p->q) {
@@ -1546,8 +1561,7 @@ static int tau_pass(tgh_problem* p, const double* u, double t, double scale, dou
   if (scale < 0.0) {
     launch_scatter(p, u, p->W[0], 1);  // owned points only: no fill needed
   } else {
-    launch_scatter(p, u, p->W[0], 1);
-    launch_fill(p, p->W[0], t);
+    launch_prepare(p, u, p->W[0], t);
   }
   TauArgs a{g, p->cs, t, scale, eps, p->W[0], p->gc};
   hipLaunchKernelGGL(k_tau, grid_points(p), dim3(256), 0, p->stream, a);

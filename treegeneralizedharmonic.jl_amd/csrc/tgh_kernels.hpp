@@ -1390,6 +1390,28 @@ struct FillArgs {
   const double* clock;  // stage_time's clock and offset
   double toff;
 };
+// A copy's twenty values: its source's (projected onto the walls of mask sw the
+// source lies on), turned tn quarter turns about z, times the parities of the
+// mirrors mm. All are read before the caller stores any: source and
+// destination are one array, and alternated they would wait on each other.
+__device__ __forceinline__ void copy_values(const double* src, long fs, int sw, int mm, int tn, double val[20]) {
+  if (tn == 0) {
+#pragma unroll
+    for (int v = 0; v < 20; ++v) val[v] = src[v * fs];
+    if (sw | mm) {
+#pragma unroll
+      for (int v = 0; v < 20; ++v) val[v] = (parity_odd_mask(v) & sw) ? 0.0 : parity_sign(v, mm) * val[v];
+    }
+    return;
+  }
+#pragma unroll
+  for (int v = 0; v < 20; ++v) {
+    int q;
+    double sg;
+    rot_power(v, tn, q, sg);
+    val[v] = (parity_odd_mask(q) & sw) ? 0.0 : parity_sign(v, mm) * sg * src[q * fs];
+  }
+}
 template <bool MOVE>
 __global__ __launch_bounds__(256) void k_fill(FillArgs a) {
   a.t = stage_time(a.t, a.clock, a.toff);
@@ -1427,20 +1449,49 @@ __global__ __launch_bounds__(256) void k_fill(FillArgs a) {
     // parities of the mirrors crossed
     const double* src = a.W + (long)owner * 20 * sv + (loc[0] + G) + (long)S * ((loc[1] + G) + (long)S * (loc[2] + G));
     const int sw = wall_mask(g, owner, loc);
-    if (tn == 0) {
+    double val[20];
+    copy_values(src, sv, sw, mm, tn, val);
 #pragma unroll
-      for (int v = 0; v < 20; ++v)
-        dst[v * sv] = (parity_odd_mask(v) & sw) ? 0.0 : parity_sign(v, mm) * src[v * sv];
-    } else {
-      // across the rotating seam: Q^tn of the (projected) source, then the mirrors
-      for (int v = 0; v < 20; ++v) {
-        int q;
-        double sg;
-        rot_power(v, tn, q, sg);
-        dst[v * sv] = (parity_odd_mask(q) & sw) ? 0.0 : parity_sign(v, mm) * sg * src[q * sv];
-      }
-    }
+    for (int v = 0; v < 20; ++v) dst[v * sv] = val[v];
   }
+}
+
+// prepare! on a uniform forest in one pass: every work point of a block from
+// the state itself -- its own point, its owner's (as k_fill maps it), or the
+// Dirichlet hook -- so that the state is read once and the work array
+// written once. Bound by memory. 512 blocks of 16^3: 1.54 ms as a scatter and
+// a fill of its copies, whose loads and stores alternated; the right-hand side
+// there 3.52 ms then, 1.51 ms with this and in tiles.
+template <bool MOVE>
+__global__ __launch_bounds__(256) void k_prepare(FillArgs a, const double* __restrict__ u) {
+  const Geom& g = a.g;
+  const int S = g.S, G = g.G, P = g.P;
+  int b, wx;
+  if (!wg_map((g.S * g.S * g.S + 255) / 256, g.nblocks, b, wx)) return;
+  const int p = wx * blockDim.x + threadIdx.x;
+  if (p >= S * S * S) return;
+  const int l[3] = {p % S - G, (p / S) % S - G, p / (S * S) - G};
+  int owner, loc[3], mm = 0, tn = 0;
+  const int cl = classify(g, b, l, owner, loc, &mm, &tn);
+  const long sv = (long)S * S * S, psz = (long)P * P * P;
+  double val[20];
+  if (cl == -2) {
+    double x[3];
+    position(g, b, l[0], l[1], l[2], x);
+    case_state_any<MOVE ? BGS_ALL : BGS_STATIC>(a.c, a.t, x, val);
+  } else {
+    if (cl == -1) {
+      owner = b;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) loc[d] = l[d];
+      mm = tn = 0;
+    }
+    copy_values(u + (long)owner * 20 * psz + loc[0] + (long)P * (loc[1] + (long)P * loc[2]), psz,
+                wall_mask(g, owner, loc), mm, tn, val);
+  }
+  double* __restrict__ dst = a.W + (long)b * 20 * sv + p;
+#pragma unroll
+  for (int v = 0; v < 20; ++v) dst[v * sv] = val[v];
 }
 
 // The ghost fill of a forest with levels, from a plan the host builds once
@@ -1633,13 +1684,14 @@ __global__ __launch_bounds__(256) void k_scatter(CopyArgs a) {
   const long sv = (long)S * S * S, psz = (long)P * P * P;
   const long wi = (long)b * 20 * sv + (i + G) + (long)S * ((j + G) + (long)S * (k + G));
   const long si = (long)b * 20 * psz + p;
-#pragma unroll 4
-  for (int v = 0; v < 20; ++v) {
-    if (a.to_work)
-      a.dst[wi + v * sv] = a.src[si + v * psz];
-    else
-      a.dst[si + v * psz] = a.src[wi + v * sv];
-  }
+  const double* __restrict__ src = a.src + (a.to_work ? si : wi);
+  double* __restrict__ dst = a.dst + (a.to_work ? wi : si);
+  const long ss = a.to_work ? psz : sv, ds = a.to_work ? sv : psz;
+  double val[20];
+#pragma unroll
+  for (int v = 0; v < 20; ++v) val[v] = src[v * ss];
+#pragma unroll
+  for (int v = 0; v < 20; ++v) dst[v * ds] = val[v];
 }
 
 // sample_gauge_source! (src/gauge.jl:156-184): H_b and d_a H_b of the
@@ -2863,19 +2915,10 @@ __global__ __launch_bounds__(256) void k_brick_frame(FrameArgs a) {
 #pragma unroll
     for (int d = 0; d < 3; ++d)
       if (!k.periodic[d] && ((k.refl[d][0] && w[d] == 0) || (k.refl[d][1] && w[d] == k.n[d] - 1))) sw |= 1 << d;
-    const double* src = a.W + brick_index(k, w[0], w[1], w[2]);
-    if (tn == 0) {
+    double val[20];
+    copy_values(a.W + brick_index(k, w[0], w[1], w[2]), k.fs, sw, mm, tn, val);
 #pragma unroll
-      for (int v = 0; v < 20; ++v)
-        dst[v * k.fs] = (parity_odd_mask(v) & sw) ? 0.0 : parity_sign(v, mm) * src[v * k.fs];
-    } else {
-      for (int v = 0; v < 20; ++v) {
-        int q;
-        double sg;
-        rot_power(v, tn, q, sg);
-        dst[v * k.fs] = (parity_odd_mask(q) & sw) ? 0.0 : parity_sign(v, mm) * sg * src[q * k.fs];
-      }
-    }
+    for (int v = 0; v < 20; ++v) dst[v * k.fs] = val[v];
   }
 }
 
@@ -2907,11 +2950,14 @@ __global__ __launch_bounds__(256) void k_brick_in(BrickCopyArgs a) {
   const long psz = (long)g.P * g.P * g.P;
   const double* s = a.src + (long)b * 20 * psz + loc[0] + (long)g.P * (loc[1] + (long)g.P * loc[2]);
   const long off = brick_index(k, x, y, z);
-#pragma unroll 4
-  for (int v = 0; v < 20; ++v) {
-    const double val = s[v * psz];
-    a.dst0[off + v * k.fs] = val;
-    if (a.dst1) a.dst1[off + v * k.fs] = val;
+  double val[20];
+#pragma unroll
+  for (int v = 0; v < 20; ++v) val[v] = s[v * psz];
+#pragma unroll
+  for (int v = 0; v < 20; ++v) a.dst0[off + v * k.fs] = val[v];
+  if (a.dst1) {
+#pragma unroll
+    for (int v = 0; v < 20; ++v) a.dst1[off + v * k.fs] = val[v];
   }
 }
 __global__ __launch_bounds__(256) void k_brick_out(BrickCopyArgs a) {
@@ -2937,14 +2983,22 @@ __global__ __launch_bounds__(256) void k_brick_out(BrickCopyArgs a) {
   const long off = brick_index(k, gp[0], gp[1], gp[2]);
   const long psz = (long)P * P * P;
   double* d0 = a.dst0 + (long)b * 20 * psz + p;
-  if (primary) {
-#pragma unroll 4
-    for (int v = 0; v < 20; ++v) d0[v * psz] = a.src[off + v * k.fs];
-  } else {
+  double val[20];
+#pragma unroll
+  for (int v = 0; v < 20; ++v) val[v] = a.src[off + v * k.fs];
+  if (!primary) {
     const double* up = a.dst0 + (long)ob * 20 * psz + loc[0] + (long)P * (loc[1] + (long)P * loc[2]);
-#pragma unroll 4
-    for (int v = 0; v < 20; ++v) d0[v * psz] = d0[v * psz] + (a.src[off + v * k.fs] - up[v * psz]);
+    double old[20], own[20];
+#pragma unroll
+    for (int v = 0; v < 20; ++v) {
+      old[v] = up[v * psz];
+      own[v] = d0[v * psz];
+    }
+#pragma unroll
+    for (int v = 0; v < 20; ++v) val[v] = own[v] + (val[v] - old[v]);
   }
+#pragma unroll
+  for (int v = 0; v < 20; ++v) d0[v * psz] = val[v];
 }
 
 // The sampled gauge source on the brick layout (as k_sample_gauge).
