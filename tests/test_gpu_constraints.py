@@ -104,6 +104,19 @@ def test_adm_constraints_match_oracle_on_a_uniform_hole(tgh, gauge_source):
     _compare_adm(tgh, dev, orc, u, 0.0)
 
 
+# the smallest block of each order, and point counts that a workgroup of 256
+# does not divide; the norms are sums of like rounding errors, whence the
+# helper's relative bound
+@pytest.mark.parametrize("q,N,roots", [(2, 4, 2), (2, 9, 3), (4, 6, 3), (4, 11, 2), (6, 8, 2), (8, 10, 2), (8, 13, 1)])
+def test_adm_constraints_match_oracle_on_odd_blocks(tgh, q, N, roots):
+    case = tgh.gauge_wave_case(eps_ko=0.5, gamma0=1.0, gamma2=-0.5)
+    dev = tgh.GHProblem(tgh.gh_forest(None, case, N=N, roots=roots), case, q=q)
+    orc = oracle_lib.OracleProblem(TD.gauge_wave_case(N=N, roots=roots, q=q, eps_ko=0.5, gamma0=1.0, gamma2=-0.5))
+    u = orc.fill_exact(0.1)
+    orc.add_noise(u, 0xADA3, 1e-6)
+    _compare_adm(tgh, dev, orc, u, 0.1)
+
+
 def test_adm_constraints_match_oracle_on_a_forest(tgh):
     case = tgh.kerr_schild_case(M=1.0, a=0.5, halfwidth=4.0, r_0=0.7, r_1=1.7, gauge_source="algebraic")
     f = tgh.hole_forest(None, case, N=8, roots=4, radii=(2.5, 1.0))

@@ -2028,36 +2028,23 @@ __global__ __launch_bounds__(256) void k_gauge_constraint(GCArgs a) {
 }
 
 // The ADM monitor (adm_constraint_kernel!, src/constraints.jl:432-534, and
-// adm_constraints_at_node, :100-210) at every owned point: d_t g and d_t Pi
-// from the evolution equations without dissipation, d_i d_t g and d_t d_t g
-// by differentiating the first one (metric_derivatives_along,
-// src/pointwise.jl:530-545), the textbook Ricci tensor of the 4-metric, and
-// H = 2 R_nn + R, M_i = -n^a (R_ai - g_ai R / 2). Partials as the gauge
-// monitor's, 9 per workgroup: sums of w H^2 and w M_i^2, maxima of |H| and
-// |M_i|, the weights.
-__device__ __forceinline__ double g4_at(const double h[NC], int a, int b) {
-  return (a == b ? (a == 0 ? -1.0 : 1.0) : 0.0) + h[pidx(a, b)];
-}
-// d alpha, d beta^j, d sqrt(gamma) along a derivative dg of g (packed).
-__device__ __forceinline__ void adm_along(const Coef& cf, const double dg[NC], double& da, double db[3],
-                                          double& dsq) {
-  double t00 = 0.0, t0[3] = {0.0, 0.0, 0.0};
-  for (int c = 0; c < 4; ++c)
-    for (int d = 0; d < 4; ++d) {
-      const double x = cf.gu[pidx(0, c)] * dg[pidx(c, d)];
-      t00 += x * cf.gu[pidx(d, 0)];
-      for (int j = 0; j < 3; ++j) t0[j] += x * cf.gu[pidx(d, j + 1)];
-    }
-  const double dgu00 = -t00;
-  da = cf.alpha * cf.alpha * cf.alpha * dgu00 / 2.0;
-  for (int j = 0; j < 3; ++j) db[j] = -(-t0[j] + cf.beta[j] * dgu00) / cf.gu[0];
-  double sq = 0.0;
-  for (int j = 0; j < 3; ++j)
-    for (int k = 0; k < 3; ++k) sq += cf.gamu[pidx(j + 1, k + 1) - 4] * dg[pidx(j + 1, k + 1)];
-  dsq = cf.sqrtg * sq / 2.0;
-}
+// adm_constraints_at_node, :100-210) at every owned point: H = 2 G_nn and
+// M_i = -G_ni of the metric whose time derivative the evolution equations
+// give (no dissipation). The reference forms the 4-metric's Ricci tensor from
+// all its second derivatives; G_nn and G_ni hold none of them twice in time
+// (Gauss and Codazzi), so d_t d_t g, and with it the gauge source and the
+// damping, never enter:
+//   H = R + K^2 - K_ij K^ij,   M_i = D^j K_ji - D_i K,
+//   K_jk = -(phi Pi_jk - B_jk - B_kj) / (2 alpha),  B_jk = d_j beta_k - beta^l d_j gamma_kl,
+// phi = alpha / sqrt(gamma), R the scalar curvature of gamma. The second
+// derivatives enter linearly and are contracted as each is formed. Partials
+// as the gauge monitor's, 9 per workgroup: sums of w H^2 and w M_i^2, maxima
+// of |H| and |M_i|, the weights.
+// Bound by FP64 arithmetic and the latency of its loads: a record (this, the
+// gauge monitor and the error norms) of 512 blocks of 16^3 takes 3.49 ms, 9.72
+// with the 4-metric's Ricci tensor, whose jets did not fit the registers.
 template <int Q>
-__global__ __launch_bounds__(256) void k_adm_constraint(GCArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_adm_constraint(GCArgs a) {
   const Geom& g = a.g;
   const int P = g.P, S = g.S, G = g.G;
   int b, wx;
@@ -2065,142 +2052,205 @@ __global__ __launch_bounds__(256) void k_adm_constraint(GCArgs a) {
   const int p = wx * blockDim.x + threadIdx.x;
   const long psz = (long)P * P * P, sv = (long)S * S * S;
   double r[9];
+#pragma unroll
   for (int n = 0; n < 9; ++n) r[n] = 0.0;
   if (p < P * P * P) {
     const int i = p % P, j = (p / P) % P, k = p / (P * P);
     double x[3];
     position(g, b, i, j, k, x);
-    const CaseP& c = a.c;
-    if (is_evolved(c, a.t, x)) {
+    if (is_evolved(a.c, a.t, x)) {
       int l[3] = {i, j, k}, owner, loc[3];
       const bool prim = g.prim ? g.prim[(long)b * psz + p] != 0 : classify(g, b, l, owner, loc) == -1;
       if (!(g.prim && !prim)) {
-        const double* w0 = a.W + (long)b * 20 * sv + (i + G) + (long)S * ((j + G) + (long)S * (k + G));
+        const double* __restrict__ w0 =
+            a.W + (long)b * 20 * sv + (i + G) + (long)S * ((j + G) + (long)S * (k + G));
         const double ih = block_inv_h(g, b), ih2 = ih * ih;
         const int st[3] = {1, S, S * S};
-        double hv[NC], Pv[NC], D[4][NC], dP[3][NC], dd[10][NC];  // dd: tt, tx, ty, tz, xx, xy, xz, yy, yz, zz
-        for (int v = 0; v < NC; ++v) {
-          const double* wh = w0 + v * sv;
-          const double* wp = w0 + (NC + v) * sv;
-          hv[v] = wh[0];
-          Pv[v] = wp[0];
-          for (int d = 0; d < 3; ++d) {
-            D[1 + d][v] = ih * st_d1<Q>(wh, st[d]);
-            dP[d][v] = ih * st_d1<Q>(wp, st[d]);
-          }
-          for (int d1 = 0; d1 < 3; ++d1)
-            for (int d2 = d1; d2 < 3; ++d2)
-              dd[pidx(d1 + 1, d2 + 1)][v] =
-                  ih2 * (d1 == d2 ? st_d2<Q>(wh, st[d1]) : st_mixed<Q>(wh, st[d1], st[d2]));
-        }
+        double hv[NC];
+#pragma unroll
+        for (int v = 0; v < NC; ++v) hv[v] = w0[v * sv];
         Coef cf;
         metric_quantities(hv, cf);
-        const double phi = cf.alpha / cf.sqrtg;
-        for (int v = 0; v < NC; ++v)
-          D[0][v] = cf.beta[0] * D[1][v] + cf.beta[1] * D[2][v] + cf.beta[2] * D[3][v] + phi * Pv[v];
-        double Hl[4] = {0.0, 0.0, 0.0, 0.0}, dH[4][4];
-        for (int q = 0; q < 16; ++q) dH[q % 4][q / 4] = 0.0;
-        if (c.gauge == GAUGE_SAMPLED) {
-          const double* Hp = a.Hsrc + (long)b * 20 * psz + p;
-          for (int q = 0; q < 4; ++q) Hl[q] = Hp[q * psz];
-          for (int n = 0; n < 16; ++n) dH[n % 4][n / 4] = Hp[(4 + n) * psz];
-        } else if (c.gauge == GAUGE_KS) {
-          ks_source(c.bg.M, c.bg.a, hv, D, Hl, dH);
-        } else if (c.gauge == GAUGE_KS_MOVING) {
-          ks_source_moving(c.bg.M, c.ks_S, c.ks_u, hv, D, Hl, dH);
-        }
-        double msrc[NC];
-        gh_source<true>(cf, hv, D, Hl, dH, damping_rate(c, a.t, x), c.g2, msrc);
-        PiCoef pc;
-        head_geometry(cf, D, pc);
-        double dtP[NC];
-        for (int v = 0; v < NC; ++v)
-          dtP[v] = pc.b[0] * dP[0][v] + pc.b[1] * dP[1][v] + pc.b[2] * dP[2][v] + pc.divb * Pv[v] +
-                   pc.divA[0] * D[1][v] + pc.divA[1] * D[2][v] + pc.divA[2] * D[3][v] + pc.A[0] * dd[4][v] +
-                   pc.A[3] * dd[7][v] + pc.A[5] * dd[9][v] +
-                   2.0 * (pc.A[1] * dd[5][v] + pc.A[2] * dd[6][v] + pc.A[4] * dd[8][v]) + msrc[v];
-        // d_i d_t g, then d_t d_t g
-        for (int ii = 0; ii < 3; ++ii) {
-          double da, db[3], dsq;
-          adm_along(cf, D[1 + ii], da, db, dsq);
-          const double dphi = (da - phi * dsq) / cf.sqrtg;
-          for (int v = 0; v < NC; ++v)
-            dd[1 + ii][v] = (dphi * Pv[v] + phi * dP[ii][v]) +
-                            (db[0] * D[1][v] + db[1] * D[2][v] + db[2] * D[3][v]) +
-                            (cf.beta[0] * dd[pidx(ii + 1, 1)][v] + cf.beta[1] * dd[pidx(ii + 1, 2)][v] +
-                             cf.beta[2] * dd[pidx(ii + 1, 3)][v]);
-        }
-        {
-          double da, db[3], dsq;
-          adm_along(cf, D[0], da, db, dsq);
-          const double dphi = (da - phi * dsq) / cf.sqrtg;
-          for (int v = 0; v < NC; ++v)
-            dd[0][v] = dphi * Pv[v] + phi * dtP[v] + (db[0] * D[1][v] + db[1] * D[2][v] + db[2] * D[3][v]) +
-                       (cf.beta[0] * dd[1][v] + cf.beta[1] * dd[2][v] + cf.beta[2] * dd[3][v]);
-        }
-        // dgu[e] = -g^-1 (d_e g) g^-1, Gamma_{a,bc}, Gamma^a_bc, Gamma^c_cd
-        double dgu[4][NC], Gl[4][NC], G4[4][NC], Gtr[4];
-        for (int e = 0; e < 4; ++e)
-          for (int a2 = 0; a2 < 4; ++a2)
-            for (int b2 = a2; b2 < 4; ++b2) {
-              double s2 = 0.0;
-              for (int cc = 0; cc < 4; ++cc)
-                for (int d = 0; d < 4; ++d) s2 += cf.gu[pidx(a2, cc)] * D[e][pidx(cc, d)] * cf.gu[pidx(d, b2)];
-              dgu[e][pidx(a2, b2)] = -s2;
+        const double* be = cf.beta;
+        auto gu = [&](int q, int s) { return cf.gamu[sidx3(q, s)]; };
+        // first derivatives of h_tt, beta_k and gamma_kl; the second ones of
+        // beta_k and gamma_kl contracted: Lm (into M_i), R2 (into R)
+        double d0[3], db[3][3], dg[3][6], Lm[3] = {0.0, 0.0, 0.0}, R2 = 0.0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) d0[d] = ih * st_d1<Q>(w0, st[d]);
+#pragma unroll
+        for (int v = 1; v < NC; ++v) {
+          const double* __restrict__ wh = w0 + v * sv;
+          double dd[6];
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            const double e = ih * st_d1<Q>(wh, st[d]);
+            if (v < 4) db[d][v - 1] = e;
+            else dg[d][v - 4] = e;
+#pragma unroll
+            for (int e2 = d; e2 < 3; ++e2)
+              dd[sidx3(d, e2)] = ih2 * (e2 == d ? st_d2<Q>(wh, st[d]) : st_mixed<Q>(wh, st[d], st[e2]));
+          }
+          double box = 0.0;  // gamma^jk d_j d_k
+#pragma unroll
+          for (int s = 0; s < 6; ++s) box += ((s == 0 || s == 3 || s == 5) ? 1.0 : 2.0) * cf.gamu[s] * dd[s];
+          if (v < 4) {
+            // gamma^jk (d_j d_k beta_i - d_i d_j beta_k)
+            const int kk = v - 1;
+            Lm[kk] += box;
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+              Lm[q] -= gu(0, kk) * dd[sidx3(q, 0)] + gu(1, kk) * dd[sidx3(q, 1)] + gu(2, kk) * dd[sidx3(q, 2)];
+          } else {
+            // beta^l gamma^jk (-d_j d_k gamma_il + d_i d_j gamma_kl), and
+            // gamma^ij gamma^kl (d_k d_j gamma_il - d_k d_l gamma_ij)
+            const int A = prow(v) - 1, B = pcol(v) - 1;
+            Lm[A] -= be[B] * box;
+            if (A != B) Lm[B] -= be[A] * box;
+            double tA[3], tB[3], rr = 0.0;  // gamma^Aj d_i d_j, gamma^Bj d_i d_j
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+              tA[q] = gu(A, 0) * dd[sidx3(q, 0)] + gu(A, 1) * dd[sidx3(q, 1)] + gu(A, 2) * dd[sidx3(q, 2)];
+              tB[q] = gu(B, 0) * dd[sidx3(q, 0)] + gu(B, 1) * dd[sidx3(q, 1)] + gu(B, 2) * dd[sidx3(q, 2)];
+              Lm[q] += be[B] * tA[q];
+              if (A != B) Lm[q] += be[A] * tB[q];
+              rr += gu(B, q) * tA[q];
             }
-        for (int a2 = 0; a2 < 4; ++a2)
-          for (int b2 = 0; b2 < 4; ++b2)
-            for (int c2 = b2; c2 < 4; ++c2)
-              Gl[a2][pidx(b2, c2)] = (D[b2][pidx(a2, c2)] + D[c2][pidx(a2, b2)] - D[a2][pidx(b2, c2)]) / 2;
-        for (int a2 = 0; a2 < 4; ++a2)
-          for (int n = 0; n < NC; ++n) {
-            double s2 = 0.0;
-            for (int xx = 0; xx < 4; ++xx) s2 += cf.gu[pidx(a2, xx)] * Gl[xx][n];
-            G4[a2][n] = s2;
+            R2 += (A == B ? 1.0 : 2.0) * (rr - gu(A, B) * box);
           }
-        for (int d = 0; d < 4; ++d) {
-          double s2 = 0.0;
-          for (int cc = 0; cc < 4; ++cc) s2 += G4[cc][pidx(cc, d)];
-          Gtr[d] = s2;
+          // this component's sums are formed before the next one's sixty loads:
+          // all nine components' at once would spill 3.5 KB a lane
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            asm volatile("" : "+v"(Lm[d]));
+            if (v < 4) asm volatile("" : "+v"(db[d][v - 1]));
+            else asm volatile("" : "+v"(dg[d][v - 4]));
+          }
+          asm volatile("" : "+v"(R2));
+          __builtin_amdgcn_sched_barrier(0);
         }
-        // d_m d_n g_ab
-        auto DD = [&](int m, int n, int a2, int b2) { return dd[pidx(m, n)][pidx(a2, b2)]; };
-        // R_ab is symmetric: its ten components a <= b, mirrored
-        double R[4][4];
-        for (int a2 = 0; a2 < 4; ++a2)
-          for (int b2 = a2; b2 < 4; ++b2) {
-            double A = 0.0, B = 0.0, Cc = 0.0, Dd = 0.0;
+        // B_jk, K_jk, and their traces
+        const double phi = cf.alpha / cf.sqrtg, ia = 1.0 / cf.alpha;
+        auto dgm = [&](int q, int m, int n) { return dg[q][sidx3(m, n)]; };
+        double Bm[3][3], Kl[6], dal[3], dlp[3];
 #pragma unroll
-            for (int cc = 0; cc < 4; ++cc)
+        for (int q = 0; q < 3; ++q)
 #pragma unroll
-              for (int d = 0; d < 4; ++d) {
-                const double gcd = cf.gu[pidx(cc, d)];
-                A += dgu[cc][pidx(cc, d)] * Gl[d][pidx(a2, b2)] +
-                     gcd * (DD(cc, a2, d, b2) + DD(cc, b2, d, a2) - DD(cc, d, a2, b2)) / 2;
-                B += dgu[b2][pidx(cc, d)] * Gl[d][pidx(cc, a2)] +
-                     gcd * (DD(b2, cc, d, a2) + DD(b2, a2, d, cc) - DD(b2, d, cc, a2)) / 2;
-                Dd += G4[cc][pidx(b2, d)] * G4[d][pidx(cc, a2)];
-              }
+          for (int s = 0; s < 3; ++s)
+            Bm[q][s] = db[q][s] - (be[0] * dgm(q, 0, s) + be[1] * dgm(q, 1, s) + be[2] * dgm(q, 2, s));
 #pragma unroll
-            for (int d = 0; d < 4; ++d) Cc += Gtr[d] * G4[d][pidx(a2, b2)];
-            R[a2][b2] = A - B + Cc - Dd;
-            R[b2][a2] = R[a2][b2];
-          }
-        double Rs = 0.0;
-        for (int a2 = 0; a2 < 4; ++a2)
-          for (int b2 = 0; b2 < 4; ++b2) Rs += cf.gu[pidx(a2, b2)] * R[a2][b2];
-        const double nv[4] = {1.0 / cf.alpha, -cf.beta[0] / cf.alpha, -cf.beta[1] / cf.alpha, -cf.beta[2] / cf.alpha};
-        double Rnn = 0.0;
-        for (int a2 = 0; a2 < 4; ++a2)
-          for (int b2 = 0; b2 < 4; ++b2) Rnn += R[a2][b2] * nv[a2] * nv[b2];
-        double vals[4];
-        vals[0] = 2 * Rnn + Rs;
         for (int q = 0; q < 3; ++q) {
-          double s2 = 0.0;
-          for (int a2 = 0; a2 < 4; ++a2) s2 += nv[a2] * (R[a2][q + 1] - g4_at(hv, a2, q + 1) * Rs / 2);
-          vals[1 + q] = -s2;
+          // alpha^2 = 1 - h_tt + beta^i beta_i; d ln phi = d ln alpha - gamma^kl d gamma_kl / 2
+          const double bdb = be[0] * (db[q][0] + Bm[q][0]) + be[1] * (db[q][1] + Bm[q][1]) + be[2] * (db[q][2] + Bm[q][2]);
+          dal[q] = 0.5 * ia * (bdb - d0[q]);
+          double tr = 0.0;
+#pragma unroll
+          for (int s = 0; s < 6; ++s) tr += ((s == 0 || s == 3 || s == 5) ? 1.0 : 2.0) * cf.gamu[s] * dg[q][s];
+          dlp[q] = ia * dal[q] - 0.5 * tr;
+        }
+        double Pv[6];
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+          Pv[s] = w0[(NC + 4 + s) * sv];
+          const int q = prow(4 + s) - 1, m = pcol(4 + s) - 1;
+          Kl[s] = -0.5 * ia * (phi * Pv[s] - (Bm[q][m] + Bm[m][q]));
+        }
+        // d_i beta^l = gamma^lm B_im
+        double dbu[3][3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+          for (int s = 0; s < 3; ++s) dbu[q][s] = gu(s, 0) * Bm[q][0] + gu(s, 1) * Bm[q][1] + gu(s, 2) * Bm[q][2];
+        // gamma^jk (d_j N_ki - d_i N_jk), N = phi Pi - B - B^T: the derivative of
+        // phi Pi, then of B (its second derivatives are in Lm)
+        double Mi[3];
+        {
+          double dN[3][6];
+#pragma unroll
+          for (int s = 0; s < 6; ++s) {
+            const double* __restrict__ wp = w0 + (NC + 4 + s) * sv;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) dN[q][s] = phi * (dlp[q] * Pv[s] + ih * st_d1<Q>(wp, st[q]));
+          }
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            double m = 0.0;
+#pragma unroll
+            for (int jj = 0; jj < 3; ++jj)
+#pragma unroll
+              for (int kk = 0; kk < 3; ++kk) {
+                double e = dN[jj][sidx3(kk, q)] - dN[q][sidx3(jj, kk)];
+                // -(C_jki + C_jik - 2 C_ijk) less the second derivatives, C_ijk =
+                // d_i B_jk: its products d_i beta^l d_j gamma_kl
+#pragma unroll
+                for (int ll = 0; ll < 3; ++ll)
+                  e += dbu[jj][ll] * (dgm(kk, q, ll) + dgm(q, kk, ll)) - 2.0 * dbu[q][ll] * dgm(jj, kk, ll);
+                m += gu(jj, kk) * e;
+              }
+            Mi[q] = m - Lm[q];
+          }
+        }
+        // K^j_i, K, K^ij; V_l = gamma^jk Gamma_l,jk
+        double Ku[3][3], Kuu[6], tr = 0.0, KK = 0.0, V[3], Vu[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+          for (int s = 0; s < 3; ++s)
+            Ku[q][s] = gu(q, 0) * Kl[sidx3(0, s)] + gu(q, 1) * Kl[sidx3(1, s)] + gu(q, 2) * Kl[sidx3(2, s)];
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+          const int q = prow(4 + s) - 1, m = pcol(4 + s) - 1;
+          Kuu[s] = Ku[q][0] * gu(0, m) + Ku[q][1] * gu(1, m) + Ku[q][2] * gu(2, m);
+          KK += (q == m ? 1.0 : 2.0) * Kuu[s] * Kl[s];
+        }
+        tr = Ku[0][0] + Ku[1][1] + Ku[2][2];
+        double Gn = 0.0;  // Gamma_l,jk Gamma^l,jk
+        double Gl[3][6];
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+          for (int s = 0; s < 6; ++s) {
+            const int m = prow(4 + s) - 1, n = pcol(4 + s) - 1;
+            Gl[q][s] = 0.5 * (dgm(m, q, n) + dgm(n, q, m) - dg[q][s]);
+          }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          double v = 0.0;
+#pragma unroll
+          for (int s = 0; s < 6; ++s) v += ((s == 0 || s == 3 || s == 5) ? 1.0 : 2.0) * cf.gamu[s] * Gl[q][s];
+          V[q] = v;
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          Vu[q] = gu(q, 0) * V[0] + gu(q, 1) * V[1] + gu(q, 2) * V[2];
+          double U[6], T[3][3];
+#pragma unroll
+          for (int s = 0; s < 6; ++s) U[s] = gu(q, 0) * Gl[0][s] + gu(q, 1) * Gl[1][s] + gu(q, 2) * Gl[2][s];
+#pragma unroll
+          for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int n = 0; n < 3; ++n)
+              T[m][n] = gu(m, 0) * U[sidx3(0, n)] + gu(m, 1) * U[sidx3(1, n)] + gu(m, 2) * U[sidx3(2, n)];
+#pragma unroll
+          for (int s = 0; s < 6; ++s) {
+            const int m = prow(4 + s) - 1, n = pcol(4 + s) - 1;
+            Gn += (m == n ? 1.0 : 2.0) * Gl[q][s] * (T[m][0] * gu(0, n) + T[m][1] * gu(1, n) + T[m][2] * gu(2, n));
+          }
+        }
+        double vals[4];
+        vals[0] = R2 + Gn - (V[0] * Vu[0] + V[1] * Vu[1] + V[2] * Vu[2]) + tr * tr - KK;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          // d_i K_jk = -(d_i N_jk + 2 K_jk d_i alpha) / (2 alpha)
+          const double kda = (Ku[0][q] * dal[0] + Ku[1][q] * dal[1] + Ku[2][q] * dal[2]) - tr * dal[q];
+          double kg = 0.0;
+#pragma unroll
+          for (int s = 0; s < 6; ++s) kg += ((s == 0 || s == 3 || s == 5) ? 1.0 : 2.0) * Kuu[s] * dg[q][s];
+          vals[1 + q] = -0.5 * ia * (Mi[q] + 2.0 * kda) -
+                        (Vu[0] * Kl[sidx3(0, q)] + Vu[1] * Kl[sidx3(1, q)] + Vu[2] * Kl[sidx3(2, q)]) + 0.5 * kg;
         }
         const double wgt = g.blevel ? ldexp(1.0, -3 * block_level(g, b)) : 1.0;
+#pragma unroll
         for (int q = 0; q < 4; ++q) {
           r[4 + q] = fabs(vals[q]);
           if (prim) r[q] = vals[q] * vals[q] * wgt;
@@ -2211,10 +2261,12 @@ __global__ __launch_bounds__(256) void k_adm_constraint(GCArgs a) {
   }
   __shared__ double sh[9][256];
   const int tid = threadIdx.x;
+#pragma unroll
   for (int n = 0; n < 9; ++n) sh[n][tid] = r[n];
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
     if (tid < w) {
+#pragma unroll
       for (int n = 0; n < 9; ++n)
         sh[n][tid] = (n >= 4 && n < 8) ? fmax(sh[n][tid], sh[n][tid + w]) : sh[n][tid] + sh[n][tid + w];
     }
