@@ -74,3 +74,37 @@ def test_stage_matches_the_oracle_at_the_edges_of_its_tiles(tgh, make, q, N, roo
         err = float(np.max(np.abs(v.cpu().numpy() - ref)))
         print(f"flags {flags}: {err:.2e} (bound {2 * step_tol:.2e})")
         assert err <= 2 * step_tol
+
+
+# (chart, axis, q, N, roots): frames and layer boxes that quads of lanes do not
+# fill, at a velocity along each axis
+MOVES = [("kerr_schild", 1, 2, 13, 4), ("kerr_schild", 3, 4, 11, 5), ("harmonic", 2, 4, 13, 4), ("harmonic", 1, 2, 9, 6)]
+
+
+@pytest.mark.parametrize("chart,axis,q,N,roots", MOVES)
+def test_a_moving_holes_frame_and_layer_match_the_oracle(tgh, chart, axis, q, N, roots):
+    torch = torch_cuda()
+    import oracle_lib
+    import tgh_desc
+    h = 1.0 / 16
+    half = N * roots * h / 2
+    args = dict(M=1.0, a=0.3, v=0.3, x0=0.1, axis=axis, halfwidth=half, r_0=0.35,
+                r_1=0.35 + max(0.55, 2 * (q // 2 + 2) * h * (1 + 1e-9)))
+    case = (tgh.harmonic_kerr_case(**args) if chart == "harmonic"
+            else tgh.kerr_schild_case(gauge_source="algebraic", **args))
+    p = tgh.GHProblem(tgh.gh_forest(None, case, N=N, roots=roots), case, q=q)
+    orc = oracle_lib.OracleProblem(tgh_desc.TghDesc.from_buffer_copy(bytes(p.desc)))
+    u0 = orc.fill_exact(0.1)
+    orc.add_noise(u0, 0x57A6F, 1e-6)
+    dt = h / 16
+    _, step_tol = bound(u0, h, dt)
+    ref = u0.copy()
+    for n in range(2):
+        orc.rk4_step(ref, 0.1 + n * dt, dt, 8)
+    # the stage-value form, the head and Pi components apart, and blocks
+    for flags in (0, tgh.TGH_RK4_SPLIT, tgh.TGH_RK4_BLOCKS | tgh.TGH_RK4_SPLIT):
+        v = torch.from_numpy(u0).cuda()
+        tgh._check(tgh._load().tgh_rk4(p.ptr, C.c_void_p(v.data_ptr()), 0.1, dt, 2, flags))
+        err = float(np.max(np.abs(v.cpu().numpy() - ref)))
+        print(f"flags {flags}: {err:.2e} (bound {2 * step_tol:.2e})")
+        assert err <= 2 * step_tol

@@ -433,14 +433,22 @@ namespace {
 
 // ---------------------------------------------------------------------------
 // The brick stepper.
-void launch_frame(tgh_problem* p, double* W, double t, double toff = 0.0) {
+// Whether the frame holds exact values alone, a function of the time, and
+// nothing of the stage's own.
+bool frame_exact(const tgh_problem* p) {
+  const Geom& g = p->geom;
+  return !g.periodic[0] && !g.periodic[1] && !g.periodic[2] && !reflects(g);
+}
+// The frame of W at t (and of W2, a stage input of the same time, where the
+// frame is exact).
+void launch_frame(tgh_problem* p, double* W, double t, double toff = 0.0, double* W2 = nullptr) {
   const Brick& k = p->brick;
   const long E = (long)(k.n[0] + 2 * k.G) * (k.n[1] + 2 * k.G) * (k.n[2] + 2 * k.G);
   // without mirrors or the seam only the frame's points have work: one thread
   // each; with them the walls' inside points are projected too
   const int shell = reflects(p->geom) ? 0 : 1;
   const long n = shell ? E - (long)k.n[0] * k.n[1] * k.n[2] : E;
-  FrameArgs a{k, p->cs, t, W, p->clock_use, toff, shell};
+  FrameArgs a{k, p->cs, t, W, p->clock_use, toff, shell, W2};
   hipLaunchKernelGGL(p->cs.moving ? k_brick_frame<true> : k_brick_frame<false>, dim3((unsigned)((n + 255) / 256)),
                      dim3(256), 0, p->stream, a);
 }
@@ -480,7 +488,7 @@ int ensure_layer_box(tgh_problem* p) {
   if (rest) {
     const long B3 = (long)p->layer_B * p->layer_B * p->layer_B;
     LayerArgs la{layer_grid(p), p->cs, 0.0, nullptr, 0.0, p->Blayer, p->layer_B};
-    hipLaunchKernelGGL(k_brick_layer<false>, dim3((unsigned)((B3 + 255) / 256), 1), dim3(256), 0, p->stream, la);
+    hipLaunchKernelGGL(k_brick_layer, dim3((unsigned)((B3 + 255) / 256)), dim3(256), 0, p->stream, la);
     HIP_TRY(hipGetLastError());
   }
   return TGH_OK;
@@ -499,14 +507,43 @@ Brick layer_grid(const tgh_problem* p) {
   k.inv_h = p->geom.inv_h * f;
   return k;
 }
-void launch_layer_box(tgh_problem* p, double t, double toff, RhsArgs& a) {
-  const long B3 = (long)p->layer_B * p->layer_B * p->layer_B;
-  if (!p->layer_static) {
-    LayerArgs la{layer_grid(p), p->cs, t, p->clock_use, toff, p->Blayer, p->layer_B};
-    hipLaunchKernelGGL(k_brick_layer<true>, dim3((unsigned)((B3 + 255) / 256), 3), dim3(256), 0, p->stream, la);
+// A moving hole's exact frame (of W and W2; W NULL: none) and layer box (if
+// it has one) at t, in one launch.
+void launch_moving(tgh_problem* p, double* W, double* W2, double t, double toff) {
+  const Brick& k = p->brick;
+  FrameArgs fa{k, p->cs, t, W, p->clock_use, toff, 1, W2};
+  LayerArgs la{};
+  unsigned fb = 0, lb = 0;
+  if (W) {
+    const long E = (long)(k.n[0] + 2 * k.G) * (k.n[1] + 2 * k.G) * (k.n[2] + 2 * k.G);
+    fb = (unsigned)((E - (long)k.n[0] * k.n[1] * k.n[2] + 63) / 64);
   }
+  if (p->Blayer && !p->layer_static) {
+    la = LayerArgs{layer_grid(p), p->cs, t, p->clock_use, toff, p->Blayer, p->layer_B};
+    lb = (unsigned)((3L * p->layer_B * p->layer_B * p->layer_B + 63) / 64);
+  }
+  if (fb + lb) hipLaunchKernelGGL(k_brick_moving, dim3(fb + lb), dim3(256), 0, p->stream, fa, la, fb);
+}
+// What a stage on the brick reads at its time besides its own values: the
+// frame of its input W, filled unless it is static, and a moving hole's layer
+// box. An RK4 step's second and third stage have the same time: the second
+// fills the third's exact frame too (W2), and nothing that depends on the time
+// alone is filled for the third (again).
+void fill_stage(tgh_problem* p, double* W, double* W2, double t, double toff, bool again) {
+  const bool exact = frame_exact(p);
+  const bool frame = !p->frame_static && !(again && exact);
+  if (p->cs.moving) {
+    if (frame && !exact) launch_frame(p, W, t, toff);
+    if (!again) launch_moving(p, frame && exact ? W : nullptr, W2, t, toff);
+  } else if (frame) {
+    launch_frame(p, W, t, toff, exact ? W2 : nullptr);
+  }
+}
+// The layer box as a stage's arguments.
+void layer_args(tgh_problem* p, RhsArgs& a) {
+  if (!p->Blayer) return;
   a.lbox = p->Blayer;
-  a.lB3 = B3;
+  a.lB3 = (long)p->layer_B * p->layer_B * p->layer_B;
   a.lB = p->layer_B;
   a.lLmax = p->layer_lmax;
 }
@@ -543,7 +580,7 @@ int ensure_brick(tgh_problem* p) {
   }
   const bool static_bg = static_background(p->cs);
   // a wrapped or mirrored frame reads the stage's own values: refilled every stage
-  p->frame_static = static_bg && !g.periodic[0] && !g.periodic[1] && !g.periodic[2] && !reflects(g);
+  p->frame_static = static_bg && frame_exact(p);
   if (p->frame_static)  // every array is a stage input in one of the forms
     for (double** a : arrs) launch_frame(p, *a, 0.0);
   {
@@ -592,18 +629,16 @@ void launch_split(tgh_problem* p, const RhsArgs& a) {
   }
 }
 // The stage's arguments on the brick: its ghosts and, for a moving hole, its
-// layer box are filled first.
-RhsArgs brick_stage_args(tgh_problem* p, double* Wc, double t, double toff) {
-  if (!p->frame_static) {
-    const bool prof = p->profiling;
-    int e0 = prof ? mark(p) : -1;
-    launch_frame(p, Wc, t, toff);
-    if (prof) p->ev_fill.push_back({e0, mark(p)});
-  }
+// layer box are filled first (fill_stage).
+RhsArgs brick_stage_args(tgh_problem* p, double* Wc, double t, double toff, double* W2 = nullptr, bool again = false) {
+  const bool prof = p->profiling && !p->frame_static;
+  int e0 = prof ? mark(p) : -1;
+  fill_stage(p, Wc, W2, t, toff, again);
+  if (prof) p->ev_fill.push_back({e0, mark(p)});
   RhsArgs a = rhs_args(p, Wc, t, nullptr);
   a.clock = p->clock_use;
   a.toff = toff;
-  if (p->Blayer) launch_layer_box(p, t, toff, a);
+  layer_args(p, a);
   a.Hsrc = p->BH;
   return a;
 }
@@ -626,13 +661,14 @@ void rk4_brick_launches(tgh_problem* p, double t, double dt, bool split) {
   if (!split && stage_values(p)) {
     double* const Y[4] = {p->BW[0], p->BW[1], p->Bus, p->Bacc};
     for (int s = 0; s < 4; ++s)
-      launch_stage(p, brick_stage_args(p, Y[s], t_stage[s], t_off[s]), stage_io(Y, Y[(s + 1) % 4], s, dt));
+      launch_stage(p, brick_stage_args(p, Y[s], t_stage[s], t_off[s], s == 1 ? Y[2] : nullptr, s == 2),
+                   stage_io(Y, Y[(s + 1) % 4], s, dt));
     return;
   }
   for (int s = 0; s < 4; ++s) {
     double* Wc = p->BW[s % 2];
     double* Wn = p->BW[(s + 1) % 2];
-    RhsArgs a = brick_stage_args(p, Wc, t_stage[s], t_off[s]);
+    RhsArgs a = brick_stage_args(p, Wc, t_stage[s], t_off[s], s == 1 ? Wn : nullptr, s == 2);
     a.us = p->Bus;
     a.acc = p->Bacc;
     a.Wn = Wn;
@@ -755,7 +791,8 @@ void rk4_block_stage_launches(tgh_problem* p, double t, double dt) {
     RhsArgs a = rhs_args(p, Wc, t_stage[s], nullptr);
     a.clock = p->clock_use;
     a.toff = t_off[s];
-    if (p->Blayer) launch_layer_box(p, t_stage[s], t_off[s], a);
+    if (p->Blayer && s != 2) launch_moving(p, nullptr, nullptr, t_stage[s], t_off[s]);  // the third: the second's time
+    layer_args(p, a);
     launch_stage_block(p, a, StageIO{s + 1, c_acc[s], c_next[s], p->Wus, p->Wus, p->Wacc, nullptr, Wn});
   }
 }
@@ -777,7 +814,8 @@ void rk4_step_launches(tgh_problem* p, double* u, double t, double dt) {
     RhsArgs a = rhs_args(p, Wc, t_stage[s], p->mat.rho ? &p->mat : nullptr);
     a.clock = p->clock_use;
     a.toff = t_off[s];
-    if (p->Blayer) launch_layer_box(p, t_stage[s], t_off[s], a);
+    if (p->Blayer && s != 2) launch_moving(p, nullptr, nullptr, t_stage[s], t_off[s]);  // the third: the second's time
+    layer_args(p, a);
     a.us = u;
     a.acc = p->acc;
     a.Wn = Wn;
@@ -1291,7 +1329,7 @@ int tgh_rhs(tgh_problem* p, double* du, double t, const tgh_matter* matter) {
   // layer box is filled once); the other cases, and a box that finds no
   // memory, one point a thread
   if (!(matter && matter->rho) && !p->cs.general && !p->cs.moving && ensure_layer_box(p) == TGH_OK && stage_ok(p)) {
-    if (p->Blayer) launch_layer_box(p, t, 0.0, a);
+    layer_args(p, a);
     launch_stage_block(p, a, StageIO{STAGE_STORE, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr, du});
   } else {
     a.du = du;
@@ -2194,11 +2232,9 @@ void batch_step_launches(tgh_batch* b, double t, double dt) {
   for (int s = 0; s < 4; ++s) {
     for (tgh_problem* p : b->probs) {
       double* const Y[4] = {p->BW[0], p->BW[1], p->Bus, p->Bacc};
-      if (!p->frame_static) launch_frame(p, stage_values(p) ? Y[s] : p->BW[s % 2], t_stage[s], t_off[s]);
-      if (p->Blayer) {
-        RhsArgs unused = rhs_args(p, p->BW[0], t_stage[s], nullptr);
-        launch_layer_box(p, t_stage[s], t_off[s], unused);
-      }
+      const bool values = stage_values(p);
+      fill_stage(p, values ? Y[s] : p->BW[s % 2], s == 1 ? (values ? Y[2] : p->BW[0]) : nullptr, t_stage[s], t_off[s],
+                 s == 2);
     }
     launch_batch_stage(b, b->d_tab + s * n);
     for (tgh_problem* p : b->probs)

@@ -638,11 +638,30 @@ TGH_HD NDual<V, K> nd_div(const NDual<V, K>& a, const NDual<V, K>& b) {
   for (int k = 0; k < K; ++k) r.d[k] = nd_div(nd_sub(nd_mul(a.d[k], b.v), nd_mul(a.v, b.d[k])), bb);
   return r;
 }
+// With a constant, whose derivatives are exact zeros: the products with them
+// and the sums of those are left out, which leaves every bit of a finite
+// result as it is.
+TGH_HD double nd_addc(double a, double b) { return nd_add(a, b); }
+TGH_HD double nd_scale(double a, double b) { return nd_mul(a, b); }
+template <class V, int K>
+TGH_HD NDual<V, K> nd_addc(const NDual<V, K>& a, double b) {
+  NDual<V, K> r = a;
+  r.v = nd_addc(a.v, b);
+  return r;
+}
+template <class V, int K>
+TGH_HD NDual<V, K> nd_scale(double a, const NDual<V, K>& b) {
+  NDual<V, K> r;
+  r.v = nd_scale(a, b.v);
+#pragma unroll
+  for (int k = 0; k < K; ++k) r.d[k] = nd_scale(a, b.d[k]);
+  return r;
+}
 template <class V, int K>
 TGH_HD NDual<V, K> nd_sqrt(const NDual<V, K>& a) {
   NDual<V, K> r;
   r.v = nd_sqrt(a.v);
-  const V two_r = nd_mul(nd_cst(2.0, (const V*)nullptr), r.v);
+  const V two_r = nd_scale(2.0, r.v);
 #pragma unroll
   for (int k = 0; k < K; ++k) r.d[k] = nd_div(a.d[k], two_r);
   return r;
@@ -658,15 +677,23 @@ TGH_HD NDual<V, K> operator*(const NDual<V, K>& a, const NDual<V, K>& b) { retur
 template <class V, int K>
 TGH_HD NDual<V, K> operator/(const NDual<V, K>& a, const NDual<V, K>& b) { return nd_div(a, b); }
 template <class V, int K>
-TGH_HD NDual<V, K> operator+(const NDual<V, K>& a, double b) { return nd_add(a, nd_cst(b, &a)); }
+TGH_HD NDual<V, K> operator+(const NDual<V, K>& a, double b) { return nd_addc(a, b); }
 template <class V, int K>
-TGH_HD NDual<V, K> operator-(const NDual<V, K>& a, double b) { return nd_sub(a, nd_cst(b, &a)); }
+TGH_HD NDual<V, K> operator+(double a, const NDual<V, K>& b) { return nd_addc(b, a); }
 template <class V, int K>
-TGH_HD NDual<V, K> operator*(double a, const NDual<V, K>& b) { return nd_mul(nd_cst(a, &b), b); }
+TGH_HD NDual<V, K> operator-(const NDual<V, K>& a, double b) { return nd_addc(a, -b); }
 template <class V, int K>
-TGH_HD NDual<V, K> operator/(const NDual<V, K>& a, double b) { return nd_div(a, nd_cst(b, &a)); }
+TGH_HD NDual<V, K> operator*(double a, const NDual<V, K>& b) { return nd_scale(a, b); }
+// a / b with a' = 0
 template <class V, int K>
-TGH_HD NDual<V, K> operator/(double a, const NDual<V, K>& b) { return nd_div(nd_cst(a, &b), b); }
+TGH_HD NDual<V, K> operator/(double a, const NDual<V, K>& b) {
+  NDual<V, K> r;
+  r.v = a / b.v;
+  const V bb = nd_mul(b.v, b.v);
+#pragma unroll
+  for (int k = 0; k < K; ++k) r.d[k] = nd_div(nd_neg(nd_scale(a, b.d[k])), bb);
+  return r;
+}
 
 // The Kerr metric in harmonic coordinates (SpacetimeMetrics' Harmonic(M, a),
 // restated from Cook & Scheel, Phys. Rev. D 56, 4775 (1997)) as the packed
@@ -682,12 +709,15 @@ TGH_HD NDual<V, K> operator/(double a, const NDual<V, K>& b) { return nd_div(nd_
 // in duals over (X, Y, Z) whose components are duals over (t, x, y, z), so
 // each entry of J carries its own first derivatives.
 using NS = NDual<double, 4>;  // a value with its derivatives in (t, x, y, z)
-TGH_HD NS ns_cst(double x) { return nd_cst(x, (const NS*)nullptr); }
+template <class S>
+TGH_HD S nd_of(double x) { return nd_cst(x, (const S*)nullptr); }
+TGH_HD NS ns_cst(double x) { return nd_of<NS>(x); }
 
 // The harmonic chart's full metric g at the hole-relative harmonic position
-// (X, Y, Z), each carried with its derivatives in (t, x, y, z).
-TGH_HD void harmonic_metric_exact(const Bg& bg, const NS& Xs, const NS& Ys, const NS& Zs, NS g[4][4]) {
-  using S = NS;
+// (X, Y, Z), each carried with its derivatives: S = NS those in (t, x, y, z),
+// S = NDual<double, 1> one of them.
+template <class S>
+TGH_HD void harmonic_metric_exact(const Bg& bg, const S& Xs, const S& Ys, const S& Zs, S g[4][4]) {
   using D3 = NDual<S, 3>;
   const double a = bg.a, M = bg.M;
   const double rm = M - sqrt(M * M - a * a);
@@ -698,11 +728,11 @@ TGH_HD void harmonic_metric_exact(const Bg& bg, const NS& Xs, const NS& Ys, cons
   for (int i = 0; i < 3; ++i) {
     P[i] = nd_cst(0.0, (const D3*)nullptr);
     P[i].v = *in[i];
-    P[i].d[i] = ns_cst(1.0);
+    P[i].d[i] = nd_of<S>(1.0);
   }
   const D3 &X = P[0], &Y = P[1], &Z = P[2];
   D3 rho2 = X * X + Y * Y + Z * Z;
-  D3 hb = (rho2 - aa) / 2.0;
+  D3 hb = 0.5 * (rho2 - aa);
   D3 R2 = hb + nd_sqrt(hb * hb + aa * Z * Z);
   D3 R = nd_sqrt(R2);
   D3 r = R + M;
@@ -712,25 +742,21 @@ TGH_HD void harmonic_metric_exact(const Bg& bg, const NS& Xs, const NS& Ys, cons
   m[0] = c1 * X - c2 * Y;
   m[1] = c2 * X + c1 * Y;
   m[2] = r * Z / R;
-  // J[c][b] = d x_KS^c / d x_H^b; the time column is the identity's.
-  S J[4][4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) J[c][b] = ns_cst(c == 0 && b == 0 ? 1.0 : 0.0);
+  // J[c][i] = d x_KS^c / d x_H^i; the time column is the identity's.
+  S J[4][3];
   const S tfac = (2.0 * M) / (r.v - rm);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    J[0][i + 1] = tfac * R.d[i];
+    J[0][i] = tfac * R.d[i];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) J[c + 1][i + 1] = m[c].d[i];
+    for (int c = 0; c < 3; ++c) J[c + 1][i] = m[c].d[i];
   }
   // g_KS at the mapped point, whose Kerr-Schild radius is r = R + M.
   const S rv = r.v, r2v = rv * rv, xv = m[0].v, yv = m[1].v, zv = m[2].v;
   const S f = (2.0 * M) * rv * r2v / (r2v * r2v + aa * zv * zv);
   const S dl = r2v + aa;
   S l[4];
-  l[0] = ns_cst(1.0);
+  l[0] = nd_of<S>(1.0);
   l[1] = (rv * xv + a * yv) / dl;
   l[2] = (rv * yv - a * xv) / dl;
   l[3] = zv / rv;
@@ -738,35 +764,46 @@ TGH_HD void harmonic_metric_exact(const Bg& bg, const NS& Xs, const NS& Ys, cons
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) gk[i][j] = ns_cst(eta(i, j)) + f * l[i] * l[j];
+    for (int j = 0; j < 4; ++j) gk[i][j] = eta(i, j) + f * l[i] * l[j];
+  // g = J^T gk J summed in the order of (c, e), without the time column's
+  // exact zeros and ones
+  g[0][0] = gk[0][0];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 3; ++i) {
+    S row = J[0][i] * gk[0][0], col = row;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      S sum = ns_cst(0.0);
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sum = sum + J[c][i] * J[e][j] * gk[c][e];
-      g[i][j] = sum;
+    for (int c = 1; c < 4; ++c) {
+      row = row + J[c][i] * gk[0][c];
+      col = col + J[c][i] * gk[c][0];
     }
+    g[0][i + 1] = row;
+    g[i + 1][0] = col;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      S sum = J[0][i] * J[0][j] * gk[0][0];
+#pragma unroll
+      for (int ce = 1; ce < 16; ++ce) sum = sum + J[ce / 4][i] * J[ce % 4][j] * gk[ce / 4][ce % 4];
+      g[i + 1][j + 1] = sum;
+    }
+  }
 }
 
 // The Kerr-Schild metric g = eta + f l l at the hole-relative position, in the
 // same fixed order (the moving hole's chart).
-TGH_HD void ks_metric_exact(const Bg& bg, const NS& X, const NS& Y, const NS& Z, NS g[4][4]) {
+template <class S>
+TGH_HD void ks_metric_exact(const Bg& bg, const S& X, const S& Y, const S& Z, S g[4][4]) {
   const double a = bg.a, M = bg.M;
-  NS rho2 = X * X + Y * Y + Z * Z;
-  NS hb = (rho2 - a * a) / 2.0;
-  NS r2 = hb + nd_sqrt(hb * hb + (a * a) * Z * Z);
-  NS r = nd_sqrt(r2);
-  NS f = (2.0 * M) * r * r2 / (r2 * r2 + (a * a) * Z * Z);
-  NS den = r2 + a * a;
-  NS l[4] = {ns_cst(1.0), (r * X + a * Y) / den, (r * Y - a * X) / den, Z / r};
+  S rho2 = X * X + Y * Y + Z * Z;
+  S hb = 0.5 * (rho2 - a * a);
+  S r2 = hb + nd_sqrt(hb * hb + (a * a) * Z * Z);
+  S r = nd_sqrt(r2);
+  S f = (2.0 * M) * r * r2 / (r2 * r2 + (a * a) * Z * Z);
+  S den = r2 + a * a;
+  S l[4] = {nd_of<S>(1.0), (r * X + a * Y) / den, (r * Y - a * X) / den, Z / r};
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) g[i][j] = ns_cst(eta(i, j)) + f * l[i] * l[j];
+    for (int j = 0; j < 4; ++j) g[i][j] = eta(i, j) + f * l[i] * l[j];
 }
 
 TGH_HD void bg_harmonic_offset(const Bg& bg, const double x[3], Dual<4> hd[NC]) {
@@ -900,6 +937,43 @@ TGH_HD void ex_lapse_shift(const double hv[NC], double& alpha, double beta[3], d
   sqrtg = sqrt(1.0 + detgm1);
 }
 
+// The moving hole's full metric at p = (t, x), its chart and boost pulled back
+// in the oracle's order with contraction off, with the derivatives that X's
+// entries are seeded with.
+template <class S>
+TGH_HD void moving_metric_exact(const Bg& bg, const S X[4], S g[4][4]) {
+  if (bg_boosted(bg)) {
+    double L[4][4];
+    lorentz_boost(bg.u, L);
+    const S xr[4] = {X[0], X[1] - bg.c[0], X[2] - bg.c[1], X[3] - bg.c[2]};
+    S xp[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) xp[c] = L[c][0] * xr[0] + L[c][1] * xr[1] + L[c][2] * xr[2] + L[c][3] * xr[3];
+    S gp[4][4];
+    if (bg.kind == BG_HARMONIC)
+      harmonic_metric_exact(bg, xp[1], xp[2], xp[3], gp);
+    else
+      ks_metric_exact(bg, xp[1], xp[2], xp[3], gp);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        S sum = nd_mul(L[0][a], L[0][b]) * gp[0][0];
+#pragma unroll
+        for (int cd = 1; cd < 16; ++cd) sum = sum + nd_mul(L[cd / 4][a], L[cd % 4][b]) * gp[cd / 4][cd % 4];
+        g[a][b] = sum;
+      }
+  } else if (bg.kind == BG_HARMONIC) {
+    harmonic_metric_exact(bg, X[1] - bg.c[0], X[2] - bg.c[1], X[3] - bg.c[2], g);
+  } else {
+    ks_metric_exact(bg, X[1] - bg.c[0], X[2] - bg.c[1], X[3] - bg.c[2], g);
+  }
+}
+// Pi = (sqrt(gamma)/alpha) q, q the metric's derivative (d_t - beta^i d_i).
+TGH_HD double moving_q(double dt, double dx, double dy, double dz, const double beta[3]) {
+  return nd_sub(nd_sub(nd_sub(dt, nd_mul(beta[0], dx)), nd_mul(beta[1], dy)), nd_mul(beta[2], dz));
+}
+
 // background_state's one dual pass (src/initialdata.jl:1683-1694) for a moving
 // hole: h = g - eta, Pi = (sqrt(gamma)/alpha)(d_t g - beta^i d_i g) and d_t h,
 // every operation in the oracle's order with contraction off. The layer's and
@@ -918,51 +992,60 @@ __host__ __device__ __noinline__ inline void bg_state_exact(const Bg& bg, double
     X[k].d[k] = 1.0;
   }
   NS g[4][4];
-  if (bg_boosted(bg)) {
-    double L[4][4];
-    lorentz_boost(bg.u, L);
-    const NS xr[4] = {X[0], X[1] - bg.c[0], X[2] - bg.c[1], X[3] - bg.c[2]};
-    NS xp[4];
+  moving_metric_exact(bg, X, g);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) xp[c] = L[c][0] * xr[0] + L[c][1] * xr[1] + L[c][2] * xr[2] + L[c][3] * xr[3];
-    NS gp[4][4];
-    if (bg.kind == BG_HARMONIC)
-      harmonic_metric_exact(bg, xp[1] - 0.0, xp[2] - 0.0, xp[3] - 0.0, gp);
-    else
-      ks_metric_exact(bg, xp[1] - 0.0, xp[2] - 0.0, xp[3] - 0.0, gp);
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        NS sum = ns_cst(0.0);
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int d = 0; d < 4; ++d) sum = sum + nd_mul(L[c][a], L[d][b]) * gp[c][d];
-        g[a][b] = sum;
-      }
-  } else if (bg.kind == BG_HARMONIC) {
-    harmonic_metric_exact(bg, X[1] - bg.c[0], X[2] - bg.c[1], X[3] - bg.c[2], g);
-  } else {
-    ks_metric_exact(bg, X[1] - bg.c[0], X[2] - bg.c[1], X[3] - bg.c[2], g);
-  }
-  double dh[3][NC];
-#pragma unroll
-  for (int n = 0; n < NC; ++n) {
-    const int i = prow(n), j = pcol(n);
-    h[n] = nd_sub(g[i][j].v, eta(i, j));
-    dtg[n] = g[i][j].d[0];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) dh[k][n] = g[i][j].d[k + 1];
-  }
+  for (int n = 0; n < NC; ++n) h[n] = nd_sub(g[prow(n)][pcol(n)].v, eta(prow(n), pcol(n)));
   double alpha, beta[3], sqrtg;
   ex_lapse_shift(h, alpha, beta, sqrtg);
   const double s = nd_div(sqrtg, alpha);
 #pragma unroll
-  for (int n = 0; n < NC; ++n)
-    P[n] = nd_mul(s, nd_sub(nd_sub(nd_sub(dtg[n], nd_mul(beta[0], dh[0][n])), nd_mul(beta[1], dh[1][n])),
-                            nd_mul(beta[2], dh[2][n])));
+  for (int n = 0; n < NC; ++n) {
+    const NS& q = g[prow(n)][pcol(n)];
+    dtg[n] = q.d[0];
+    P[n] = nd_mul(s, moving_q(q.d[0], q.d[1], q.d[2], q.d[3], beta));
+  }
 }
+
+#ifdef __HIP__
+// Lane M's value of each quad of lanes (M, +-): lanes 4 q to 4 q + 3.
+template <int M>
+__device__ __forceinline__ double quad_lane(double x) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)u, M * 0x55, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), M * 0x55, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+// bg_state_exact with the point on a quad of lanes, lane k = 0..3 carrying the
+// derivative in (t, x, y, z)[k]: the same operations, value and derivative
+// rounding as there, so the results are the same to the last bit. One
+// derivative a lane needs 2/5 of the registers, so that nothing spills, and
+// four times the waves for four times the values' work. All four lanes of a
+// quad come with the same point.
+__device__ __forceinline__ void bg_state_quad(const Bg& bg, double t, const double x[3], int k, double h[NC],
+                                              double P[NC], double dtg[NC]) {
+  using S = NDual<double, 1>;
+  S X[4];
+  const double p[4] = {t, x[0], x[1], x[2]};
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    X[m].v = p[m];
+    X[m].d[0] = m == k ? 1.0 : 0.0;
+  }
+  S g[4][4];
+  moving_metric_exact(bg, X, g);
+#pragma unroll
+  for (int n = 0; n < NC; ++n) h[n] = nd_sub(g[prow(n)][pcol(n)].v, eta(prow(n), pcol(n)));
+  double alpha, beta[3], sqrtg;
+  ex_lapse_shift(h, alpha, beta, sqrtg);
+  const double s = nd_div(sqrtg, alpha);
+#pragma unroll
+  for (int n = 0; n < NC; ++n) {
+    const double d = g[prow(n)][pcol(n)].d[0];
+    dtg[n] = quad_lane<0>(d);
+    P[n] = nd_mul(s, moving_q(dtg[n], quad_lane<1>(d), quad_lane<2>(d), quad_lane<3>(d), beta));
+  }
+}
+#endif
 
 // Sets of backgrounds, as bit masks over the kinds: a kernel compiled for one
 // set keeps only those backgrounds' code (and registers). The gauge-source

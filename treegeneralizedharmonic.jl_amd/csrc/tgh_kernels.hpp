@@ -2774,13 +2774,13 @@ struct FrameArgs {
   const double* clock;  // stage_time's clock and offset
   double toff;
   int shell;  // 1: one thread per frame point (brick_shell_point); 0: per extent point
+  double* __restrict__ W2;  // Dirichlet frames: a second array of the same time, or NULL
 };
 // A moving :damped hole's core and layer on the brick: per stage, the exact
 // background's dual passes (bg_state_exact) that the head's core and layer
 // targets are made of, for every core and layer point of the B^3 box about the
 // hole (its corner one point below the layer's bounding box about c(t)), into
-// slot layer_slot(x, y, z, B) of LAYER_FIELDS fields; grid.y is the pass, so the
-// three passes of a point run on three threads:
+// slot layer_slot(x, y, z, B) of LAYER_FIELDS fields, in three passes:
 //   a layer point (background_state_rate): pass 0 the state h, Pi and d_t h
 //     at t (fields 0-29), passes 1 and 2 Pi at t +- delta (30-39, 40-49);
 //   a core point (moving_core_target): pass 0 the state at the core rule's
@@ -2798,72 +2798,38 @@ struct LayerArgs {
   double* __restrict__ box;
   int B;
 };
-template <bool MOVING>
-__global__ __launch_bounds__(256) void k_brick_layer(LayerArgs a) {
-  a.t = stage_time(a.t, a.clock, a.toff);
+// The box slot s's grid point, if it is a core or layer point (the only ones
+// the head reads): its coordinates p, its position x, whether it is the core's.
+__device__ __forceinline__ bool layer_point(const LayerArgs& a, long s, int p[3], double x[3], bool& core) {
   const Brick& k = a.k;
   const CaseP& c = a.c;
-  const int B = a.B, pass = blockIdx.y;
-  const long B3 = (long)B * B * B;
-  const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= B3) return;
+  const int B = a.B;
   const int l[3] = {(int)(s % B), (int)((s / B) % B), (int)(s / ((long)B * B))};
   double cc[3];
   center_at(c, a.t, cc);
-  int p[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     p[d] = (int)floor((cc[d] - c.r1 - k.lo[d]) * k.inv_h) - 1 + l[d];
-    if (p[d] < 0 || p[d] >= k.n[d]) return;
+    if (p[d] < 0 || p[d] >= k.n[d]) return false;
+    x[d] = k.lo[d] + (double)p[d] * k.h;
   }
-  const double x[3] = {k.lo[0] + (double)p[0] * k.h, k.lo[1] + (double)p[1] * k.h, k.lo[2] + (double)p[2] * k.h};
   double r;
-  const bool core = frozen_core<1>(c, a.t, x, r);
-  if (!core && !(r < c.r1)) return;  // the head reads core and layer points only
-  double* dst = a.box + layer_slot(p[0], p[1], p[2], B);
-  if constexpr (!MOVING) {
-    // a hole at rest: the layer's target, once (the core's rates are zero)
-    if (core) return;
-    double ue[20];
-    case_state<BGS_STATIC>(c, a.t, x, ue);
+  core = frozen_core<1>(c, a.t, x, r);
+  return core || r < c.r1;
+}
+// A hole at rest: the layer's target, once (the core's rates are zero).
+__global__ __launch_bounds__(256) void k_brick_layer(LayerArgs a) {
+  const long B3 = (long)a.B * a.B * a.B;
+  const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= B3) return;
+  int p[3];
+  double x[3], ue[20];
+  bool core;
+  if (!layer_point(a, s, p, x, core) || core) return;
+  case_state<BGS_STATIC>(a.c, a.t, x, ue);
+  double* dst = a.box + layer_slot(p[0], p[1], p[2], a.B);
 #pragma unroll
-    for (int v = 0; v < 20; ++v) dst[v * B3] = ue[v];
-    return;
-  }
-  double hh[NC], PP[NC], dd[NC];
-  if (core) {
-    double xq[3];
-    double tq = a.t;
-    if (pass > 0) {
-#pragma clang fp contract(off)
-      const double w = smoothstep(4.0 * hole_radius(c, a.t, x) / c.r0 - 1.0);
-      if (w == 0.0) return;  // no rate there
-      tq = pass == 1 ? a.t + c.delta : a.t - c.delta;
-    }
-    core_point(c, tq, x, xq);
-    bg_state_exact(c.bg, tq, xq, hh, PP, dd);
-    const int f0 = 20 * pass;
-#pragma unroll
-    for (int v = 0; v < NC; ++v) {
-      dst[(f0 + v) * B3] = hh[v];
-      dst[(f0 + NC + v) * B3] = PP[v];
-    }
-    return;
-  }
-  const double tq = pass == 0 ? a.t : pass == 1 ? a.t + c.delta : a.t - c.delta;
-  bg_state_exact(c.bg, tq, x, hh, PP, dd);
-  if (pass == 0) {
-#pragma unroll
-    for (int v = 0; v < NC; ++v) {
-      dst[v * B3] = hh[v];
-      dst[(NC + v) * B3] = PP[v];
-      dst[(2 * NC + v) * B3] = dd[v];
-    }
-  } else {
-    const int f0 = pass == 1 ? 3 * NC : 4 * NC;
-#pragma unroll
-    for (int v = 0; v < NC; ++v) dst[(f0 + v) * B3] = PP[v];
-  }
+  for (int v = 0; v < 20; ++v) dst[v * B3] = ue[v];
 }
 
 // The frame's points (the brick's extent less its n0 x n1 x n2 inside) in x-fastest
@@ -2897,6 +2863,98 @@ __device__ __forceinline__ void brick_shell_point(const Brick& k, long s, int e[
     e[0] = (int)(q < G ? q : q + k.n[0]);
   }
 }
+// A moving hole's exact states of one stage time, in one launch: blocks below
+// frame_blocks take the frame's points (k_brick_frame's Dirichlet values, into
+// f.W and, where a second stage of the same time reads another array, f.W2),
+// the rest the layer box's points, a pass after the other. A point is a quad of
+// lanes (bg_state_quad); its lanes share the stores. Bound by FP64 arithmetic:
+// 64^3 with its layer took 0.60 ms at each of a step's four stages as two
+// kernels of one thread a point, whose five-wide duals spilled 5 KB a lane;
+// eight steps took 23.9 ms then and 6.99 with this at three of the four.
+__device__ __forceinline__ double pick4(int k, double a, double b, double c, double d) {
+  return k < 2 ? (k == 0 ? a : b) : (k == 2 ? c : d);
+}
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_brick_moving(FrameArgs f, LayerArgs a,
+                                                                                              unsigned frame_blocks) {
+  const int lane = threadIdx.x & 3;
+  double xq[3], tq;
+  double *dst, *dst2 = nullptr;
+  long stride;
+  int fh = 0, fp = NC;  // the fields of h and Pi; -1: not kept
+  bool rates = false;   // and d_t h, in the next NC
+  if (blockIdx.x < frame_blocks) {
+    const Brick& k = f.k;
+    const long s = (long)blockIdx.x * 64 + (threadIdx.x >> 2);
+    if (s >= shell_size(k)) return;
+    int e[3];
+    brick_shell_point(k, s, e);
+    double x[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) x[d] = k.lo[d] + (double)(e[d] - k.G) * k.h;
+    tq = stage_time(f.t, f.clock, f.toff);
+    core_point(f.c, tq, x, xq);
+    const long at = brick_index(k, e[0] - k.G, e[1] - k.G, e[2] - k.G);
+    dst = f.W + at;
+    if (f.W2) dst2 = f.W2 + at;
+    stride = k.fs;
+  } else {
+    a.t = stage_time(a.t, a.clock, a.toff);
+    const CaseP& c = a.c;
+    const long B3 = (long)a.B * a.B * a.B;
+    const long s3 = (long)(blockIdx.x - frame_blocks) * 64 + (threadIdx.x >> 2);
+    if (s3 >= 3 * B3) return;
+    const int pass = (int)(s3 / B3);
+    int p[3];
+    double x[3];
+    bool core;
+    if (!layer_point(a, s3 - pass * B3, p, x, core)) return;
+    tq = pass == 0 ? a.t : pass == 1 ? a.t + c.delta : a.t - c.delta;
+    dst = a.box + layer_slot(p[0], p[1], p[2], a.B);
+    stride = B3;
+    if (core) {
+      if (pass > 0) {
+#pragma clang fp contract(off)
+        const double w = smoothstep(4.0 * hole_radius(c, a.t, x) / c.r0 - 1.0);
+        if (w == 0.0) return;  // no rate there
+      }
+      core_point(c, tq, x, xq);
+      fh = 20 * pass;
+      fp = 20 * pass + NC;
+    } else {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) xq[d] = x[d];
+      rates = pass == 0;
+      if (pass > 0) {
+        fh = -1;
+        fp = (2 + pass) * NC;
+      }
+    }
+  }
+  double h[NC], P[NC], dt[NC];
+  bg_state_quad(f.c.bg, tq, xq, lane, h, P, dt);
+  // lane k keeps values 4 m + k of each ten
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    const int n = 4 * m + lane;
+    if (n >= NC) continue;
+    const bool last = m == 2;
+    const double hn = last ? (lane == 0 ? h[8] : h[9])
+                           : pick4(lane, h[4 * m & 7], h[(4 * m & 7) + 1], h[(4 * m & 7) + 2], h[(4 * m & 7) + 3]);
+    const double Pn = last ? (lane == 0 ? P[8] : P[9])
+                           : pick4(lane, P[4 * m & 7], P[(4 * m & 7) + 1], P[(4 * m & 7) + 2], P[(4 * m & 7) + 3]);
+    if (fh >= 0) dst[(fh + n) * stride] = hn;
+    dst[(fp + n) * stride] = Pn;
+    if (dst2) {
+      dst2[n * stride] = hn;
+      dst2[(NC + n) * stride] = Pn;
+    }
+    if (rates)
+      dst[(2 * NC + n) * stride] =
+          last ? (lane == 0 ? dt[8] : dt[9])
+               : pick4(lane, dt[4 * m & 7], dt[(4 * m & 7) + 1], dt[(4 * m & 7) + 2], dt[(4 * m & 7) + 3]);
+  }
+}
+
 template <bool MOVE>
 __global__ __launch_bounds__(256) void k_brick_frame(FrameArgs a) {
   a.t = stage_time(a.t, a.clock, a.toff);
@@ -2960,6 +3018,11 @@ __global__ __launch_bounds__(256) void k_brick_frame(FrameArgs a) {
     case_state<MOVE ? BGS_ALL : BGS_STATIC>(a.c, a.t, x, s);
 #pragma unroll
     for (int v = 0; v < 20; ++v) dst[v * k.fs] = s[v];
+    if (a.W2) {
+      double* dst2 = a.W2 + (dst - a.W);
+#pragma unroll
+      for (int v = 0; v < 20; ++v) dst2[v * k.fs] = s[v];
+    }
   } else {
     // the source brick point, projected as its own walls would be, times the
     // parities of the mirrors crossed
