@@ -274,7 +274,11 @@ void launch_fill(tgh_problem* p, double* W, double t, double toff = 0.0) {
       a.n = end - p->plan_off[s];
       if (a.n == 0) continue;
       a.ops = (const PlanOp*)p->d_plan + p->plan_off[s];
-      const dim3 grid((a.n + 255) / 256, 20);
+      if (s == 0) {
+        hipLaunchKernelGGL(k_fill_copies, dim3((a.n + 255) / 256), dim3(256), 0, p->stream, a);
+        continue;
+      }
+      const dim3 grid((a.n + 255) / 256, 20 / PLAN_VARS);
       switch (p->prolong) {
         case 2: launch_plan<2>(grid, p->stream, a); break;
         case 4: launch_plan<4>(grid, p->stream, a); break;
