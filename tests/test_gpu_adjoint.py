@@ -74,6 +74,39 @@ def test_vjp_is_the_transpose_of_the_oracle_tangent(tgh, name):
         assert thb[0] == thb[1] == thb[3] == thb[4] == 0.0
 
 
+# runs of 256 points that end inside a plane, one block, the wide stencils, a
+# hole without a gauge source
+ODD = {
+    "gauge_wave_q2": lambda tgh: (tgh.gauge_wave_case(eps_ko=0.5, gamma0=1.0, gamma2=-0.5), 5, 1, 2),
+    "gauge_wave_q6": lambda tgh: (tgh.gauge_wave_case(eps_ko=0.5, gamma0=1.0, gamma2=-0.5), 9, 2, 6),
+    "gauge_wave_q8": lambda tgh: (tgh.gauge_wave_case(eps_ko=0.5, gamma0=1.0, gamma2=-0.5), 11, 1, 8),
+    "harmonic_q2": lambda tgh: (tgh.harmonic_kerr_case(M=1.0, a=0.3, halfwidth=1.625, r_0=0.35, r_1=0.95, gamma2=0.1,
+                                                       rho_max=4.0), 13, 4, 2),
+    "kerr_schild_q6": lambda tgh: (tgh.kerr_schild_case(M=1.0, a=0.7, halfwidth=1.75, r_0=0.71, r_1=1.36, gamma2=0.1,
+                                                        rho_max=4.0, gauge_source="algebraic"), 14, 4, 6),
+}
+
+
+@pytest.mark.parametrize("name", list(ODD))
+def test_vjp_at_the_edges_of_its_runs(tgh, name):
+    """The identity above. Both sides are sums of the same products, each term
+    rounded a few hundred times, of up to 3e5 points: 1e-12 of the sum of their
+    magnitudes, as above."""
+    torch = torch_cuda()
+    case, N, roots, q = ODD[name](tgh)
+    dev, orc = _pair(tgh, case, N, roots, q)
+    u = orc.fill_exact(0.05)
+    orc.add_noise(u, 0xAD2, 1e-4)
+    rng = np.random.default_rng(8)
+    lam, v, pd = rng.standard_normal(u.shape), rng.standard_normal(u.shape), rng.standard_normal(5)
+    _, dF = oracle_lib.gh_rhs_jvp(orc, u, v, 0.05, pd)
+    ub, thb = tgh.vjp_rhs(dev, torch.from_numpy(u).cuda(), 0.05, torch.from_numpy(lam).cuda())
+    lhs, rhs = float(np.dot(lam, dF)), float(np.dot(ub.cpu().numpy(), v) + np.dot(thb, pd))
+    scale = float(np.abs(lam * dF).sum())
+    print(f"{name}: |diff| / scale = {abs(lhs - rhs) / scale:.2e}")
+    assert abs(lhs - rhs) <= 1e-12 * scale
+
+
 def test_adjoint_gradient_matches_the_oracle_tangent_linear_model(tgh):
     """The masked L2 error of the a = 0.7 hole (27 blocks of 12^3 at q = 2,
     closed-form source, :damped layer) after 8 steps, checkpoints every 3

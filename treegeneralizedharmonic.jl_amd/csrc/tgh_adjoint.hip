@@ -12,7 +12,7 @@ namespace tgh {
 template <int Q, int GAUGE>
 static void adj_point_hole(const tgh_problem* p, const AdjPointArgs& a, bool hole) {
   if (hole)
-    hipLaunchKernelGGL((k_adj_point<Q, GAUGE, 1>), grid_brick(p), dim3(256), 0, p->stream, a);
+    hipLaunchKernelGGL((k_adj_point<Q, GAUGE, HOLE_BOXED>), grid_brick(p), dim3(256), 0, p->stream, a);
   else
     hipLaunchKernelGGL((k_adj_point<Q, GAUGE, 0>), grid_brick(p), dim3(256), 0, p->stream, a);
 }
@@ -34,11 +34,12 @@ void launch_adj_point(const tgh_problem* p, const AdjPointArgs& a) {
   }
 }
 void launch_adj_gather(const tgh_problem* p, const AdjGatherArgs& a) {
+  const dim3 grid(grid_brick(p).x, NC);
   switch (p->q) {
-    case 2: hipLaunchKernelGGL(k_adj_gather<2>, grid_brick(p), dim3(256), 0, p->stream, a); break;
-    case 4: hipLaunchKernelGGL(k_adj_gather<4>, grid_brick(p), dim3(256), 0, p->stream, a); break;
-    case 6: hipLaunchKernelGGL(k_adj_gather<6>, grid_brick(p), dim3(256), 0, p->stream, a); break;
-    default: hipLaunchKernelGGL(k_adj_gather<8>, grid_brick(p), dim3(256), 0, p->stream, a); break;
+    case 2: hipLaunchKernelGGL(k_adj_gather<2>, grid, dim3(256), 0, p->stream, a); break;
+    case 4: hipLaunchKernelGGL(k_adj_gather<4>, grid, dim3(256), 0, p->stream, a); break;
+    case 6: hipLaunchKernelGGL(k_adj_gather<6>, grid, dim3(256), 0, p->stream, a); break;
+    default: hipLaunchKernelGGL(k_adj_gather<8>, grid, dim3(256), 0, p->stream, a); break;
   }
 }
 void launch_adj_init(const tgh_problem* p, const AdjInitArgs& a) {

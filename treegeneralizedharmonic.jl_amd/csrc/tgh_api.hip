@@ -1815,6 +1815,7 @@ int adj_prepare(tgh_problem* p) {
     return fail(TGH_EUNSUPPORTED, "the adjoint is built for the static gauge-source kinds");
   int rc = ensure_brick(p);
   if (rc) return rc;
+  if (!stage_ok(p)) return fail(TGH_EDEVICE, "allocating the layer's targets");
   const size_t fb = sizeof(double) * (size_t)p->brick.fs;
   if (!p->adjF) {
     HIP_TRY(hipMalloc(&p->adjF, AF_N * fb));
@@ -1828,6 +1829,11 @@ int adj_prepare(tgh_problem* p) {
     HIP_TRY(hipMalloc(&p->adjTh, sizeof(double) * ADJ_NPAR * adj_runs(p->brick)));
   }
   return TGH_OK;
+}
+
+AdjPointArgs adj_point_args(tgh_problem* p, double t, const double* W, const double* kb) {
+  return AdjPointArgs{p->brick, p->cs, t, W, p->BH, kb, p->adjF, p->adjTh, p->Blayer,
+                      (long)p->layer_B * p->layer_B * p->layer_B, p->layer_B};
 }
 
 // The parameters' cotangent: the per-workgroup accumulators folded in order.
@@ -1876,7 +1882,7 @@ int tgh_vjp_rhs(tgh_problem* p, const double* u, double t, const double* du_bar,
   if (!p->frame_static) launch_frame(p, p->BW[0], t);
   launch_adj_fold_copies(p, AdjCopiesArgs{p->geom, k, du_bar, p->adjK[0]});
   HIP_TRY(hipMemsetAsync(p->adjTh, 0, sizeof(double) * ADJ_NPAR * adj_runs(k), p->stream));
-  launch_adj_point(p, AdjPointArgs{k, p->cs, t, p->BW[0], p->BH, p->adjK[0], p->adjF, p->adjTh});
+  launch_adj_point(p, adj_point_args(p, t, p->BW[0], p->adjK[0]));
   launch_adj_gather(p, AdjGatherArgs{k, p->adjF, nullptr, nullptr, nullptr, p->adjL[0], 0.0, 0.0, 0, 0});
   HIP_TRY(hipMemsetAsync(u_bar, 0, sizeof(double) * (size_t)p->state_len, p->stream));
   launch_adj_to_primaries(p, AdjCopiesArgs{p->geom, k, p->adjL[0], u_bar});
@@ -1965,7 +1971,7 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
       for (int s = 4; s-- > 0;) {
         double* Wc = slot(4 * j + s);
         if (!p->frame_static) launch_frame(p, Wc, t_stage[s]);
-        launch_adj_point(p, AdjPointArgs{k, p->cs, t_stage[s], Wc, p->BH, kb, p->adjF, p->adjTh});
+        launch_adj_point(p, adj_point_args(p, t_stage[s], Wc, kb));
         launch_adj_gather(p, AdjGatherArgs{k, p->adjF, lam, lacc, kbn, nullptr, cl[s], cy[s], s == 3, s == 0});
         std::swap(kb, kbn);
       }
