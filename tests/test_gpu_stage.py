@@ -42,8 +42,10 @@ def bound(u, h, dt):
 
 
 # (q, N, roots): one 16-point row and a point over it, rows shorter than a
-# tile, y and z remainders of 1, 2 and 3, the smallest block of each order
-WAVES = [(2, 4, 1), (2, 9, 2), (4, 6, 1), (4, 6, 3), (4, 17, 1), (4, 10, 2), (6, 8, 2), (6, 11, 2), (8, 10, 2), (8, 13, 1)]
+# tile, y and z remainders of 1, 2 and 3, the smallest block of each order;
+# meshes of 1 to 243 tiles, whose Pi components 5, 2 and 1 workgroups share
+WAVES = [(2, 4, 1), (2, 9, 2), (4, 6, 1), (4, 6, 3), (4, 17, 1), (4, 10, 2), (6, 8, 2), (6, 11, 2), (8, 10, 2), (8, 13, 1),
+         (4, 12, 3)]
 HOLES = [(2, 13, 4), (4, 13, 4), (4, 11, 5), (6, 18, 3), (8, 27, 2)]
 
 
@@ -64,11 +66,11 @@ def test_stage_matches_the_oracle_at_the_edges_of_its_tiles(tgh, make, q, N, roo
     err = float(np.max(np.abs(du.cpu().numpy() - orc.gh_rhs(u0, 0.1, 8))))
     print(f"rhs: {err:.2e} (bound {rhs_tol:.2e})")
     assert err <= rhs_tol
-    # two steps in the stage-value form, on bricks and in the block layout's tiles
+    # two steps in the stage-value form, on bricks, replayed, and in the block layout's tiles
     ref = u0.copy()
     for n in range(2):
         orc.rk4_step(ref, 0.1 + n * dt, dt, 8)
-    for flags in (0, tgh.TGH_RK4_BLOCKS | tgh.TGH_RK4_SPLIT):
+    for flags in (0, tgh.TGH_RK4_GRAPH, tgh.TGH_RK4_BLOCKS | tgh.TGH_RK4_SPLIT):
         v = torch.from_numpy(u0).cuda()
         tgh._check(tgh._load().tgh_rk4(p.ptr, C.c_void_p(v.data_ptr()), 0.1, dt, 2, flags))
         err = float(np.max(np.abs(v.cpu().numpy() - ref)))

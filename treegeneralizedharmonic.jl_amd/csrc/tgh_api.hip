@@ -632,12 +632,25 @@ void launch_split(tgh_problem* p, const RhsArgs& a) {
     default: launch_rhs_brick<8>(p, a); break;
   }
 }
+// Whether the stages write their results' images across the periodic faces
+// themselves, so that only a call's first stage finds its frame by a launch of
+// its own: all of the frame is images, at most one a point and axis, and no
+// interior (whose kernels have no registers to spare). Nothing then depends on
+// the time. One block of 16^3, ten steps: 1247 us with the frame kernel, the
+// clock's launch and a tile's Pi components in one workgroup, 775 without.
+bool stage_wraps(const tgh_problem* p) {
+  const Brick& k = p->brick;
+  bool ok = p->cs.interior == INT_NONE && !p->cs.moving && stage_values(p);
+  for (int d = 0; d < 3; ++d) ok = ok && k.periodic[d] && k.n[d] >= 2 * k.G;
+  return ok;
+}
 // The stage's arguments on the brick: its ghosts and, for a moving hole, its
 // layer box are filled first (fill_stage).
-RhsArgs brick_stage_args(tgh_problem* p, double* Wc, double t, double toff, double* W2 = nullptr, bool again = false) {
-  const bool prof = p->profiling && !p->frame_static;
+RhsArgs brick_stage_args(tgh_problem* p, double* Wc, double t, double toff, double* W2 = nullptr, bool again = false,
+                         bool filled = false) {
+  const bool prof = p->profiling && !p->frame_static && !filled;
   int e0 = prof ? mark(p) : -1;
-  fill_stage(p, Wc, W2, t, toff, again);
+  if (!filled) fill_stage(p, Wc, W2, t, toff, again);
   if (prof) p->ev_fill.push_back({e0, mark(p)});
   RhsArgs a = rhs_args(p, Wc, t, nullptr);
   a.clock = p->clock_use;
@@ -651,7 +664,7 @@ RhsArgs brick_stage_args(tgh_problem* p, double* Wc, double t, double toff, doub
 // the result in out.
 StageIO stage_io(double* const Y[4], double* out, int s, double dt) {
   const double c_next[4] = {dt / 2, dt / 2, dt, 0.0};
-  return StageIO{STAGE_Y1 + s, dt / 6, c_next[s], Y[0], nullptr, Y[1], Y[2], out};
+  return StageIO{STAGE_Y1 + s, dt / 6, c_next[s], Y[0], nullptr, Y[1], Y[2], out, 0};
 }
 
 // One RK4 step on the brick arrays. In the stage-value form u_n and u_{n+1}
@@ -664,9 +677,12 @@ void rk4_brick_launches(tgh_problem* p, double t, double dt, bool split) {
   const double t_stage[4] = {t, t + dt / 2, t + dt / 2, t + dt};
   if (!split && stage_values(p)) {
     double* const Y[4] = {p->BW[0], p->BW[1], p->Bus, p->Bacc};
-    for (int s = 0; s < 4; ++s)
-      launch_stage(p, brick_stage_args(p, Y[s], t_stage[s], t_off[s], s == 1 ? Y[2] : nullptr, s == 2),
-                   stage_io(Y, Y[(s + 1) % 4], s, dt));
+    const bool wraps = stage_wraps(p);
+    for (int s = 0; s < 4; ++s) {
+      StageIO io = stage_io(Y, Y[(s + 1) % 4], s, dt);
+      io.images = wraps;
+      launch_stage(p, brick_stage_args(p, Y[s], t_stage[s], t_off[s], s == 1 ? Y[2] : nullptr, s == 2, wraps), io);
+    }
     return;
   }
   for (int s = 0; s < 4; ++s) {
@@ -682,7 +698,7 @@ void rk4_brick_launches(tgh_problem* p, double t, double dt, bool split) {
     if (split)
       launch_split(p, a);
     else
-      launch_stage(p, a, StageIO{s + 1, c_acc[s], c_next[s], p->Bus, p->Bus, p->Bacc, nullptr, Wn});
+      launch_stage(p, a, StageIO{s + 1, c_acc[s], c_next[s], p->Bus, p->Bus, p->Bacc, nullptr, Wn, 0});
     // the stage limiter on the stage value (and on the step's result): the
     // range projection, then the :pasted overwrite
     if (p->has_bounds) launch_bounds_brick(p, s == 3 ? p->Bus : Wn, s == 3 ? Wn : nullptr);
@@ -797,7 +813,7 @@ void rk4_block_stage_launches(tgh_problem* p, double t, double dt) {
     a.toff = t_off[s];
     if (p->Blayer && s != 2) launch_moving(p, nullptr, nullptr, t_stage[s], t_off[s]);  // the third: the second's time
     layer_args(p, a);
-    launch_stage_block(p, a, StageIO{s + 1, c_acc[s], c_next[s], p->Wus, p->Wus, p->Wacc, nullptr, Wn});
+    launch_stage_block(p, a, StageIO{s + 1, c_acc[s], c_next[s], p->Wus, p->Wus, p->Wacc, nullptr, Wn, 0});
   }
 }
 
@@ -1334,7 +1350,7 @@ int tgh_rhs(tgh_problem* p, double* du, double t, const tgh_matter* matter) {
   // memory, one point a thread
   if (!(matter && matter->rho) && !p->cs.general && !p->cs.moving && ensure_layer_box(p) == TGH_OK && stage_ok(p)) {
     layer_args(p, a);
-    launch_stage_block(p, a, StageIO{STAGE_STORE, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr, du});
+    launch_stage_block(p, a, StageIO{STAGE_STORE, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr, du, 0});
   } else {
     a.du = du;
     launch_rhs(p, a, EPI_STORE);
@@ -1689,6 +1705,7 @@ int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int
     double* un = brick_un(p, split);
     BrickCopyArgs ca{p->geom, p->brick, u, p->BW[0], un == p->BW[0] ? nullptr : un, 0};
     hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, p->stream, ca);
+    if (form == 2 && stage_wraps(p)) launch_frame(p, p->BW[0], t0);
   } else {
     // the first stage input: u_n scattered into W[0]
     launch_scatter(p, u, p->W[0], 1);
@@ -1765,7 +1782,9 @@ int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int
         p->graph_key[0] = dt;
         p->graph_key[1] = (double)(uintptr_t)u;
       }
-      hipLaunchKernelGGL(k_set_clock, dim3(1), dim3(1), 0, p->stream, p->d_clock, t);
+      // (unless nothing depends on the time)
+      if (n == 0 || form != 2 || !stage_wraps(p))
+        hipLaunchKernelGGL(k_set_clock, dim3(1), dim3(1), 0, p->stream, p->d_clock, t);
       HIP_TRY(hipGraphLaunch(p->graph_exec, p->stream));
     }
   }
@@ -2141,7 +2160,7 @@ int batch_tables(tgh_batch* b, double t, double dt) {
       e.W = (decltype(e.W))e.a.W;
       e.Hsrc = (decltype(e.Hsrc))e.a.Hsrc;
       entry_io(e, values ? stage_io(Y, Y[(s + 1) % 4], s, dt)
-                         : StageIO{s + 1, c_acc[s], c_next[s], p->Bus, p->Bus, p->Bacc, nullptr, p->BW[(s + 1) % 2]});
+                         : StageIO{s + 1, c_acc[s], c_next[s], p->Bus, p->Bus, p->Bacc, nullptr, p->BW[(s + 1) % 2], 0});
       e.wg0 = w0;
     }
     w0 += stage_tiles(p);
@@ -2179,7 +2198,7 @@ int batch_tables_blocks(tgh_batch* b, double* const* u, double t, double dt) {
       e.W = (decltype(e.W))e.a.W;
       e.Hsrc = (decltype(e.Hsrc))e.a.Hsrc;
       double* us = b->lds ? p->Wus : u[i];
-      entry_io(e, StageIO{s + 1, c_acc[s], c_next[s], us, us, b->lds ? p->Wacc : p->acc, nullptr, p->W[(s + 1) % 2]});
+      entry_io(e, StageIO{s + 1, c_acc[s], c_next[s], us, us, b->lds ? p->Wacc : p->acc, nullptr, p->W[(s + 1) % 2], 0});
       e.wg0 = w0;
       e.lLmax = p->layer_lmax;
     }

@@ -212,8 +212,9 @@ struct StageBrickLaunch {
     using TT = StageTile<Q, TILE_BRICK>;
     const Brick& k = p->brick;
     const int total = brick_stage_tiles<Q>(k);
-    hipLaunchKernelGGL((k_brick_stage<Q, GAUGE, HOLE>), xcd_grid(total), dim3(256), 0, p->stream, a, k, a.W, a.Hsrc,
-                       io, total);
+    dim3 grid = xcd_grid(total);
+    if (HOLE == 0) grid.y = stage_parts(total);
+    hipLaunchKernelGGL((k_brick_stage<Q, GAUGE, HOLE>), grid, dim3(256), 0, p->stream, a, k, a.W, a.Hsrc, io, total);
   }
 };
 template <int Q>

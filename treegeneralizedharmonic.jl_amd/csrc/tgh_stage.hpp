@@ -272,7 +272,26 @@ struct StageIO {
   double* acc;        // the accumulator (1-4), or Y1 (14)
   const double* y2;   // Y2 (14)
   double* out;        // the next stage's input; k (0)
+  int images;         // 11-14: out's images across the periodic faces too (stage_wraps)
 };
+// A point's images across the periodic faces; a mesh of at least 2 G points an
+// axis has one an axis at most.
+struct Images {
+  int mask;  // per axis two bits: 1 the image lies above, 2 below
+  int n[3];  // the axes' lengths in bytes
+};
+template <bool ON>
+__device__ __forceinline__ Images images_of(const Brick& k, int on, int x, int y, int z) {
+  Images m{0, {8 * k.n[0], 8 * (int)k.py * k.n[1], 8 * (int)k.pz * k.n[2]}};
+  if constexpr (ON) {
+    if (on) {
+      const int p[3] = {x, y, z};
+#pragma unroll
+      for (int d = 0; d < 3; ++d) m.mask |= (p[d] < k.G ? 1 : p[d] >= k.n[d] - k.G ? 2 : 0) << (2 * d);
+    }
+  }
+  return m;
+}
 // The epilogue's kinds, compiled apart so that a kind's loads are unconditional:
 // loads under a branch make the wait for them a wait for every load in flight,
 // the next component's prefetch among them.
@@ -306,9 +325,9 @@ __device__ __forceinline__ EpiIn stage_load(const StageIO& s, int v, long ss, un
   if (K == K_Y4) e.b = field_ld(s.y2, v, ss, o);
   return e;
 }
-template <int K>
+template <int K, bool IMG>
 __device__ __forceinline__ void stage_store(const StageIO& s, int v, long ss, unsigned& o, double own, const EpiIn& e,
-                                            double k) {
+                                            double k, const Images& im) {
 #pragma clang fp contract(off)
   double x = k;
   if (K == K_Y1) x = fma(s.cnext, k, own);
@@ -321,6 +340,23 @@ __device__ __forceinline__ void stage_store(const StageIO& s, int v, long ss, un
     field_st(s.usw, v, ss, o, x);
   }
   field_st(s.out, v, ss, o, x);
+  if constexpr (IMG && (K == K_Y1 || K == K_Y23 || K == K_Y4)) {
+    if (im.mask) {
+#pragma unroll
+      for (int m = 1; m < 8; ++m) {
+        unsigned oi = o;
+        bool has = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+          if (m >> d & 1) {
+            const int b = im.mask >> (2 * d) & 3;
+            has = has && b;
+            oi += (unsigned)(b == 1 ? im.n[d] : -im.n[d]);
+          }
+        if (has) field_st(s.out, v, ss, oi, x);
+      }
+    }
+  }
 }
 template <int K>
 struct KindC {
@@ -365,11 +401,12 @@ __device__ __forceinline__ void stage_kind(int stage, const F& f) {
   return f(KindC<K_C4>{});
 }
 
-// One tile, corner (X0, Y0, Z0), of the stage's right-hand side.
+// One tile, corner (X0, Y0, Z0), of the stage's right-hand side: the head with
+// h's results (where vb is 0), and the Pi components vb to ve - 1.
 template <int Q, int GAUGE, int HOLE, int T>
 __device__ __forceinline__ void stage_tile(const RhsArgs& a, const Brick& k, const double* __restrict__ W,
                                            const double* __restrict__ Hsrc, const StageIO& io, bool state_out,
-                                           int X0, int Y0, int Z0) {
+                                           int X0, int Y0, int Z0, int vb = 0, int ve = NC) {
 #pragma clang fp contract(off)
   using TT = StageTile<Q, T>;
   constexpr int TX = TT::X, TY = TT::Y, TZ = TT::Z, R = TT::R, H = TT::H;
@@ -392,6 +429,8 @@ __device__ __forceinline__ void stage_tile(const RhsArgs& a, const Brick& k, con
     ss = (long)P * P * P;
     so = valid ? (unsigned)(x + P * (y + P * z)) * 8u : 0u;
   }
+  constexpr bool IMG = HOLE == 0 && T == TILE_BRICK;
+  const Images im = images_of<IMG>(k, io.images, x, y, z);
   double* c1 = sc1 + t;
   double pb[3], pdivb = 0.0, pA[6], pw = 1.0, pe = 0.0;
 #pragma unroll
@@ -416,12 +455,13 @@ __device__ __forceinline__ void stage_tile(const RhsArgs& a, const Brick& k, con
       double dh[NC], dP[NC];
       const GlobalSrc src{W + off, k.fs, py, pz};
       core_rates<GAUGE, HOLE>(a, xp, lslot, src, dh, dP);
-      stage_kind<T>(io.stage, [&](auto kc) {
-        constexpr int K = decltype(kc)::value;
+      if (vb == 0)
+        stage_kind<T>(io.stage, [&](auto kc) {
+          constexpr int K = decltype(kc)::value;
 #pragma unroll
-        for (int v = 0; v < NC; ++v)
-          stage_store<K>(io, v, ss, so, at(v, off), stage_load<K>(io, v, ss, so), dh[v]);
-      });
+          for (int v = 0; v < NC; ++v)
+            stage_store<K, IMG>(io, v, ss, so, at(v, off), stage_load<K>(io, v, ss, so), dh[v], im);
+        });
 #pragma unroll
       for (int v = 0; v < NC; ++v) c1[v * 256] = dP[v];
       pw = -1.0;
@@ -513,17 +553,18 @@ __device__ __forceinline__ void stage_tile(const RhsArgs& a, const Brick& k, con
         }
         dth[v] = d;
       }
-      stage_kind<T>(io.stage, [&](auto kc) {
-        constexpr int K = decltype(kc)::value;
+      if (vb == 0)
+        stage_kind<T>(io.stage, [&](auto kc) {
+          constexpr int K = decltype(kc)::value;
 #pragma unroll
-        for (int v0 = 0; v0 < NC; v0 += 5) {
-          EpiIn e[5];
+          for (int v0 = 0; v0 < NC; v0 += 5) {
+            EpiIn e[5];
 #pragma unroll
-          for (int q = 0; q < 5; ++q) e[q] = stage_load<K>(io, v0 + q, ss, so);
+            for (int q = 0; q < 5; ++q) e[q] = stage_load<K>(io, v0 + q, ss, so);
 #pragma unroll
-          for (int q = 0; q < 5; ++q) stage_store<K>(io, v0 + q, ss, so, h[v0 + q], e[q], dth[v0 + q]);
-        }
-      });
+            for (int q = 0; q < 5; ++q) stage_store<K, IMG>(io, v0 + q, ss, so, h[v0 + q], e[q], dth[v0 + q], im);
+          }
+        });
       // the gauge source in the frame, and its symmetrised derivative dHs
       double Hf[4] = {0.0, 0.0, 0.0, 0.0}, dHs[NC];
       constexpr bool HAS_H = gauge_has_source(GAUGE);
@@ -710,7 +751,7 @@ __device__ __forceinline__ void stage_tile(const RhsArgs& a, const Brick& k, con
     for (int j = 0; j < TT::NPL; ++j) rp[j] = lane_ld(wp, gp[j]);
     rc = lane_ld(wp, offc);
   };
-  fetch(0);
+  fetch(vb);
   const int ch = (lx + R) + TT::BX * ((ly + R) + TT::BY * (lz + R));
   const int cpx = (ly + TY * lz) * (TX + 2 * H) + lx + H;
   const int cpy = TT::PX + (lz * (TY + 2 * H) + ly + H) * TX + lx;
@@ -718,7 +759,7 @@ __device__ __forceinline__ void stage_tile(const RhsArgs& a, const Brick& k, con
   stage_kind<T>(io.stage, [&](auto kc) {
     constexpr int K = decltype(kc)::value;
 #pragma unroll 1
-    for (int v = 0; v < NC; ++v) {
+    for (int v = vb; v < ve; ++v) {
       double* bh = sh + (TT::NB == 2 ? (v & 1) * TT::LV : 0);
       double* bp = bh + TT::BV;
       if (TT::NB == 1) __syncthreads();  // the previous component's reads are done
@@ -738,7 +779,7 @@ __device__ __forceinline__ void stage_tile(const RhsArgs& a, const Brick& k, con
       // components back from the writes above
       __syncthreads();
       const EpiIn e = stage_load<K>(io, NC + v, ss, so);
-      if (v + 1 < NC) fetch(v + 1);
+      if (v + 1 < ve) fetch(v + 1);
       const double* ph = bh + ch;
       constexpr int st[3] = {1, TT::BX, TT::BX * TT::BY};
       constexpr int pst[3] = {1, TX, TX * TY};
@@ -822,7 +863,7 @@ __device__ __forceinline__ void stage_tile(const RhsArgs& a, const Brick& k, con
       s = fma(pA[4], mixed_sum(mx[0]), s);
       // in the frozen core (pw < 0) the rate is the coefficient itself
       s = (pw < 0.0 ? 0.0 : s * pw) + c1[v * 256];
-      if (valid) stage_store<K>(io, NC + v, ss, so, P, e, s);
+      if (valid) stage_store<K, IMG>(io, NC + v, ss, so, P, e, s, im);
     }
   });
 }
@@ -832,6 +873,12 @@ __host__ __device__ inline int brick_stage_tiles(const Brick& k) {
   using TT = StageTile<Q, TILE_BRICK>;
   return ((k.n[0] + TT::X - 1) / TT::X) * ((k.n[1] + TT::Y - 1) / TT::Y) * ((k.n[2] + TT::Z - 1) / TT::Z);
 }
+// How many workgroups share a tile's Pi components, each with the head of its
+// own, on a mesh without an interior: as many as leave at most one workgroup a
+// CU, where a tile takes as long as its instructions do one after another. A
+// stage at q = 4 in 1, 2 and 5 parts: 16 tiles 31, 24 and 20 us; 72 tiles 32,
+// 25 and 27; 128 tiles 33, 26 and 35; 243 tiles 34, 34 and 52.
+__host__ __device__ inline int stage_parts(int tiles) { return tiles * 5 <= 256 ? 5 : tiles * 2 <= 256 ? 2 : 1; }
 // The brick's tiles in launch order: the XCDs take contiguous ranges of slabs
 // in y, each swept plane of tiles by plane of tiles in z, so that the eight
 // sweep the same planes and share them in the memory-side cache (a step of
@@ -859,7 +906,14 @@ TGH_STAGE_KERNEL void k_brick_stage(RhsArgs a, Brick k, const double* __restrict
   if (L >= total) return;  // uniform over the workgroup
   int X0, Y0, Z0;
   stage_brick_tile<Q>(k, L, X0, Y0, Z0);
-  stage_tile<Q, GAUGE, HOLE, TILE_BRICK>(a, k, W, Hsrc, io, false, X0, Y0, Z0);
+  if constexpr (HOLE != 0) {
+    stage_tile<Q, GAUGE, HOLE, TILE_BRICK>(a, k, W, Hsrc, io, false, X0, Y0, Z0);
+  } else {
+    // part blockIdx.y of the Pi components (stage_parts)
+    const int parts = gridDim.y, part = blockIdx.y;
+    stage_tile<Q, GAUGE, HOLE, TILE_BRICK>(a, k, W, Hsrc, io, false, X0, Y0, Z0, NC * part / parts,
+                                           NC * (part + 1) / parts);
+  }
 }
 
 // The block layout: tile wx of block b, each block's work array a brick. The
@@ -897,7 +951,7 @@ TGH_STAGE_KERNEL void k_block_stage(RhsArgs a, const double* __restrict__ W, con
 // range of logical workgroups from wg0.
 __device__ __forceinline__ StageIO batch_io(const BatchEntry& e) {
   return StageIO{e.a.stage, e.a.cacc, e.a.cnext, (double*)e.us, (double*)e.us, (double*)e.acc, (double*)e.y2,
-                 (double*)e.Wn};
+                 (double*)e.Wn, 0};
 }
 template <int Q, int GAUGE, int HOLE>
 TGH_STAGE_KERNEL void k_brick_stage_batch(const BatchEntry* __restrict__ tab, int n, int total) {
