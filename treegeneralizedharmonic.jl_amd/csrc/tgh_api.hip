@@ -1703,7 +1703,7 @@ int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int
     }
     // u_n into the first stage input, and into the stepper's u_n where that is another array
     double* un = brick_un(p, split);
-    BrickCopyArgs ca{p->geom, p->brick, u, p->BW[0], un == p->BW[0] ? nullptr : un, 0};
+    BrickCopyArgs ca{p->geom, p->brick, u, p->BW[0], un == p->BW[0] ? nullptr : un};
     hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, p->stream, ca);
     if (form == 2 && stage_wraps(p)) launch_frame(p, p->BW[0], t0);
   } else {
@@ -1790,11 +1790,9 @@ int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int
   }
   if (rc == TGH_OK && form == 5) launch_scatter(p, u, p->Wus, 0);  // u_{n+1} back into the state
   if (rc == TGH_OK && in_brick) {
-    // u_{n+1} back into the state: the copies, then the primaries
-    for (int pass = 0; pass < 2; ++pass) {
-      BrickCopyArgs ca{p->geom, p->brick, brick_un(p, split), u, nullptr, pass};
-      hipLaunchKernelGGL(k_brick_out, grid_points(p), dim3(256), 0, p->stream, ca);
-    }
+    // u_{n+1} back into the state
+    BrickCopyArgs ca{p->geom, p->brick, brick_un(p, split), u, nullptr};
+    hipLaunchKernelGGL(k_brick_out, grid_brick(p), dim3(256), 0, p->stream, ca);
   }
   if (rc == TGH_OK && reflects(p->geom)) {
     // gh_solve returns a settled state (src/stepping.jl:235-239): the walls'
@@ -1896,7 +1894,7 @@ int tgh_vjp_rhs(tgh_problem* p, const double* u, double t, const double* du_bar,
   int rc = adj_prepare(p);
   if (rc) return rc;
   const Brick& k = p->brick;
-  BrickCopyArgs ca{p->geom, k, u, p->BW[0], p->Bus, 0};
+  BrickCopyArgs ca{p->geom, k, u, p->BW[0], p->Bus};
   hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, p->stream, ca);
   if (!p->frame_static) launch_frame(p, p->BW[0], t);
   launch_adj_fold_copies(p, AdjCopiesArgs{p->geom, k, du_bar, p->adjK[0]});
@@ -1947,7 +1945,7 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
   const bool split = !stage_ok(p);  // as tgh_rk4's default
   // ---- forward: u_0 into the brick, a checkpoint at each segment's start ----
   HIP_TRY(hipEventRecord(ev[0], p->stream));
-  BrickCopyArgs ca{p->geom, k, u, p->BW[0], p->Bus, 0};
+  BrickCopyArgs ca{p->geom, k, u, p->BW[0], p->Bus};
   hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, p->stream, ca);
   for (size_t sg = 0; sg < nseg; ++sg) {
     HIP_TRY(hipMemcpyAsync(ckpt(sg), p->BW[0], fb20, hipMemcpyDeviceToDevice, p->stream));
@@ -1955,10 +1953,8 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
     for (int n = n0; n < n1; ++n) rk4_brick_launches(p, t0 + n * dt, dt, split);
   }
   HIP_TRY(hipEventRecord(ev[1], p->stream));
-  for (int pass = 0; pass < 2; ++pass) {
-    BrickCopyArgs co{p->geom, k, brick_un(p, split), u, nullptr, pass};
-    hipLaunchKernelGGL(k_brick_out, grid_points(p), dim3(256), 0, p->stream, co);
-  }
+  BrickCopyArgs co{p->geom, k, brick_un(p, split), u, nullptr};
+  hipLaunchKernelGGL(k_brick_out, grid_brick(p), dim3(256), 0, p->stream, co);
   // J = the masked L2 error at T, and lambda_T = dJ/du_T
   const double T = t0 + nsteps * dt;
   rc = reduce(p, u, T, 1);
@@ -2390,7 +2386,7 @@ int tgh_batch_rk4(tgh_batch* b, double* const* u, double t0, double dt, int32_t 
       continue;
     }
     double* un = brick_un(p, false);
-    BrickCopyArgs ca{p->geom, p->brick, u[i], p->BW[0], un == p->BW[0] ? nullptr : un, 0};
+    BrickCopyArgs ca{p->geom, p->brick, u[i], p->BW[0], un == p->BW[0] ? nullptr : un};
     hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, b->stream, ca);
   }
   const std::vector<double*> uv(u, u + n);
@@ -2444,10 +2440,8 @@ int tgh_batch_rk4(tgh_batch* b, double* const* u, double t0, double dt, int32_t 
     for (int i = 0; i < n && b->lds; ++i) launch_scatter(b->probs[i], u[i], b->probs[i]->Wus, 0);
     for (int i = 0; i < n && !b->blocks; ++i) {  // (the block layout wrote u in place)
       tgh_problem* p = b->probs[i];
-      for (int pass = 0; pass < 2; ++pass) {
-        BrickCopyArgs ca{p->geom, p->brick, brick_un(p, false), u[i], nullptr, pass};
-        hipLaunchKernelGGL(k_brick_out, grid_points(p), dim3(256), 0, b->stream, ca);
-      }
+      BrickCopyArgs ca{p->geom, p->brick, brick_un(p, false), u[i], nullptr};
+      hipLaunchKernelGGL(k_brick_out, grid_brick(p), dim3(256), 0, b->stream, ca);
     }
     hipError_t e = hipStreamSynchronize(b->stream);
     if (e == hipSuccess) e = hipGetLastError();
