@@ -1596,8 +1596,9 @@ __global__ __launch_bounds__(256) void k_fill_copies(PlanArgs a) {
 }
 // The prolongations (the later passes): one thread per entry and PLAN_VARS of
 // its variables; a pass's entries are sorted by mode on the host, so a wave
-// takes one branch.
-enum { PLAN_VARS = 4 };
+// takes one branch. Bound by the L1 (43 loads a value at order 6): 1, 2, 4 and
+// 10 variables a thread take 0.736, 0.719, 0.750 and 0.823 ms a pass there.
+enum { PLAN_VARS = 2 };
 template <int NP>
 __global__ __launch_bounds__(256) void k_fill_plan(PlanArgs a) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
