@@ -107,6 +107,24 @@ def test_vjp_at_the_edges_of_its_runs(tgh, name):
     assert abs(lhs - rhs) <= 1e-12 * scale
 
 
+@pytest.mark.parametrize("N,roots,q", [(8, 2, 4), (9, 1, 6)])
+def test_the_adjoints_forward_sweep_on_a_periodic_mesh_is_the_steppers(tgh, N, roots, q):
+    """The state that the forward sweep leaves is the stepper's, bit for bit: it
+    enters the brick with its frame filled, whatever the brick held before."""
+    torch = torch_cuda()
+    case = tgh.gauge_wave_case(eps_ko=0.5, gamma0=1.0, gamma2=-0.5)
+    dev, orc = _pair(tgh, case, N, roots, q)
+    u0 = orc.fill_exact(0.0)
+    orc.add_noise(u0, 0xAD3, 1e-4)
+    dt = 1.0 / (8 * N * roots)
+    u = torch.from_numpy(u0).cuda()
+    J, _, _ = tgh.adjoint(dev, u, 0.0, dt, 3, every=2)
+    fresh, _ = _pair(tgh, case, N, roots, q)
+    v = torch.from_numpy(u0).cuda()
+    tgh._check(tgh._load().tgh_rk4(fresh.ptr, tgh.C.c_void_p(v.data_ptr()), 0.0, dt, 3, 0))
+    assert np.isfinite(J) and torch.equal(u, v)
+
+
 def test_adjoint_gradient_matches_the_oracle_tangent_linear_model(tgh):
     """The masked L2 error of the a = 0.7 hole (27 blocks of 12^3 at q = 2,
     closed-form source, :damped layer) after 8 steps, checkpoints every 3

@@ -463,7 +463,7 @@ bool static_background(const CaseP& c) {
   return !c.moving && (kind == BG_MINKOWSKI || kind == BG_KERR_SCHILD || kind == BG_SHIFTED || kind == BG_HARMONIC);
 }
 
-// The layer box (k_brick_layer) of a moving :damped hole or of a hole at
+// The layer box (k_brick_moving, k_brick_layer) of a moving :damped hole or of a hole at
 // rest, on the finest level's grid: the layer's bounding box about c(t) with
 // a point of margin each side, whatever t (slots wrap modulo B). Nothing for
 // other cases.
@@ -636,7 +636,8 @@ void launch_split(tgh_problem* p, const RhsArgs& a) {
 // themselves, so that only a call's first stage finds its frame by a launch of
 // its own: all of the frame is images, at most one a point and axis, and no
 // interior (whose kernels have no registers to spare). Nothing then depends on
-// the time. One block of 16^3, ten steps: 1247 us with the frame kernel, the
+// the time. Whoever brings a state into the brick for rk4_brick_launches fills
+// its frame then. One block of 16^3, ten steps: 1247 us with the frame kernel, the
 // clock's launch and a tile's Pi components in one workgroup, 775 without.
 bool stage_wraps(const tgh_problem* p) {
   const Brick& k = p->brick;
@@ -1947,6 +1948,7 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
   HIP_TRY(hipEventRecord(ev[0], p->stream));
   BrickCopyArgs ca{p->geom, k, u, p->BW[0], p->Bus};
   hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, p->stream, ca);
+  if (!split && stage_wraps(p)) launch_frame(p, p->BW[0], t0);
   for (size_t sg = 0; sg < nseg; ++sg) {
     HIP_TRY(hipMemcpyAsync(ckpt(sg), p->BW[0], fb20, hipMemcpyDeviceToDevice, p->stream));
     const int n0 = (int)(sg * every), n1 = std::min(nsteps, (int)((sg + 1) * every));

@@ -19,7 +19,7 @@ enum { GAUGE_NONE = 0, GAUGE_SAMPLED = 1, GAUGE_KS = 2, GAUGE_KS_MOVING = 3, GAU
 // The kernels' interior kinds (template HOLE): 0 none, 1 the sphere, 2 the
 // general interior (tracked geometry, :fitted), 3 the sphere of a moving
 // :damped hole or of a harmonic hole at rest, whose core and layer targets
-// come from the box of k_brick_layer (per stage, or once at rest) instead of
+// come from the layer box (k_brick_moving, or k_brick_layer at rest) instead of
 // the dual passes in the head.
 enum { HOLE_BOXED = 3 };
 constexpr bool gauge_has_source(int gauge) { return gauge == GAUGE_SAMPLED || gauge == GAUGE_KS || gauge == GAUGE_KS_MOVING; }
@@ -675,7 +675,7 @@ struct RhsArgs {
   const double* clock;  // stage_time's clock (NULL: t as given) and offset
   double toff;
   // a moving hole's layer targets and rates on the brick, evaluated per stage by
-  // k_brick_layer (LAYER_FIELDS fields of lB^3 slots, slot = brick coordinates mod lB);
+  // k_brick_moving (LAYER_FIELDS fields of lB^3 slots, slot = brick coordinates mod lB);
   // NULL: the head evaluates them itself
   const double* lbox;
   long lB3;
@@ -876,7 +876,7 @@ __device__ __forceinline__ void head_source(const RhsArgs& a, const PointRef& pr
     double ue[20], re[20];
     if (layer) {
       if constexpr (HOLE == HOLE_BOXED && MOVE) {
-        // a moving :damped hole's box (k_brick_layer): background_state_rate's
+        // a moving :damped hole's box (k_brick_moving): background_state_rate's
         // values, its d_t Pi formed here from Pi at t +- delta as it forms it
 #pragma clang fp contract(off)
         const double* lb = a.lbox + pr.lslot;
