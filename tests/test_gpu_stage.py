@@ -110,3 +110,52 @@ def test_a_moving_holes_frame_and_layer_match_the_oracle(tgh, chart, axis, q, N,
         err = float(np.max(np.abs(v.cpu().numpy() - ref)))
         print(f"flags {flags}: {err:.2e} (bound {2 * step_tol:.2e})")
         assert err <= 2 * step_tol
+
+
+# (gauge, v, q, halfwidth, N, roots, r_0, r_1): spacings that are no power of two,
+# spheres through grid points whose radius a fused multiply-add in their
+# position moves across r_0 (12 to 57 of them) or r_1
+EDGES = [("algebraic", 0.0, 2, 1.6, 10, 4, 0.8, 1.44), (None, 0.0, 4, 1.6, 10, 4, 0.8, 1.52),
+         ("algebraic", 0.0, 4, 1.4, 14, 4, 0.75, 1.25), ("harmonic", 0.0, 2, 1.4, 14, 4, 0.75, 1.25),
+         ("algebraic", 0.3, 4, 1.4, 14, 4, 0.75, 1.25)]
+
+
+@pytest.mark.parametrize("gauge,v,q,half,N,roots,r0,r1", EDGES)
+def test_points_on_the_layers_spheres_are_sorted_as_the_oracle_sorts_them(tgh, gauge, v, q, half, N, roots, r0, r1):
+    """A point of the sphere r_0 is the layer's (relaxed at rho_max) or the
+    core's (frozen): every form decides as the oracle does, and the layer's
+    targets are there for the points that it calls the layer's."""
+    torch = torch_cuda()
+    import oracle_lib
+    import tgh_desc
+    args = dict(M=1.0, a=0.5, v=v, halfwidth=half, r_0=r0, r_1=r1, rho_max=4.0)
+    case = (tgh.harmonic_kerr_case(**args) if gauge == "harmonic" else tgh.kerr_schild_case(gauge_source=gauge, **args))
+    p = tgh.GHProblem(tgh.gh_forest(None, case, N=N, roots=roots), case, q=q)
+    orc = oracle_lib.OracleProblem(tgh_desc.TghDesc.from_buffer_copy(bytes(p.desc)))
+    h = 2 * half / (N * roots)
+    u0 = orc.fill_exact(0.0)
+    orc.add_noise(u0, 0x57A70, 1e-4)
+    dt = h / 16
+    rhs_tol, step_tol = bound(u0, h, dt)
+    u, du = torch.from_numpy(u0).cuda(), torch.empty(len(u0), dtype=torch.float64, device="cuda")
+    tgh.gh_rhs(du, u, p, 0.0)
+    err = float(np.max(np.abs(du.cpu().numpy() - orc.gh_rhs(u0, 0.0, 8))))
+    print(f"rhs: {err:.2e} (bound {rhs_tol:.2e})")
+    assert err <= rhs_tol
+    ref = u0.copy()
+    orc.rk4_step(ref, 0.0, dt, 8)
+    for flags in (0, tgh.TGH_RK4_SPLIT, tgh.TGH_RK4_BLOCKS | tgh.TGH_RK4_SPLIT, tgh.TGH_RK4_BLOCKS | tgh.TGH_RK4_FUSED):
+        w = torch.from_numpy(u0).cuda()
+        tgh._check(tgh._load().tgh_rk4(p.ptr, C.c_void_p(w.data_ptr()), 0.0, dt, 1, flags))
+        err = float(np.max(np.abs(w.cpu().numpy() - ref)))
+        print(f"flags {flags}: {err:.2e} (bound {step_tol:.2e})")
+        assert err <= step_tol
+    if v == 0.0:
+        rng = np.random.default_rng(9)
+        lam, du_dir, pd = rng.standard_normal(u0.shape), rng.standard_normal(u0.shape), rng.standard_normal(5)
+        _, dF = oracle_lib.gh_rhs_jvp(orc, u0, du_dir, 0.0, pd)
+        ub, thb = tgh.vjp_rhs(p, torch.from_numpy(u0).cuda(), 0.0, torch.from_numpy(lam).cuda())
+        lhs, rhs = float(np.dot(lam, dF)), float(np.dot(ub.cpu().numpy(), du_dir) + np.dot(thb, pd))
+        scale = float(np.abs(lam * dF).sum())
+        print(f"vjp: |diff| / scale = {abs(lhs - rhs) / scale:.2e}")
+        assert abs(lhs - rhs) <= 1e-12 * scale

@@ -374,7 +374,7 @@ __device__ __forceinline__ void adj_point(const AdjPointArgs& a, int x, int y, i
   const CaseP& c = a.c;
   const long off = brick_index(k, x, y, z), fs = k.fs;
   const int sy = (int)k.py, sz = (int)k.pz;
-  const double xp[3] = {k.lo[0] + (double)x * k.h, k.lo[1] + (double)y * k.h, k.lo[2] + (double)z * k.h};
+  const double xp[3] = {grid_coord(k.lo[0], x, k.h), grid_coord(k.lo[1], y, k.h), grid_coord(k.lo[2], z, k.h)};
   double* __restrict__ F = a.F + off;
   double r = 0.0;
   if (frozen_core<HOLE>(c, a.t, xp, r)) {

@@ -126,6 +126,16 @@ TGH_HD void position(const Geom& g, int b, int i, int j, int k, double x[3]) {
   x[2] = g.lo[2] + (double)(B[2] * g.N + k) * h;
 }
 
+// The coordinate of grid index n, rounded as the oracle rounds it. Whoever
+// decides whether a point lies in the core, in the layer or outside takes its
+// position from here: on a spacing that is not a power of two a fused
+// multiply-add moves points across the spheres r_0 and r_1, and the layer box
+// holds targets only for the points that its own kernels found inside.
+TGH_HD double grid_coord(double lo, int n, double h) {
+#pragma clang fp contract(off)
+  return lo + (double)n * h;
+}
+
 // center_at (src/interior.jl:86-93): c(t) = c0 + v t. It and the radius and
 // the core rule below round as the oracle does (no contraction): the moving
 // core's target rate is a difference over 2 delta of values taken at them.
@@ -1279,7 +1289,13 @@ __device__ __forceinline__ bool block_point_at(const RhsArgs& a, const double* _
   pr.sv = sv;
   pr.s2 = S;
   pr.s3 = S * S;
-  position(g, b, i, j, k, pr.x);
+  {
+    const int* Bc = g.bcoord + 3 * b;
+    const double h = block_h(g, b);
+    pr.x[0] = grid_coord(g.lo[0], Bc[0] * g.N + i, h);
+    pr.x[1] = grid_coord(g.lo[1], Bc[1] * g.N + j, h);
+    pr.x[2] = grid_coord(g.lo[2], Bc[2] * g.N + k, h);
+  }
   pr.ih = block_inv_h(g, b);
   pr.ti0 = (long)b * 40 * psz + p;
   pr.si0 = (long)b * 20 * psz + p;
@@ -2473,9 +2489,9 @@ __device__ __forceinline__ void brick_head_at(const RhsArgs& a, const Brick& k, 
   pr.sv = k.fs;
   pr.s2 = (int)k.py;
   pr.s3 = (int)k.pz;
-  pr.x[0] = k.lo[0] + (double)(x + k.gx0[0]) * k.h;
-  pr.x[1] = k.lo[1] + (double)(y + k.gx0[1]) * k.h;
-  pr.x[2] = k.lo[2] + (double)(z + k.gx0[2]) * k.h;
+  pr.x[0] = grid_coord(k.lo[0], x + k.gx0[0], k.h);
+  pr.x[1] = grid_coord(k.lo[1], y + k.gx0[1], k.h);
+  pr.x[2] = grid_coord(k.lo[2], z + k.gx0[2], k.h);
   pr.si0 = off;
   pr.ssv = k.fs;
   pr.wi0 = off;
@@ -2833,7 +2849,7 @@ __device__ __forceinline__ bool layer_point(const LayerArgs& a, long s, int p[3]
   for (int d = 0; d < 3; ++d) {
     p[d] = (int)floor((cc[d] - c.r1 - k.lo[d]) * k.inv_h) - 1 + l[d];
     if (p[d] < 0 || p[d] >= k.n[d]) return false;
-    x[d] = k.lo[d] + (double)p[d] * k.h;
+    x[d] = grid_coord(k.lo[d], p[d], k.h);
   }
   double r;
   core = frozen_core<1>(c, a.t, x, r);

@@ -445,8 +445,8 @@ __device__ __forceinline__ void stage_tile(const RhsArgs& a, const Brick& k, con
 
   // ---- the head ----
   if (valid) {
-    const double xp[3] = {k.lo[0] + (double)(x + k.gx0[0]) * k.h, k.lo[1] + (double)(y + k.gx0[1]) * k.h,
-                          k.lo[2] + (double)(z + k.gx0[2]) * k.h};
+    const double xp[3] = {grid_coord(k.lo[0], x + k.gx0[0], k.h), grid_coord(k.lo[1], y + k.gx0[1], k.h),
+                          grid_coord(k.lo[2], z + k.gx0[2], k.h)};
     long lslot = 0;
     if (HOLE && a.lbox)
       lslot = layer_slot((x + k.gx0[0]) << k.lsh, (y + k.gx0[1]) << k.lsh, (z + k.gx0[2]) << k.lsh, a.lB);
