@@ -1,0 +1,98 @@
+"""The interior layer's targets on the device where they are not a hole's at
+rest: an interior on a background that changes with time (the gauge wave), in
+the right-hand side verb, every form of the stepper, a batch, the
+vector-Jacobian product and the adjoint, against the oracle, which evaluates
+each target at the time of the call."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle_lib
+import tgh_desc as TD
+from test_gpu_stage import bound, torch_cuda
+
+pytestmark = pytest.mark.gpu
+
+
+def wave_with_a_layer(tgh, N, roots, q, a=0.05):
+    case = tgh.with_interior(tgh.gauge_wave_case(A=a, eps_ko=0.5, gamma0=1.0, gamma2=-0.5),
+                             tgh.Interior(center=(0.5, 0.5, 0.5), r_0=0.1, r_1=0.4, rho_max=4.0))
+    p = tgh.GHProblem(tgh.gh_forest(None, case, N=N, roots=roots), case, q=q)
+    return p, oracle_lib.OracleProblem(TD.TghDesc.from_buffer_copy(bytes(p.desc))), 1.0 / (N * roots)
+
+
+@pytest.mark.parametrize("N,roots,q", [(8, 4, 2), (14, 2, 4)])
+def test_a_layer_on_a_time_dependent_background_follows_it(tgh, N, roots, q):
+    torch = torch_cuda()
+    p, orc, h = wave_with_a_layer(tgh, N, roots, q)
+    t = 0.1
+    u0 = orc.fill_exact(t)
+    orc.add_noise(u0, 0x1A7E5, 1e-4)
+    dt = h / 8
+    rhs_tol, step_tol = bound(u0, h, dt)
+    du = torch.empty(len(u0), dtype=torch.float64, device="cuda")
+    for s in (t, 0.0, 3 * t):  # the verb's target is the call's, whatever came before
+        tgh.gh_rhs(du, torch.from_numpy(u0).cuda(), p, s)
+        err = float(np.max(np.abs(du.cpu().numpy() - orc.gh_rhs(u0, s, 8))))
+        print(f"rhs at t = {s}: {err:.2e} (bound {rhs_tol:.2e})")
+        assert err <= rhs_tol
+    ref = u0.copy()
+    for n in range(2):
+        orc.rk4_step(ref, t + n * dt, dt, 8)
+    B, S, F, G = tgh.TGH_RK4_BLOCKS, tgh.TGH_RK4_SPLIT, tgh.TGH_RK4_FUSED, tgh.TGH_RK4_GRAPH
+    for flags in (0, G, S, F, B, B | G, B | F):
+        v = torch.from_numpy(u0).cuda()
+        tgh._check(tgh._load().tgh_rk4(p.ptr, C.c_void_p(v.data_ptr()), t, dt, 2, flags))
+        err = float(np.max(np.abs(v.cpu().numpy() - ref)))
+        print(f"flags {flags}: {err:.2e} (bound {2 * step_tol:.2e})")
+        assert err <= 2 * step_tol
+    # the transposed right-hand side: 1e-12 of the terms' magnitudes, as in test_gpu_adjoint.py
+    rng = np.random.default_rng(10)
+    lam, dirn, pd = rng.standard_normal(u0.shape), rng.standard_normal(u0.shape), rng.standard_normal(5)
+    _, dF = oracle_lib.gh_rhs_jvp(orc, u0, dirn, t, pd)
+    ub, thb = tgh.vjp_rhs(p, torch.from_numpy(u0).cuda(), t, torch.from_numpy(lam).cuda())
+    lhs, rhs = float(np.dot(lam, dF)), float(np.dot(ub.cpu().numpy(), dirn) + np.dot(thb, pd))
+    scale = float(np.abs(lam * dF).sum())
+    print(f"vjp: |diff| / scale = {abs(lhs - rhs) / scale:.2e}")
+    assert abs(lhs - rhs) <= 1e-12 * scale
+    # rho_max's and rho_ramp's share alone, sums of lambda (u - u_exact): u and
+    # u_exact (a sine, a few roundings of 1) cancel to the noise of 1e-4, so
+    # each term is good to some 10 eps / 1e-4 = 2e-11 of itself
+    pd[:3] = 0.0
+    _, dF = oracle_lib.gh_rhs_jvp(orc, u0, np.zeros_like(u0), t, pd)
+    err, scale = abs(float(np.dot(lam, dF)) - float(np.dot(thb, pd))), float(np.abs(lam * dF).sum())
+    print(f"vjp, the layer's parameters: |diff| / scale = {err / scale:.2e}")
+    assert err <= 2e-11 * scale
+
+
+def test_the_adjoint_reads_each_stages_own_target(tgh):
+    """Three steps, a checkpoint every two: dJ/d(gamma2, rho_max, rho_ramp)
+    against the oracle's tangent linear model, as in test_gpu_adjoint.py."""
+    torch = torch_cuda()
+    p, orc, h = wave_with_a_layer(tgh, 8, 4, 2)
+    t0, dt, nsteps = 0.1, h / 8, 3
+    u0 = orc.fill_exact(t0)
+    orc.add_noise(u0, 0x1A7E6, 1e-4)
+    ud = torch.from_numpy(u0.copy()).cuda()
+    J, grad, _ = tgh.adjoint(p, ud, t0, dt, nsteps, every=2)
+    want = np.zeros(5)
+    for k in range(2, 5):
+        pd = np.zeros(5)
+        pd[k] = 1.0
+        u, udot = u0.copy(), np.zeros_like(u0)
+        for n in range(nsteps):
+            oracle_lib.rk4_step_jvp(orc, u, udot, t0 + n * dt, dt, pd)
+        want[k] = oracle_lib.error_tangent(orc, u, udot, t0 + nsteps * dt)
+    l2, _ = orc.error_norms(u, t0 + nsteps * dt)
+    print(f"J {J:.15e} {l2:.15e}; gradient {list(grad[2:])} {list(want[2:])}")
+    assert abs(J - l2) <= 1e-12 * l2
+    for k in range(2, 5):
+        assert abs(grad[k] - want[k]) <= 1e-9 * max(abs(want[k]), 1e-3 * np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_a_batch_of_layers_on_waves_steps_each_as_alone(tgh, graph):
+    from test_gpu_batch import check_batch_equals_alone
+    probs = [wave_with_a_layer(tgh, 8, r, 2, a)[0] for r, a in ((4, 0.05), (5, 0.03))]
+    check_batch_equals_alone(tgh, probs, 2, graph)

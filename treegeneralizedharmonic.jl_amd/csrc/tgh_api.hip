@@ -463,15 +463,20 @@ bool static_background(const CaseP& c) {
   return !c.moving && (kind == BG_MINKOWSKI || kind == BG_KERR_SCHILD || kind == BG_SHIFTED || kind == BG_HARMONIC);
 }
 
-// The layer box (k_brick_moving, k_brick_layer) of a moving :damped hole or of a hole at
-// rest, on the finest level's grid: the layer's bounding box about c(t) with
-// a point of margin each side, whatever t (slots wrap modulo B). Nothing for
-// other cases.
+// The targets of a box at rest, at time t.
 Brick layer_grid(const tgh_problem* p);
+void launch_layer(tgh_problem* p, double t, double toff) {
+  const long B3 = (long)p->layer_B * p->layer_B * p->layer_B;
+  LayerArgs la{layer_grid(p), p->cs, t, p->clock_use, toff, p->Blayer, p->layer_B};
+  hipLaunchKernelGGL(k_brick_layer, dim3((unsigned)((B3 + 255) / 256)), dim3(256), 0, p->stream, la);
+}
+// The layer box (k_brick_moving, k_brick_layer) of a moving :damped hole or of
+// an interior at rest, on the finest level's grid: the layer's bounding box
+// about c(t) with a point of margin each side, whatever t (slots wrap modulo
+// B). Nothing for other cases.
 int ensure_layer_box(tgh_problem* p) {
   if (p->Blayer || p->cs.general || p->cs.interior == INT_NONE || p->cs.interior == INT_PASTED) return TGH_OK;
   const bool moving = p->cs.moving && p->cs.interior == INT_DAMPED;
-  // a hole at rest: its layer's target is the same at every t, so the box is filled once
   const bool rest = !p->cs.moving;
   if (!moving && !rest) return TGH_OK;
   int lmax = 0;
@@ -488,11 +493,11 @@ int ensure_layer_box(tgh_problem* p) {
     if (rest && p->cs.gauge != GAUGE_NONE) return TGH_OK;
     return fail(TGH_EDEVICE, std::string("allocating the layer box: ") + hipGetErrorString(e));
   }
-  p->layer_static = rest;
-  if (rest) {
-    const long B3 = (long)p->layer_B * p->layer_B * p->layer_B;
-    LayerArgs la{layer_grid(p), p->cs, 0.0, nullptr, 0.0, p->Blayer, p->layer_B};
-    hipLaunchKernelGGL(k_brick_layer, dim3((unsigned)((B3 + 255) / 256)), dim3(256), 0, p->stream, la);
+  // a static background's target is the same at every t: filled once (fill_layer
+  // fills the gauge wave's and a moving hole's at each stage's time)
+  p->layer_static = static_background(p->cs);
+  if (p->layer_static) {
+    launch_layer(p, 0.0, 0.0);
     HIP_TRY(hipGetLastError());
   }
   return TGH_OK;
@@ -528,20 +533,27 @@ void launch_moving(tgh_problem* p, double* W, double* W2, double t, double toff)
   }
   if (fb + lb) hipLaunchKernelGGL(k_brick_moving, dim3(fb + lb), dim3(256), 0, p->stream, fa, la, fb);
 }
+// The layer box's targets at a time, unless it is filled once.
+void fill_layer(tgh_problem* p, double t, double toff) {
+  if (!p->Blayer || p->layer_static) return;
+  if (p->cs.moving) launch_moving(p, nullptr, nullptr, t, toff);
+  else launch_layer(p, t, toff);
+}
 // What a stage on the brick reads at its time besides its own values: the
-// frame of its input W, filled unless it is static, and a moving hole's layer
-// box. An RK4 step's second and third stage have the same time: the second
-// fills the third's exact frame too (W2), and nothing that depends on the time
-// alone is filled for the third (again).
+// frame of its input W, filled unless it is static, and the layer box. An RK4
+// step's second and third stage have the same time: the second fills the
+// third's exact frame too (W2), and nothing that depends on the time alone is
+// filled for the third (again).
 void fill_stage(tgh_problem* p, double* W, double* W2, double t, double toff, bool again) {
   const bool exact = frame_exact(p);
   const bool frame = !p->frame_static && !(again && exact);
   if (p->cs.moving) {
     if (frame && !exact) launch_frame(p, W, t, toff);
     if (!again) launch_moving(p, frame && exact ? W : nullptr, W2, t, toff);
-  } else if (frame) {
-    launch_frame(p, W, t, toff, exact ? W2 : nullptr);
+    return;
   }
+  if (frame) launch_frame(p, W, t, toff, exact ? W2 : nullptr);
+  if (!again) fill_layer(p, t, toff);
 }
 // The layer box as a stage's arguments.
 void layer_args(tgh_problem* p, RhsArgs& a) {
@@ -812,7 +824,7 @@ void rk4_block_stage_launches(tgh_problem* p, double t, double dt) {
     RhsArgs a = rhs_args(p, Wc, t_stage[s], nullptr);
     a.clock = p->clock_use;
     a.toff = t_off[s];
-    if (p->Blayer && s != 2) launch_moving(p, nullptr, nullptr, t_stage[s], t_off[s]);  // the third: the second's time
+    if (s != 2) fill_layer(p, t_stage[s], t_off[s]);  // the third: the second's time
     layer_args(p, a);
     launch_stage_block(p, a, StageIO{s + 1, c_acc[s], c_next[s], p->Wus, p->Wus, p->Wacc, nullptr, Wn, 0});
   }
@@ -835,7 +847,7 @@ void rk4_step_launches(tgh_problem* p, double* u, double t, double dt) {
     RhsArgs a = rhs_args(p, Wc, t_stage[s], p->mat.rho ? &p->mat : nullptr);
     a.clock = p->clock_use;
     a.toff = t_off[s];
-    if (p->Blayer && s != 2) launch_moving(p, nullptr, nullptr, t_stage[s], t_off[s]);  // the third: the second's time
+    if (s != 2) fill_layer(p, t_stage[s], t_off[s]);  // the third: the second's time
     layer_args(p, a);
     a.us = u;
     a.acc = p->acc;
@@ -1346,10 +1358,10 @@ int tgh_rhs(tgh_problem* p, double* du, double t, const tgh_matter* matter) {
   if (matter && matter->rho && (!matter->S || !matter->Sij))
     return fail(TGH_EINVAL, "a matter adapter needs rho, S and Sij");
   RhsArgs a = rhs_args(p, p->W[0], t, matter);
-  // in tiles, as a stage of the stepper, for vacuum and a hole at rest (whose
-  // layer box is filled once); the other cases, and a box that finds no
-  // memory, one point a thread
+  // in tiles, as a stage of the stepper, for vacuum and an interior at rest;
+  // the other cases, and a layer box that finds no memory, one point a thread
   if (!(matter && matter->rho) && !p->cs.general && !p->cs.moving && ensure_layer_box(p) == TGH_OK && stage_ok(p)) {
+    fill_layer(p, t, 0.0);
     layer_args(p, a);
     launch_stage_block(p, a, StageIO{STAGE_STORE, 0.0, 0.0, nullptr, nullptr, nullptr, nullptr, du, 0});
   } else {
@@ -1898,6 +1910,7 @@ int tgh_vjp_rhs(tgh_problem* p, const double* u, double t, const double* du_bar,
   BrickCopyArgs ca{p->geom, k, u, p->BW[0], p->Bus};
   hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, p->stream, ca);
   if (!p->frame_static) launch_frame(p, p->BW[0], t);
+  fill_layer(p, t, 0.0);
   launch_adj_fold_copies(p, AdjCopiesArgs{p->geom, k, du_bar, p->adjK[0]});
   HIP_TRY(hipMemsetAsync(p->adjTh, 0, sizeof(double) * ADJ_NPAR * adj_runs(k), p->stream));
   launch_adj_point(p, adj_point_args(p, t, p->BW[0], p->adjK[0]));
@@ -1988,6 +2001,7 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
       for (int s = 4; s-- > 0;) {
         double* Wc = slot(4 * j + s);
         if (!p->frame_static) launch_frame(p, Wc, t_stage[s]);
+        fill_layer(p, t_stage[s], 0.0);
         launch_adj_point(p, adj_point_args(p, t_stage[s], Wc, kb));
         launch_adj_gather(p, AdjGatherArgs{k, p->adjF, lam, lacc, kbn, nullptr, cl[s], cy[s], s == 3, s == 0});
         std::swap(kb, kbn);
@@ -2225,7 +2239,10 @@ void batch_step_launches_blocks(tgh_batch* b, double t, double dt) {
   const double t_off[4] = {0.0, dt / 2, dt / 2, dt};
   const double t_stage[4] = {t, t + dt / 2, t + dt / 2, t + dt};
   for (int s = 0; s < 4; ++s) {
-    for (tgh_problem* p : b->probs) launch_fill(p, p->W[s % 2], t_stage[s], t_off[s]);
+    for (tgh_problem* p : b->probs) {
+      launch_fill(p, p->W[s % 2], t_stage[s], t_off[s]);
+      if (b->lds && s != 2) fill_layer(p, t_stage[s], t_off[s]);
+    }
     const BatchEntry* tab = b->d_tab + s * n;
     if (b->lds) {
       launch_batch_stage(b, tab);

@@ -2855,8 +2855,9 @@ __device__ __forceinline__ bool layer_point(const LayerArgs& a, long s, int p[3]
   core = frozen_core<1>(c, a.t, x, r);
   return core || r < c.r1;
 }
-// A hole at rest: the layer's target, once (the core's rates are zero).
+// An interior at rest: the layer's target (the core's rates are zero).
 __global__ __launch_bounds__(256) void k_brick_layer(LayerArgs a) {
+  a.t = stage_time(a.t, a.clock, a.toff);
   const long B3 = (long)a.B * a.B * a.B;
   const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= B3) return;
