@@ -96,3 +96,44 @@ def test_a_batch_of_layers_on_waves_steps_each_as_alone(tgh, graph):
     from test_gpu_batch import check_batch_equals_alone
     probs = [wave_with_a_layer(tgh, 8, r, 2, a)[0] for r, a in ((4, 0.05), (5, 0.03))]
     check_batch_equals_alone(tgh, probs, 2, graph)
+
+
+def moving_hole(tgh, chart, variant, a, roots, v, N=14):
+    half = roots * N / 32  # h = 1/16
+    args = dict(M=1.0, a=a, v=v, x0=0.1, axis=2, halfwidth=half, r_0=0.35, r_1=0.9, interior=variant)
+    case = (tgh.harmonic_kerr_case(**args) if chart == "harmonic"
+            else tgh.kerr_schild_case(gauge_source="algebraic", **args))
+    return tgh.GHProblem(tgh.gh_forest(None, case, N=N, roots=roots), case, q=4)
+
+
+@pytest.mark.parametrize("chart", ["kerr_schild", "harmonic"])
+def test_a_moving_frozen_hole_matches_the_oracle_in_every_form(tgh, chart):
+    """A :frozen layer has no target and a :frozen core no rate."""
+    torch = torch_cuda()
+    p = moving_hole(tgh, chart, "frozen", 0.3, 4, 0.3)
+    orc = oracle_lib.OracleProblem(TD.TghDesc.from_buffer_copy(bytes(p.desc)))
+    h, t = 1.0 / 16, 0.1
+    u0 = orc.fill_exact(t)
+    orc.add_noise(u0, 0x1A7E7, 1e-6)
+    dt = h / 16
+    _, step_tol = bound(u0, h, dt)
+    ref = u0.copy()
+    for n in range(2):
+        orc.rk4_step(ref, t + n * dt, dt, 8)
+    B, S, F, G = tgh.TGH_RK4_BLOCKS, tgh.TGH_RK4_SPLIT, tgh.TGH_RK4_FUSED, tgh.TGH_RK4_GRAPH
+    for flags in (0, G, S, F, B, B | F):
+        u = torch.from_numpy(u0).cuda()
+        tgh._check(tgh._load().tgh_rk4(p.ptr, C.c_void_p(u.data_ptr()), t, dt, 2, flags))
+        err = float(np.max(np.abs(u.cpu().numpy() - ref)))
+        print(f"flags {flags}: {err:.2e} (bound {2 * step_tol:.2e})")
+        assert err <= 2 * step_tol
+
+
+@pytest.mark.parametrize("chart", ["kerr_schild", "harmonic"])
+@pytest.mark.parametrize("variants", [("frozen", "frozen"), ("frozen", "damped")])
+def test_a_batch_takes_moving_frozen_holes(tgh, chart, variants):
+    """To an ulp of the state, as test_gpu_batch.py's moving holes."""
+    from test_gpu_batch import check_batch_equals_alone
+    probs = [moving_hole(tgh, chart, w, a, roots, v)
+             for w, a, roots, v in zip(variants, (0.0, 0.3), (3, 4), (0.3, -0.2))]
+    check_batch_equals_alone(tgh, probs, 2, True, roundoff=True)

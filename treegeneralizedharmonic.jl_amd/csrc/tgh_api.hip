@@ -473,17 +473,16 @@ void launch_layer(tgh_problem* p, double t, double toff) {
 // The layer box (k_brick_moving, k_brick_layer) of a moving :damped hole or of
 // an interior at rest, on the finest level's grid: the layer's bounding box
 // about c(t) with a point of margin each side, whatever t (slots wrap modulo
-// B). Nothing for other cases.
+// B). A :frozen layer has no target (its rate rho is zero): its box is one
+// slot of zeros, which every point reads. Nothing for other cases.
 int ensure_layer_box(tgh_problem* p) {
   if (p->Blayer || p->cs.general || p->cs.interior == INT_NONE || p->cs.interior == INT_PASTED) return TGH_OK;
-  const bool moving = p->cs.moving && p->cs.interior == INT_DAMPED;
-  const bool rest = !p->cs.moving;
-  if (!moving && !rest) return TGH_OK;
+  const bool frozen = p->cs.interior == INT_FROZEN, rest = !p->cs.moving;
   int lmax = 0;
   for (int l : p->level_host) lmax = std::max(lmax, l);
   p->layer_lmax = lmax;
-  p->layer_B = 2 * (int)std::ceil(p->cs.r1 * p->geom.inv_h * (double)(1 << lmax)) + 4;
-  const size_t lb = sizeof(double) * (moving ? LAYER_FIELDS : 20) * (size_t)p->layer_B * p->layer_B * p->layer_B;
+  p->layer_B = frozen ? 1 : 2 * (int)std::ceil(p->cs.r1 * p->geom.inv_h * (double)(1 << lmax)) + 4;
+  const size_t lb = sizeof(double) * (rest ? 20 : LAYER_FIELDS) * (size_t)p->layer_B * p->layer_B * p->layer_B;
   hipError_t e = hipMalloc(&p->Blayer, lb);
   if (e != hipSuccess) {
     p->Blayer = nullptr;
@@ -495,8 +494,10 @@ int ensure_layer_box(tgh_problem* p) {
   }
   // a static background's target is the same at every t: filled once (fill_layer
   // fills the gauge wave's and a moving hole's at each stage's time)
-  p->layer_static = static_background(p->cs);
-  if (p->layer_static) {
+  p->layer_static = frozen || static_background(p->cs);
+  if (frozen) {
+    HIP_TRY(hipMemsetAsync(p->Blayer, 0, lb, p->stream));
+  } else if (p->layer_static) {
     launch_layer(p, 0.0, 0.0);
     HIP_TRY(hipGetLastError());
   }
