@@ -15,6 +15,7 @@
 
 #include "tgh_forest.hpp"
 #include "tgh_problem.hpp"
+#include "tgh_scratch.hpp"
 #include "tgh_adjoint.hpp"
 #include "tgh_fit.hpp"
 
@@ -33,6 +34,21 @@ int fail(int code, const std::string& msg) {
     if (e_ != hipSuccess)                                                                  \
       return fail(TGH_EDEVICE, std::string(#expr) + ": " + hipGetErrorString(e_));         \
   } while (0)
+
+// Device arrays, cleared, made at their first use on p's stream.
+int ensure_device(tgh_problem* p, std::initializer_list<ScratchArray> arrays, const char* what) {
+  return ensure_arrays(arrays, [&](double** at, size_t bytes) {
+    hipError_t e = hipMalloc(at, bytes);
+    if (e == hipSuccess) {
+      e = hipMemsetAsync(*at, 0, bytes, p->stream);
+      if (e == hipSuccess) return (int)TGH_OK;
+      (void)hipFree(*at);
+    }
+    (void)hipGetLastError();
+    return fail(TGH_EDEVICE, std::string("allocating ") + what + " (" + std::to_string(bytes >> 20) +
+                                 " MiB each): " + hipGetErrorString(e));
+  });
+}
 
 uint64_t morton3(uint32_t x, uint32_t y, uint32_t z) {
   uint64_t k = 0;
@@ -495,13 +511,17 @@ int ensure_layer_box(tgh_problem* p) {
   // a static background's target is the same at every t: filled once (fill_layer
   // fills the gauge wave's and a moving hole's at each stage's time)
   p->layer_static = frozen || static_background(p->cs);
+  e = hipSuccess;
   if (frozen) {
-    HIP_TRY(hipMemsetAsync(p->Blayer, 0, lb, p->stream));
+    e = hipMemsetAsync(p->Blayer, 0, lb, p->stream);
   } else if (p->layer_static) {
     launch_layer(p, 0.0, 0.0);
-    HIP_TRY(hipGetLastError());
+    e = hipGetLastError();
   }
-  return TGH_OK;
+  if (e == hipSuccess) return TGH_OK;
+  (void)hipFree(p->Blayer);  // never an unfilled box
+  p->Blayer = nullptr;
+  return fail(TGH_EDEVICE, std::string("filling the layer box: ") + hipGetErrorString(e));
 }
 // The box kernel's view of the finest level's grid (its corner, spacing and
 // closed point counts; the other fields are unused there).
@@ -587,30 +607,23 @@ int ensure_brick(tgh_problem* p) {
   k.pz = k.py * (k.n[1] + 2 * k.G);
   k.fs = k.pz * (k.n[2] + 2 * k.G);
   const size_t bytes = sizeof(double) * 20 * (size_t)k.fs;
-  double** arrs[4] = {&p->BW[0], &p->BW[1], &p->Bus, &p->Bacc};
-  for (double** a : arrs) {
-    hipError_t e = hipMalloc(a, bytes);
-    if (e != hipSuccess)
-      return fail(TGH_EDEVICE, std::string("allocating the stepper's brick arrays (") + std::to_string(bytes >> 20) +
-                                   " MiB each): " + hipGetErrorString(e));
-    HIP_TRY(hipMemsetAsync(*a, 0, bytes, p->stream));
-  }
+  int rc = ensure_device(p, {{&p->BW[0], bytes}, {&p->BW[1], bytes}, {&p->Bus, bytes}, {&p->Bacc, bytes}},
+                         "the stepper's brick arrays");
+  if (rc) return rc;
   const bool static_bg = static_background(p->cs);
   // a wrapped or mirrored frame reads the stage's own values: refilled every stage
   p->frame_static = static_bg && frame_exact(p);
   if (p->frame_static)  // every array is a stage input in one of the forms
-    for (double** a : arrs) launch_frame(p, *a, 0.0);
-  {
-    const int rc = ensure_layer_box(p);
-    if (rc) return rc;
-  }
+    for (double* w : {p->BW[0], p->BW[1], p->Bus, p->Bacc}) launch_frame(p, w, 0.0);
+  rc = ensure_layer_box(p);
+  if (rc) return rc;
   if (p->cs.gauge == GAUGE_SAMPLED) {
-    HIP_TRY(hipMalloc(&p->BH, bytes));
-    HIP_TRY(hipMemsetAsync(p->BH, 0, bytes, p->stream));
+    rc = ensure_device(p, {{&p->BH, bytes}}, "the brick's gauge source");
+    if (rc) return rc;
     BrickSampleArgs sa{k, p->cs, 0.0, p->BH};
     hipLaunchKernelGGL(k_brick_sample, grid_brick(p), dim3(256), 0, p->stream, sa);
   }
-  int rc = sync(p);
+  rc = sync(p);
   if (rc) return rc;
   p->brick_ready = true;
   return TGH_OK;
@@ -800,11 +813,8 @@ bool block_stage_ok(const tgh_problem* p) {
   return !p->has_bounds && p->cs.interior != INT_PASTED && !p->mat.rho && !p->cs.general && stage_ok(p);
 }
 int ensure_block_stage(tgh_problem* p) {
-  if (p->Wus) return TGH_OK;
   const size_t wbytes = sizeof(double) * (size_t)p->work_len;
-  HIP_TRY(hipMalloc(&p->Wus, wbytes));
-  HIP_TRY(hipMalloc(&p->Wacc, wbytes));
-  return TGH_OK;
+  return ensure_device(p, {{&p->Wus, wbytes}, {&p->Wacc, wbytes}}, "the block stepper's work arrays");
 }
 // One RK4 step on the block layout in tiles (form 5): u_n in Wus, the
 // accumulator in Wacc (both in the work layout), the stage input in W[0]
@@ -1711,9 +1721,9 @@ int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int
   const int form = (flags & TGH_RK4_PER_BLOCK) ? 4 : blocks ? (split ? (lds_ok ? 5 : 0) : 1) : (split ? 3 : 2);
   const bool in_brick = form == 2 || form == 3;
   if (in_brick) {
-    if (form == 3 && !p->Bcoef) {
-      HIP_TRY(hipMalloc(&p->Bcoef, sizeof(double) * CF_N * (size_t)p->brick.fs));
-      HIP_TRY(hipMemsetAsync(p->Bcoef, 0, sizeof(double) * CF_N * (size_t)p->brick.fs, p->stream));
+    if (form == 3) {
+      int rc = ensure_device(p, {{&p->Bcoef, sizeof(double) * CF_N * (size_t)p->brick.fs}}, "the split form's coefficients");
+      if (rc) return rc;
     }
     // u_n into the first stage input, and into the stepper's u_n where that is another array
     double* un = brick_un(p, split);
@@ -1848,18 +1858,11 @@ int adj_prepare(tgh_problem* p) {
   if (rc) return rc;
   if (!stage_ok(p)) return fail(TGH_EDEVICE, "allocating the layer's targets");
   const size_t fb = sizeof(double) * (size_t)p->brick.fs;
-  if (!p->adjF) {
-    HIP_TRY(hipMalloc(&p->adjF, AF_N * fb));
-    HIP_TRY(hipMemsetAsync(p->adjF, 0, AF_N * fb, p->stream));  // the frame stays zero
-    for (int i = 0; i < 2; ++i) {
-      HIP_TRY(hipMalloc(&p->adjL[i], 20 * fb));
-      HIP_TRY(hipMemsetAsync(p->adjL[i], 0, 20 * fb, p->stream));
-      HIP_TRY(hipMalloc(&p->adjK[i], 20 * fb));
-      HIP_TRY(hipMemsetAsync(p->adjK[i], 0, 20 * fb, p->stream));
-    }
-    HIP_TRY(hipMalloc(&p->adjTh, sizeof(double) * ADJ_NPAR * adj_runs(p->brick)));
-  }
-  return TGH_OK;
+  // (the frames of adjF, adjL and adjK stay zero)
+  return ensure_device(p, {{&p->adjF, AF_N * fb}, {&p->adjL[0], 20 * fb}, {&p->adjL[1], 20 * fb},
+                           {&p->adjK[0], 20 * fb}, {&p->adjK[1], 20 * fb},
+                           {&p->adjTh, sizeof(double) * ADJ_NPAR * adj_runs(p->brick)}},
+                       "the adjoint's arrays");
 }
 
 AdjPointArgs adj_point_args(tgh_problem* p, double t, const double* W, const double* kb) {
