@@ -348,3 +348,34 @@ def test_limiters_on_a_segment_are_the_vectors_own(tgh, which):
     assert torch.equal(seg2, seg)
     assert torch.equal(u[:n_other], before[:n_other])
     assert torch.equal(u[n_other + n_gh:], before[n_other + n_gh:])
+
+
+def test_a_refused_right_hand_side_launches_nothing(tgh):
+    """gh_rhs! answers a bad argument before it reads the state: with no output
+    array or with matter fields missing, the work array still holds what an
+    earlier prepare! left (every verb synchronises, so a caller may free its
+    state after the error)."""
+    import ctypes as C
+    import torch
+    case = tgh.gauge_wave_case(eps_ko=0.5, gamma0=1.0, gamma2=-0.5)
+    p = tgh.GHProblem(tgh.gh_forest(None, case, N=8, roots=2), case, q=4)
+    L = tgh._load()
+    u, v = p.statevector(), p.statevector()
+    tgh.initial_state(u, p, 0.0)
+    tgh.initial_state(v, p, 0.3)
+    tgh.prepare(p, u, 0.0)
+
+    def work():
+        w = torch.empty(L.tgh_work_length(p.ptr), dtype=torch.float64, device="cuda")
+        tgh._check(L.tgh_copy_work(p.ptr, C.c_void_p(w.data_ptr())))
+        return w
+
+    before = work()
+    du = torch.zeros_like(u)
+    m = tgh.TghMatter(v.data_ptr(), None, None)
+    for out, matter in ((None, None), (du, m)):
+        rc = L.tgh_gh_rhs(p.ptr, None if out is None else C.c_void_p(out.data_ptr()), C.c_void_p(v.data_ptr()), 0.3,
+                          None if matter is None else C.byref(matter))
+        assert rc == tgh.TGH_EINVAL, rc
+        assert torch.equal(work(), before)
+        assert not du.any()

@@ -1361,13 +1361,20 @@ int tgh_prepare(tgh_problem* p, const double* u, double t) {
   return sync(p);
 }
 
-int tgh_rhs(tgh_problem* p, double* du, double t, const tgh_matter* matter) {
+// What a right-hand side refuses, before anything is launched.
+static int check_rhs(const tgh_problem* p, const double* du, const tgh_matter* matter) {
   if (!p || !du) return fail(TGH_EINVAL, "NULL argument");
   if (p->cs.interior == INT_FITTED && !p->cs.tw)
     return fail(TGH_EINVAL, "the :fitted variant reads its target cache, and none is set: call "
                             "tgh_set_target first");
   if (matter && matter->rho && (!matter->S || !matter->Sij))
     return fail(TGH_EINVAL, "a matter adapter needs rho, S and Sij");
+  return TGH_OK;
+}
+
+int tgh_rhs(tgh_problem* p, double* du, double t, const tgh_matter* matter) {
+  const int rc = check_rhs(p, du, matter);
+  if (rc) return rc;
   RhsArgs a = rhs_args(p, p->W[0], t, matter);
   // in tiles, as a stage of the stepper, for vacuum and an interior at rest;
   // the other cases, and a layer box that finds no memory, one point a thread
@@ -1383,7 +1390,9 @@ int tgh_rhs(tgh_problem* p, double* du, double t, const tgh_matter* matter) {
 }
 
 int tgh_gh_rhs(tgh_problem* p, double* du, const double* u, double t, const tgh_matter* matter) {
-  if (!p || !u) return fail(TGH_EINVAL, "NULL argument");
+  if (!u) return fail(TGH_EINVAL, "NULL argument");
+  const int rc = check_rhs(p, du, matter);
+  if (rc) return rc;
   launch_prepare(p, u, p->W[0], t);
   return tgh_rhs(p, du, t, matter);
 }
