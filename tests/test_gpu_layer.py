@@ -137,3 +137,80 @@ def test_a_batch_takes_moving_frozen_holes(tgh, chart, variants):
     probs = [moving_hole(tgh, chart, w, a, roots, v)
              for w, a, roots, v in zip(variants, (0.0, 0.3), (3, 4), (0.3, -0.2))]
     check_batch_equals_alone(tgh, probs, 2, True, roundoff=True)
+
+
+def against_the_oracle(tgh, p, orc, h, t, seed, forms):
+    torch = torch_cuda()
+    u0 = orc.fill_exact(t)
+    orc.add_noise(u0, seed, 1e-6)
+    dt = h / 16
+    rhs_tol, step_tol = bound(u0, h, dt)
+    du = torch.empty(len(u0), dtype=torch.float64, device="cuda")
+    tgh.gh_rhs(du, torch.from_numpy(u0).cuda(), p, t)
+    err = float(np.max(np.abs(du.cpu().numpy() - orc.gh_rhs(u0, t, 8))))
+    print(f"rhs: {err:.2e} (bound {rhs_tol:.2e})")
+    assert err <= rhs_tol
+    ref = u0.copy()
+    orc.rk4_step(ref, t, dt, 8)
+    for flags in forms:
+        u = torch.from_numpy(u0).cuda()
+        tgh._check(tgh._load().tgh_rk4(p.ptr, C.c_void_p(u.data_ptr()), t, dt, 1, flags))
+        err = float(np.max(np.abs(u.cpu().numpy() - ref)))
+        print(f"flags {flags}: {err:.2e} (bound {step_tol:.2e})")
+        assert err <= step_tol
+    return u0
+
+
+def test_a_mesh_inside_a_huge_layer_steps_batches_and_differentiates(tgh):
+    """The layer's targets take no more room than the mesh: a cube about r_1 =
+    4000 M at h = M/16 would hold 2e15 points."""
+    torch = torch_cuda()
+
+    def problem(lo):
+        case = tgh.GHCase(None, tgh.KerrSchild(1.0, 0.5), box=[(lo, lo + 1.0)] * 3, periodic=(False,) * 3, eps_ko=0.5,
+                          gamma0=1.0, gamma2=0.1, interior=tgh.Interior(r_0=0.8, r_1=4000.0, rho_max=4.0),
+                          gauge_source="algebraic")
+        return tgh.GHProblem(tgh.gh_forest(None, case, N=8, roots=2), case, q=2)
+
+    p, q = problem(1.0), problem(2.0)
+    orc = oracle_lib.OracleProblem(TD.TghDesc.from_buffer_copy(bytes(p.desc)))
+    B, S, F = tgh.TGH_RK4_BLOCKS, tgh.TGH_RK4_SPLIT, tgh.TGH_RK4_FUSED
+    u0 = against_the_oracle(tgh, p, orc, 1.0 / 16, 0.0, 0x1A7E8, (0, S, F, B))
+    us = []
+    for x in (p, q):
+        us.append(x.statevector())
+        tgh.initial_state(us[-1], x, 0.0)
+    alone, dt = [u.clone() for u in us], 1.0 / 256
+    tgh.gh_solve_batch(tgh.GHBatch([p, q]), us, (0.0, 2 * dt), dt=dt, graph=True)
+    for x, u, v in zip((p, q), us, alone):
+        tgh.gh_solve(x, v, (0.0, 2 * dt), dt=dt)
+        assert torch.isfinite(u).all() and torch.equal(u, v)
+    rng = np.random.default_rng(11)
+    lam, dirn, pd = rng.standard_normal(u0.shape), rng.standard_normal(u0.shape), rng.standard_normal(5)
+    _, dF = oracle_lib.gh_rhs_jvp(orc, u0, dirn, 0.0, pd)
+    ub, thb = tgh.vjp_rhs(p, torch.from_numpy(u0).cuda(), 0.0, torch.from_numpy(lam).cuda())
+    lhs, rhs = float(np.dot(lam, dF)), float(np.dot(ub.cpu().numpy(), dirn) + np.dot(thb, pd))
+    assert abs(lhs - rhs) <= 1e-12 * float(np.abs(lam * dF).sum())
+
+
+@pytest.mark.parametrize("axis,x0", [(1, 0.3), (3, -0.3)])
+def test_a_moving_layer_that_leaves_the_mesh(tgh, axis, x0):
+    """25 points an axis, a layer 33 across that reaches over the mesh's face."""
+    case = tgh.harmonic_kerr_case(M=1.0, a=0.3, v=0.3, x0=x0, axis=axis, halfwidth=0.75, r_0=0.35, r_1=0.9)
+    p = tgh.GHProblem(tgh.gh_forest(None, case, N=12, roots=2), case, q=2)
+    orc = oracle_lib.OracleProblem(TD.TghDesc.from_buffer_copy(bytes(p.desc)))
+    against_the_oracle(tgh, p, orc, 1.0 / 16, 0.1, 0x1A7E9, (0, tgh.TGH_RK4_SPLIT, tgh.TGH_RK4_BLOCKS))
+
+
+@pytest.mark.parametrize("center", [(2.5, 2.5, 2.5), (0.9, 0.0, 0.0)])
+def test_levels_away_from_the_layer_and_across_it(tgh, center):
+    """The box is on the finest level that meets the layer: the mesh's own
+    spacing where the finer levels lie elsewhere, theirs where a part of the
+    layer is refined and a part is not."""
+    case = tgh.kerr_schild_case(M=1.0, a=0.5, halfwidth=4.0, r_0=0.7, r_1=1.5, gauge_source="algebraic")
+    f = tgh.hole_forest(None, case, N=8, roots=8, center=center, radii=[0.9, 0.45])
+    p = tgh.GHProblem(f, case, q=2, ops=tgh.Operators(prolongation=4))
+    assert max(int(lf[0]) for lf in f.leaves) == 2
+    orc = oracle_lib.OracleProblem(TD.TghDesc.from_buffer_copy(bytes(p.desc)), leaves=[tuple(lf) for lf in f.leaves],
+                                   prolongation=4)
+    against_the_oracle(tgh, p, orc, 1.0 / 32, 0.0, 0x1A7EA, (0, tgh.TGH_RK4_FUSED, tgh.TGH_RK4_GRAPH))

@@ -489,15 +489,32 @@ void launch_layer(tgh_problem* p, double t, double toff) {
 // The layer box (k_brick_moving, k_brick_layer) of a moving :damped hole or of
 // an interior at rest, on the finest level's grid: the layer's bounding box
 // about c(t) with a point of margin each side, whatever t (slots wrap modulo
-// B). A :frozen layer has no target (its rate rho is zero): its box is one
-// slot of zeros, which every point reads. Nothing for other cases.
+// B), but no wider than the mesh's longest axis. A :frozen layer has no target (its rate rho
+// is zero): its box is one slot of zeros, which every point reads. Nothing for
+// other cases. At rest the grid is the finest level's among the blocks that
+// meet the layer: levels elsewhere do not make its box larger.
+// The one-kernel stage on the brick needs 20 fields of the layer's cube, where
+// the split form's two kernels need 25 of the whole brick.
 int ensure_layer_box(tgh_problem* p) {
   if (p->Blayer || p->cs.general || p->cs.interior == INT_NONE || p->cs.interior == INT_PASTED) return TGH_OK;
   const bool frozen = p->cs.interior == INT_FROZEN, rest = !p->cs.moving;
+  const Geom& g = p->geom;
   int lmax = 0;
-  for (int l : p->level_host) lmax = std::max(lmax, l);
+  for (size_t b = 0; b < p->level_host.size(); ++b) {
+    // the block's distance from the centre, a spacing short
+    const double h = g.h / (double)(1 << p->level_host[b]);
+    double d2 = 0.0;
+    for (int d = 0; d < 3 && rest; ++d) {
+      const double a = g.lo[d] + (double)p->bcoord_host[3 * b + d] * g.N * h - h - p->cs.center[d];
+      const double gap = std::max({a, -(a + (g.N + 2) * h), 0.0});
+      d2 += gap * gap;
+    }
+    if (d2 <= p->cs.r1 * p->cs.r1) lmax = std::max(lmax, p->level_host[b]);
+  }
   p->layer_lmax = lmax;
-  p->layer_B = frozen ? 1 : 2 * (int)std::ceil(p->cs.r1 * p->geom.inv_h * (double)(1 << lmax)) + 4;
+  const Brick mesh = layer_grid(p);
+  const double across = 2.0 * std::ceil(p->cs.r1 * mesh.inv_h) + 4.0;
+  p->layer_B = frozen ? 1 : (int)std::min(across, (double)std::max({mesh.n[0], mesh.n[1], mesh.n[2]}));
   const size_t lb = sizeof(double) * (rest ? 20 : LAYER_FIELDS) * (size_t)p->layer_B * p->layer_B * p->layer_B;
   hipError_t e = hipMalloc(&p->Blayer, lb);
   if (e != hipSuccess) {

@@ -690,8 +690,8 @@ struct RhsArgs {
   const double* lbox;
   long lB3;
   int lB;
-  int lLmax;  // the box's grid: the finest level's (a block point of level L is
-              // at index (B N + i) 2^(lLmax - L) on it)
+  int lLmax;  // the box's grid: the finest level's that meets the layer (a block
+              // point of level L is at index (B N + i) 2^(lLmax - L) on it)
 };
 // The layer box's slot of brick point (x, y, z).
 TGH_HD long layer_slot(int x, int y, int z, int B) {
@@ -1310,7 +1310,7 @@ __device__ __forceinline__ bool block_point_at(const RhsArgs& a, const double* _
   pr.lslot = 0;
   if (a.lbox) {
     const int* Bc = g.bcoord + 3 * b;
-    const int sh = a.lLmax - block_level(g, b);
+    const int sh = max(a.lLmax - block_level(g, b), 0);  // finer blocks do not meet the layer
     pr.lslot = layer_slot((Bc[0] * g.N + i) << sh, (Bc[1] * g.N + j) << sh, (Bc[2] * g.N + k) << sh, a.lB);
   }
   pidx = (long)b * psz + p;
@@ -2407,7 +2407,7 @@ struct Brick {
   // point (x, y, z) is at lo + (x + gx0) h: 0 for the brick; a block's first
   // index (B N) when a block's work array is run as a brick, so that positions
   // round as the block layout's do; lsh: its layer-box slot's shift to the
-  // finest level's grid
+  // box's grid
   int gx0[3];
   int lsh;
 };
@@ -2734,7 +2734,7 @@ struct BatchEntry {
   TGH_GLOBAL double* y2;
   TGH_GLOBAL double* Wn;  // the next stage's input
   int wg0;    // first logical workgroup of the launch
-  int lLmax;  // the block layout's tiles: the problem's finest level
+  int lLmax;  // the block layout's tiles: the layer box's level
 };
 __device__ __forceinline__ int batch_find(const BatchEntry* __restrict__ tab, int n, int L) {
   int p = 0;
@@ -2742,8 +2742,7 @@ __device__ __forceinline__ int batch_find(const BatchEntry* __restrict__ tab, in
   return p;
 }
 // Block b's work array as a brick of P^3 points (strides S, S^2, S^3 per
-// variable, G ghosts) at index offset B N; lLmax the finest level (the layer
-// box's grid).
+// variable, G ghosts) at index offset B N; lLmax the layer box's level.
 __device__ __forceinline__ Brick block_brick(const Geom& g, int b, int lLmax) {
   Brick k;
   const int* B = g.bcoord + 3 * b;
@@ -2764,7 +2763,7 @@ __device__ __forceinline__ Brick block_brick(const Geom& g, int b, int lLmax) {
   k.fs = (long)g.S * g.S * g.S;
   k.h = block_h(g, b);
   k.inv_h = block_inv_h(g, b);
-  k.lsh = lLmax - block_level(g, b);
+  k.lsh = max(lLmax - block_level(g, b), 0);  // finer blocks do not meet the layer
   return k;
 }
 // One RK4 stage of a batch on the block layout: the fused kernel over every
@@ -2847,8 +2846,9 @@ __device__ __forceinline__ bool layer_point(const LayerArgs& a, long s, int p[3]
   center_at(c, a.t, cc);
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    p[d] = (int)floor((cc[d] - c.r1 - k.lo[d]) * k.inv_h) - 1 + l[d];
-    if (p[d] < 0 || p[d] >= k.n[d]) return false;
+    // from the layer's corner, or the mesh's
+    p[d] = (int)fmin(fmax(floor((cc[d] - c.r1 - k.lo[d]) * k.inv_h) - 1.0, 0.0), (double)k.n[d]) + l[d];
+    if (p[d] >= k.n[d]) return false;
     x[d] = grid_coord(k.lo[d], p[d], k.h);
   }
   double r;

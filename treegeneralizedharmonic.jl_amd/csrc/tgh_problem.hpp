@@ -71,7 +71,7 @@ struct tgh_problem {
   double* Bcoef = nullptr;            // the split form's coefficients (CF_N brick fields)
   double* Blayer = nullptr;           // a hole's layer box (LAYER_FIELDS x layer_B^3 moving, 20 x layer_B^3 at rest)
   int layer_B = 0;
-  int layer_lmax = 0;                 // the finest level, whose grid the box is on
+  int layer_lmax = 0;                 // the level whose grid the box is on: the finest that meets the layer
   bool layer_static = false;          // filled once (a static background's)
   // the block layout's tiled form: u_n and the accumulator in the work layout
   // during a step (allocated at its first use)
