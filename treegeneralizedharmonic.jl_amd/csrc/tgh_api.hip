@@ -1910,24 +1910,9 @@ int adj_theta(tgh_problem* p, double* out) {
 
 // The stage inputs of one step from u_n = Y[0]: Y[1 .. 3], and u_{n+1} in Y[4].
 void brick_step_slots(tgh_problem* p, double* const Y[5], double t, double dt) {
-  const double c_acc[4] = {dt / 6, dt / 3, dt / 3, dt / 6};
-  const double c_next[4] = {dt / 2, dt / 2, dt, 0.0};
   const double t_stage[4] = {t, t + dt / 2, t + dt / 2, t + dt};
-  const bool split = !stage_ok(p);
-  for (int s = 0; s < 4; ++s) {
-    RhsArgs a = brick_stage_args(p, Y[s], t_stage[s], 0.0);
-    if (!split) {
-      launch_stage(p, a, stage_io(Y, Y[s + 1], s, dt));
-      continue;
-    }
-    a.us = p->Bus;
-    a.acc = p->Bacc;
-    a.Wn = Y[s + 1];
-    a.cacc = c_acc[s];
-    a.cnext = c_next[s];
-    a.stage = s + 1;
-    launch_split(p, a);
-  }
+  for (int s = 0; s < 4; ++s)
+    launch_stage(p, brick_stage_args(p, Y[s], t_stage[s], 0.0), stage_io(Y, Y[s + 1], s, dt));
 }
 
 }  // namespace
@@ -1937,7 +1922,7 @@ int tgh_vjp_rhs(tgh_problem* p, const double* u, double t, const double* du_bar,
   int rc = adj_prepare(p);
   if (rc) return rc;
   const Brick& k = p->brick;
-  BrickCopyArgs ca{p->geom, k, u, p->BW[0], p->Bus};
+  BrickCopyArgs ca{p->geom, k, u, p->BW[0], nullptr};
   hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, p->stream, ca);
   if (!p->frame_static) launch_frame(p, p->BW[0], t);
   fill_layer(p, t, 0.0);
@@ -1978,27 +1963,22 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
     HIP_TRY(hipMalloc(&p->adjCkpt, nseg * fb20));
     p->adjCkptN = nseg;
   }
-  if (!stage_ok(p) && !p->Bcoef) {
-    HIP_TRY(hipMalloc(&p->Bcoef, sizeof(double) * CF_N * (size_t)k.fs));
-    HIP_TRY(hipMemsetAsync(p->Bcoef, 0, sizeof(double) * CF_N * (size_t)k.fs, p->stream));
-  }
   auto slot = [&](size_t i) { return p->adjSlots + i * 20 * (size_t)k.fs; };
   auto ckpt = [&](size_t i) { return p->adjCkpt + i * 20 * (size_t)k.fs; };
   hipEvent_t ev[4];
   for (auto& e : ev) HIP_TRY(hipEventCreate(&e));
-  const bool split = !stage_ok(p);  // as tgh_rk4's default
   // ---- forward: u_0 into the brick, a checkpoint at each segment's start ----
   HIP_TRY(hipEventRecord(ev[0], p->stream));
-  BrickCopyArgs ca{p->geom, k, u, p->BW[0], p->Bus};
+  BrickCopyArgs ca{p->geom, k, u, p->BW[0], nullptr};
   hipLaunchKernelGGL(k_brick_in, grid_brick(p), dim3(256), 0, p->stream, ca);
-  if (!split && stage_wraps(p)) launch_frame(p, p->BW[0], t0);
+  if (stage_wraps(p)) launch_frame(p, p->BW[0], t0);
   for (size_t sg = 0; sg < nseg; ++sg) {
     HIP_TRY(hipMemcpyAsync(ckpt(sg), p->BW[0], fb20, hipMemcpyDeviceToDevice, p->stream));
     const int n0 = (int)(sg * every), n1 = std::min(nsteps, (int)((sg + 1) * every));
-    for (int n = n0; n < n1; ++n) rk4_brick_launches(p, t0 + n * dt, dt, split);
+    for (int n = n0; n < n1; ++n) rk4_brick_launches(p, t0 + n * dt, dt, false);
   }
   HIP_TRY(hipEventRecord(ev[1], p->stream));
-  BrickCopyArgs co{p->geom, k, brick_un(p, split), u, nullptr};
+  BrickCopyArgs co{p->geom, k, brick_un(p, false), u, nullptr};
   hipLaunchKernelGGL(k_brick_out, grid_brick(p), dim3(256), 0, p->stream, co);
   // J = the masked L2 error at T, and lambda_T = dJ/du_T
   const double T = t0 + nsteps * dt;
@@ -2011,7 +1991,7 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
   }
   *J = den > 0 ? std::sqrt(num / den) : 0.0;
   double *lam = p->adjL[0], *lacc = p->adjL[1], *kb = p->adjK[0], *kbn = p->adjK[1];
-  launch_adj_init(p, AdjInitArgs{k, p->cs, T, *J, den, dt / 6, brick_un(p, split), lam, kb});
+  launch_adj_init(p, AdjInitArgs{k, p->cs, T, *J, den, dt / 6, brick_un(p, false), lam, kb});
   HIP_TRY(hipMemsetAsync(p->adjTh, 0, sizeof(double) * ADJ_NPAR * adj_runs(k), p->stream));
   // ---- backward: per segment, its stage inputs recomputed from the
   // checkpoint, then its steps reversed ----
@@ -2020,7 +2000,6 @@ int tgh_adjoint(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps,
   for (size_t sg = nseg; sg-- > 0;) {
     const int n0 = (int)(sg * every), n1 = std::min(nsteps, (int)((sg + 1) * every)), ns = n1 - n0;
     HIP_TRY(hipMemcpyAsync(slot(0), ckpt(sg), fb20, hipMemcpyDeviceToDevice, p->stream));
-    if (split) HIP_TRY(hipMemcpyAsync(p->Bus, ckpt(sg), fb20, hipMemcpyDeviceToDevice, p->stream));
     for (int j = 0; j < ns; ++j) {
       double* const Y[5] = {slot(4 * j), slot(4 * j + 1), slot(4 * j + 2), slot(4 * j + 3), slot(4 * j + 4)};
       brick_step_slots(p, Y, t0 + (n0 + j) * dt, dt);
