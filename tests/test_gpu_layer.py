@@ -214,3 +214,42 @@ def test_levels_away_from_the_layer_and_across_it(tgh, center):
     orc = oracle_lib.OracleProblem(TD.TghDesc.from_buffer_copy(bytes(p.desc)), leaves=[tuple(lf) for lf in f.leaves],
                                    prolongation=4)
     against_the_oracle(tgh, p, orc, 1.0 / 32, 0.0, 0x1A7EA, (0, tgh.TGH_RK4_FUSED, tgh.TGH_RK4_GRAPH))
+
+
+PARAMETERS = {
+    "harmonic_q4": lambda tgh: (tgh.harmonic_kerr_case(M=1.0, a=0.3, halfwidth=1.5, r_0=0.4, r_1=0.95, gamma2=0.1,
+                                                       rho_max=4.0), 12, 4, 4),
+    "kerr_schild_sampled_q6": lambda tgh: (tgh.kerr_schild_case(M=1.0, a=0.5, halfwidth=1.6875, r_0=0.71, r_1=1.4,
+                                                                gamma2=0.1, rho_max=4.0), 9, 6, 6),
+    "kerr_schild_closed_form_q8": lambda tgh: (tgh.kerr_schild_case(M=1.0, a=0.5, halfwidth=1.75, r_0=0.71, r_1=1.5,
+                                                                    gamma2=0.1, rho_max=4.0,
+                                                                    gauge_source="algebraic"), 14, 4, 8),
+}
+
+
+@pytest.mark.parametrize("name", list(PARAMETERS))
+def test_the_parameters_cotangent_alone(tgh, name):
+    """theta_bar against the oracle's derivative along a parameter direction with
+    the state held: beside the state's own terms, a million times larger, an
+    error in it would not show. The layer's terms are sums of u - u_exact and
+    the damping's of the constraint, differences of values of size 1 to 1/h that
+    cancel to the noise of 1e-4: some 1e3 roundings over that, 2e-9 of each."""
+    torch = torch_cuda()
+    case, N, roots, q = PARAMETERS[name](tgh)
+    p = tgh.GHProblem(tgh.gh_forest(None, case, N=N, roots=roots), case, q=q)
+    orc = oracle_lib.OracleProblem(TD.TghDesc.from_buffer_copy(bytes(p.desc)))
+    u = orc.fill_exact(0.05)
+    orc.add_noise(u, 0x1A7EB, 1e-4)
+    rng = np.random.default_rng(12)
+    lam, v = rng.standard_normal(u.shape), rng.standard_normal(u.shape)
+    ub, thb = tgh.vjp_rhs(p, torch.from_numpy(u).cuda(), 0.05, torch.from_numpy(lam).cuda())
+    for k in range(5):
+        pd = np.zeros(5)
+        pd[k] = 1.0
+        _, dF = oracle_lib.gh_rhs_jvp(orc, u, np.zeros_like(u), 0.05, pd)
+        want, scale = float(np.dot(lam, dF)), float(np.abs(lam * dF).sum())
+        print(f"{tgh.ADJOINT_PARAMS[k]}: {thb[k]:.12e} oracle {want:.12e}, |diff| / scale = "
+              f"{abs(thb[k] - want) / scale:.2e}")
+        assert abs(thb[k] - want) <= 2e-9 * scale
+    _, dF = oracle_lib.gh_rhs_jvp(orc, u, v, 0.05, np.zeros(5))
+    assert abs(float(np.dot(lam, dF)) - float(np.dot(ub.cpu().numpy(), v))) <= 1e-12 * float(np.abs(lam * dF).sum())
