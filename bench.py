@@ -70,7 +70,7 @@ def parse():
     ap.add_argument("--no-per-block", action="store_true", help="skip the plain per-block form")
     ap.add_argument("--no-batch", action="store_true", help="skip the four-hole batch")
     ap.add_argument("--no-forest", action="store_true", help="skip the three-level forest")
-    ap.add_argument("--no-tune", action="store_true", help="keep the default Pi tile shape (no autotuner)")
+    ap.add_argument("--no-tune", action="store_true", help="with --form brick-split: keep the default Pi tile shape (no autotuner)")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="end with a 1 GiB device-to-device copy, the known-size reference for "
                          "rocprofv3's FETCH_SIZE / WRITE_SIZE counters")

@@ -74,7 +74,9 @@ enum { /* which block holds a point on a block face as its own (tgh_desc.ownersh
 };
 enum { /* tgh_rk4 flags */
   TGH_RK4_GRAPH = 1,  /* capture the step in a hipGraph and replay it */
-  TGH_RK4_FUSED = 2,  /* one kernel per right-hand side */
+  TGH_RK4_FUSED = 2,  /* one kernel per right-hand side (on the brick, where the
+                         layer's targets of an interior at rest find no memory,
+                         the split form, which evaluates them itself) */
   TGH_RK4_BLOCKS = 4, /* run the stages on the per-block ghosted work arrays
                          (a ghost fill per stage) instead of the default brick
                          layout (every point once, a frame of ghosts around
@@ -363,17 +365,19 @@ int tgh_refinement_indicator(tgh_problem* p, const double* u, double t, double s
  * over the evolved owned points, the indicator's reference amplitude. */
 int tgh_field_scale(tgh_problem* p, const double* u, double t, double* scale);
 /* No reference counterpart (the reference's kernels take no launch shape):
- * the autotuner of the brick stepper's tile shapes. Steps u three times per
- * candidate shape of the Pi kernel's LDS tile (TGH_PI_TILES of them; every
- * shape computes the same bits, so u is advanced 3 TGH_PI_TILES steps from
- * t0 as the default form would), times each shape's Pi launches with
+ * the autotuner of the brick's split form (TGH_RK4_SPLIT); the default form's
+ * one kernel a stage has one tile shape and is left as it is. Steps u three
+ * times per candidate shape of the Pi kernel's LDS tile (TGH_PI_TILES of them;
+ * every shape computes the same bits, so u is advanced 3 TGH_PI_TILES steps
+ * from t0 as TGH_RK4_SPLIT would), times each shape's Pi launches with
  * hipEvents, writes the average ms per launch into ms (TGH_PI_TILES doubles,
- * or NULL) and keeps the fastest for the problem's later tgh_rk4 calls.
- * Pass a scratch copy of the state. TGH_EUNSUPPORTED on the block layout. */
+ * or NULL) and keeps the fastest for the problem's later TGH_RK4_SPLIT steps.
+ * Allocates the split form's coefficients. Pass a scratch copy of the state.
+ * TGH_EUNSUPPORTED on the block layout. */
 enum { TGH_PI_TILES = 6 };
 int tgh_autotune(tgh_problem* p, double* u, double t0, double dt, double* ms);
-/* No reference counterpart: pins the Pi kernel's tile shape (0 .. TGH_PI_TILES - 1;
- * 0 is the default). */
+/* No reference counterpart: pins the split form's Pi tile shape
+ * (0 .. TGH_PI_TILES - 1; 0 is the default). */
 int tgh_set_tile(tgh_problem* p, int32_t tile);
 /* Several independent problems stepped together (the batched form: holes of
  * uneven block counts in one launch per stage, driven by a device-side table

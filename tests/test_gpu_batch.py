@@ -1,5 +1,5 @@
 """The batched stepper (several independent holes of uneven block counts, one
-head and one Pi launch per RK4 stage) and the plain per-block form, through
+launch per RK4 stage) and the plain per-block form, through
 the C ABI. A problem in a batch runs the same kernel code on the same arrays
 as the problem alone, so it must reproduce the brick stepper's bits; the
 per-block form runs the fused block kernel one block at a time and must
@@ -44,8 +44,8 @@ def noisy_states(tgh, probs, amplitude=1e-8):
 
 def check_batch_equals_alone(tgh, probs, nsteps, graph, roundoff=False):
     """Every problem of the batch computes the bits it computes alone; with
-    roundoff, to an ulp of the state's scale (a moving hole's head is its own
-    kernel alone and in a batch, and their arithmetic may round apart)."""
+    roundoff, to an ulp of the state's scale (what a moving hole's test asks
+    for)."""
     torch = torch_cuda()
     us = noisy_states(tgh, probs)
     ref = [u.clone() for u in us]
@@ -91,7 +91,7 @@ def test_batch_of_harmonic_holes_steps_each_as_alone(tgh):
 
 
 def test_batch_of_moving_frames_steps_each_as_alone(tgh):
-    """Gauge waves: periodic frames refilled every stage, tables re-made every step."""
+    """Gauge waves: periodic frames refilled every stage."""
     probs = []
     for roots, N in ((2, 8), (3, 8)):
         case = tgh.gauge_wave_case(eps_ko=0.5, gamma0=1.0, gamma2=0.0)

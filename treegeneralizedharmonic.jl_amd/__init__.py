@@ -1252,9 +1252,10 @@ TGH_PI_TILES = 6
 
 
 def autotune(p, u, dt, t=0.0):
-    """The brick stepper's autotuner (no reference counterpart): times each
-    tile shape of the Π kernel on a scratch copy of u and keeps the fastest
-    for p's later steps; returns the average ms per Π launch of each shape."""
+    """The autotuner of the brick's split form (no reference counterpart): times
+    each tile shape of its Π kernel on a scratch copy of u and keeps the fastest
+    for p's later TGH_RK4_SPLIT steps; returns the average ms per Π launch of
+    each shape. gh_solve's default form, one kernel a stage, has one shape."""
     w = u.clone()
     ms = (C.c_double * TGH_PI_TILES)()
     _check(_load().tgh_autotune(p.ptr, _dev(w, p, "u"), float(t), float(dt), ms))

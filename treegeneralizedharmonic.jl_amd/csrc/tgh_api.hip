@@ -1734,9 +1734,13 @@ int tgh_rk4(tgh_problem* p, double* u, double t0, double dt, int32_t nsteps, int
   // forms: 0 block layout, head + Pi; 1 block layout, fused; 2 brick layout,
   // one kernel a stage; 3 brick layout, head + LDS-tiled Pi; 4 block layout,
   // fused, one launch per block; 5 block layout, each block run as a brick in
-  // one kernel a stage (block_stage_ok; else form 0). Without FUSED or SPLIT the layout's faster form on MI355X (measured: the
-  // brick's one kernel a stage; on the block layout form 5 where it runs,
-  // else the fused kernel).
+  // one kernel a stage (block_stage_ok; else form 0). Without FUSED or SPLIT
+  // the layout's faster form: form 2 on the brick, on blocks form 5 where it
+  // runs, else the fused kernel. A step of the Kerr-Schild hole on 512 blocks
+  // of 16^3 in forms 3 and 2 at q = 2, 4, 6, 8: 5.73 and 2.62 ms, 6.93 and
+  // 3.21, 10.2 and 6.66, 85.7 and 12.1; of the wave on 96^3 points at q = 6 and
+  // 8: 3.95 and 2.17, 28.2 and 4.70. (The stage spills 48 to 132 registers at
+  // q = 6 and 309 to 495 at q = 8, and is the faster there too.)
   {
     int rc = blocks ? ensure_layer_box(p) : ensure_brick(p);
     if (rc) return rc;

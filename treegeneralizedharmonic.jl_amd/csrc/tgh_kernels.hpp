@@ -17,10 +17,10 @@ enum { INT_NONE = 0, INT_DAMPED = 1, INT_FROZEN = 2, INT_PASTED = 3, INT_FITTED 
 // a moving hole its own (its kernels carry the moving core and layer).
 enum { GAUGE_NONE = 0, GAUGE_SAMPLED = 1, GAUGE_KS = 2, GAUGE_KS_MOVING = 3, GAUGE_NONE_MOVING = 4 };
 // The kernels' interior kinds (template HOLE): 0 none, 1 the sphere, 2 the
-// general interior (tracked geometry, :fitted), 3 the sphere of a moving
-// :damped hole or of a harmonic hole at rest, whose core and layer targets
-// come from the layer box (k_brick_moving, or k_brick_layer at rest) instead of
-// the dual passes in the head.
+// general interior (tracked geometry, :fitted), 3 the sphere with its core and
+// layer targets from the layer box (k_brick_moving, or k_brick_layer at rest):
+// every interior of the one-kernel stage and the adjoint, and in the other
+// kernels those whose target is a dual pass (moving and harmonic holes).
 enum { HOLE_BOXED = 3 };
 constexpr bool gauge_has_source(int gauge) { return gauge == GAUGE_SAMPLED || gauge == GAUGE_KS || gauge == GAUGE_KS_MOVING; }
 enum { EPI_STORE = 0, EPI_RK4 = 1 };
@@ -684,9 +684,9 @@ struct RhsArgs {
   double* __restrict__ coef;
   const double* clock;  // stage_time's clock (NULL: t as given) and offset
   double toff;
-  // a moving hole's layer targets and rates on the brick, evaluated per stage by
-  // k_brick_moving (LAYER_FIELDS fields of lB^3 slots, slot = brick coordinates mod lB);
-  // NULL: the head evaluates them itself
+  // the layer box: lB^3 slots (slot = grid coordinates mod lB) of a moving hole's
+  // targets and rates (LAYER_FIELDS fields) or of an interior's at rest (20);
+  // NULL: none, and a head that needs targets evaluates them itself
   const double* lbox;
   long lB3;
   int lB;
@@ -899,7 +899,7 @@ __device__ __forceinline__ void head_source(const RhsArgs& a, const PointRef& pr
           re[NC + v] = (lb[(3 * NC + v) * a.lB3] - lb[(4 * NC + v) * a.lB3]) / (tp - tm);
         }
       } else if constexpr (HOLE == HOLE_BOXED) {
-        // a harmonic hole at rest: its target from the box, filled once
+        // at rest, without a gauge source: the target from the box
         const double* lb = a.lbox + pr.lslot;
 #pragma unroll
         for (int v = 0; v < 20; ++v) ue[v] = lb[v * a.lB3];
@@ -999,7 +999,7 @@ __device__ __forceinline__ void core_rates(const RhsArgs& a, const double x[3], 
         Pu[v] = src.P(v);
       }
       if constexpr (HOLE == HOLE_BOXED) {
-        // the target from the box (k_brick_layer) and its rates formed here as
+        // the target from the box (k_brick_moving) and its rates formed here as
         // core_target_rate forms them
 #pragma clang fp contract(off)
         const CaseP& c = a.c;

@@ -69,7 +69,7 @@ struct tgh_problem {
   double* Bacc = nullptr;
   double* BH = nullptr;
   double* Bcoef = nullptr;            // the split form's coefficients (CF_N brick fields)
-  double* Blayer = nullptr;           // a hole's layer box (LAYER_FIELDS x layer_B^3 moving, 20 x layer_B^3 at rest)
+  double* Blayer = nullptr;           // the layer box (LAYER_FIELDS x layer_B^3 moving, 20 x layer_B^3 at rest)
   int layer_B = 0;
   int layer_lmax = 0;                 // the level whose grid the box is on: the finest that meets the layer
   bool layer_static = false;          // filled once (a static background's)

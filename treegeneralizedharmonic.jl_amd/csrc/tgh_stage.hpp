@@ -367,7 +367,11 @@ struct KindC {
 // the brick (a row of 16 doubles is a 128-byte line), 17 x 5 x 3 on a block of
 // 17^3 owned points (80 % of the threads busy, where 16 x 4 x 4 would keep 43
 // %): the octree of 2416 blocks takes 5.6 ms a stage where the two kernels it
-// replaces took 6.2 + 4.1.
+// replaces took 6.2 + 4.1. The shape is the same for every N: away from 16 it
+// keeps fewer threads busy (22 % at N = 6, 57 % at 12, 52 % at 20) and is still
+// the faster. Steps of a three-level forest over one box with blocks of N = 6,
+// 8, 10, 12, 16, 20, 24 and 32 take 77, 51, 40, 39, 37, 38, 37 and 45 ms, where
+// the two kernels took 99, 74, 56, 55, 58, 52, 53 and 70.
 enum { TILE_BRICK = 0, TILE_BLOCK = 1 };
 template <int Q, int T> struct StageTile {
   static constexpr int X = T == TILE_BRICK ? 16 : 17, Y = T == TILE_BRICK ? 4 : 5, Z = T == TILE_BRICK ? 4 : 3;
