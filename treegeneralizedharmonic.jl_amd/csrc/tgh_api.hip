@@ -487,14 +487,14 @@ void launch_layer(tgh_problem* p, double t, double toff) {
   hipLaunchKernelGGL(k_brick_layer, dim3((unsigned)((B3 + 255) / 256)), dim3(256), 0, p->stream, la);
 }
 // The layer box (k_brick_moving, k_brick_layer) of a moving :damped hole or of
-// an interior at rest, on the finest level's grid: the layer's bounding box
-// about c(t) with a point of margin each side, whatever t (slots wrap modulo
-// B), but no wider than the mesh's longest axis. A :frozen layer has no target (its rate rho
-// is zero): its box is one slot of zeros, which every point reads. Nothing for
-// other cases. At rest the grid is the finest level's among the blocks that
-// meet the layer: levels elsewhere do not make its box larger.
-// The one-kernel stage on the brick needs 20 fields of the layer's cube, where
-// the split form's two kernels need 25 of the whole brick.
+// an interior at rest: the layer's bounding box about c(t) with a point of
+// margin each side, whatever t (slots wrap modulo B), but no wider than the
+// mesh's longest axis, on the finest level's grid (at rest the finest among the
+// blocks that meet the layer: levels elsewhere do not make the box larger). A
+// :frozen layer has no target (its rate rho is zero): its box is one slot of
+// zeros, which every point reads. Nothing for other cases. The one-kernel stage
+// on the brick needs these 20 fields of the layer's cube, where the split
+// form's two kernels need 25 of the whole brick.
 int ensure_layer_box(tgh_problem* p) {
   if (p->Blayer || p->cs.general || p->cs.interior == INT_NONE || p->cs.interior == INT_PASTED) return TGH_OK;
   const bool frozen = p->cs.interior == INT_FROZEN, rest = !p->cs.moving;
@@ -540,8 +540,8 @@ int ensure_layer_box(tgh_problem* p) {
   p->Blayer = nullptr;
   return fail(TGH_EDEVICE, std::string("filling the layer box: ") + hipGetErrorString(e));
 }
-// The box kernel's view of the finest level's grid (its corner, spacing and
-// closed point counts; the other fields are unused there).
+// The box kernels' view of their level's grid (its corner, spacing and closed
+// point counts; the other fields are unused there).
 Brick layer_grid(const tgh_problem* p) {
   Brick k;
   std::memset(&k, 0, sizeof(k));
